@@ -238,7 +238,12 @@ struct SampleWs {
   void *sort_tmp = nullptr;        /* radix-sort temporary storage */
   size_t sort_bytes = 0;
   int cap = 0;                     /* vocabulary the buffers hold */
+  void *topk = nullptr;            /* candidate lists of the three-launch top-k */
+  int topk_cap = 0;                /* vocabulary they hold */
 };
+/* bytes of SampleWs.topk for a vocabulary; 0: the one-workgroup replay takes
+ * the call */
+size_t gq_sample_topk_bytes(int vocab, int top_k);
 /* radix-sort temporary bytes for a vocabulary */
 size_t gq_sample_ws_bytes(int vocab);
 /* The reference's sampler choice (generate.c:302-311) for rnd = its rand()

@@ -100,7 +100,7 @@ struct gq_ctx {
   void *stage[2] = {nullptr, nullptr};
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
   SampleWs sw;
-  int *d_sample = nullptr; /* sampled token (device) */
+  int *h_sample = nullptr; /* sampled token: pinned, written by the kernels, read after the wait */
   /* graph */
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
@@ -234,6 +234,7 @@ extern "C" void gq_hip_destroy(gq_ctx *c) {
   (void)hipStreamSynchronize(c->stream);
   free_graph(c);
   if (c->st_pinned) (void)hipHostFree(c->st_pinned);
+  if (c->h_sample) (void)hipHostFree(c->h_sample);
   for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
   for (void *p : c->allocs) (void)hipFree(p);
   for (int i = 0; i < 2; i++) {
@@ -1740,9 +1741,19 @@ extern "C" int gq_hip_argmax_dev(gq_ctx *c, const float *x, int n, int *out_inde
 }
 
 /* ---- on-device sampling (tokenizer.c:175-333, generate.c:302-311) ---- */
-static int sample_ensure(gq_ctx *c, int vocab, bool big) {
+static int sample_ensure(gq_ctx *c, int vocab, bool big, int top_k) {
   SampleWs &w = c->sw;
-  if (!c->d_sample && !(c->d_sample = (int *)dev_alloc(c, sizeof(int)))) return -4;
+  if (!c->h_sample && hipHostMalloc((void **)&c->h_sample, sizeof(int)) != hipSuccess) {
+    c->h_sample = nullptr;
+    return -4;
+  }
+  if (const size_t tb = top_k > 0 ? gq_sample_topk_bytes(vocab, top_k) : 0; tb && w.topk_cap < vocab) {
+    void *p = dev_alloc(c, tb);
+    if (p) { /* without it the one-workgroup replay runs */
+      if (w.topk) gq_hip_free(c, w.topk);
+      w.topk = p, w.topk_cap = vocab;
+    }
+  }
   if (!big || w.cap >= vocab) return 0;
   const size_t sort_bytes = gq_sample_ws_bytes(vocab);
   float *keys = (float *)dev_alloc(c, sizeof(float) * vocab);
@@ -1760,15 +1771,15 @@ static int sample_on_device(gq_ctx *c, const float *logits, int vocab, float tem
                             int rnd) {
   /* top-p and plain temperature sampling use the vocabulary-sized buffers */
   const bool big = temperature > 0.0f && !(top_k > 0 && top_k < vocab) && top_p > 0.0f;
-  int rc = sample_ensure(c, vocab, big);
+  int rc = sample_ensure(c, vocab, big, temperature > 0.0f && top_k < vocab ? top_k : 0);
   if (rc) return rc;
-  rc = gq_launch_sample(logits, vocab, temperature, top_k, top_p, rnd, c->sw, c->d_sample, c->stream);
+  rc = gq_launch_sample(logits, vocab, temperature, top_k, top_p, rnd, c->sw, c->h_sample, c->stream);
   if (rc == 1) { /* greedy */
     const int nblk = gq_argmax_blocks(vocab);
     float *scratch = c->ws.amax && c->ws.amax_blocks >= nblk ? c->ws.amax
                                                              : (float *)dev_alloc(c, sizeof(float) * 2 * nblk);
     if (!scratch) return -4;
-    rc = gq_launch_argmax(logits, vocab, scratch, nblk, c->d_sample, nullptr, nullptr, nullptr, c->stream);
+    rc = gq_launch_argmax(logits, vocab, scratch, nblk, c->h_sample, nullptr, nullptr, nullptr, c->stream);
     if (scratch != c->ws.amax) {
       (void)hipStreamSynchronize(c->stream);
       gq_hip_free(c, scratch);
@@ -1776,10 +1787,8 @@ static int sample_on_device(gq_ctx *c, const float *logits, int vocab, float tem
   }
   if (rc == -2) return fail(c, -2, "top_k %d above the device limit %d", top_k, kMaxTopK);
   if (rc) return fail(c, rc, "sampling launch failed");
-  int tok = -1;
-  HIPCHK(c, hipMemcpyAsync(&tok, c->d_sample, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  return tok;
+  return *c->h_sample;
 }
 
 extern "C" int gq_hip_sample_dev(gq_ctx *c, const float *logits, int vocab, float temperature, int top_k,

@@ -118,3 +118,56 @@ def test_forward_sample_matches_reference(ctx, orc, samplers):
         got = H.lib.gq_hip_forward_sample(ctx.h, tok, pos, T, k, p, LIBC.rand())
         assert got == want, (step, got, want)
         tok = got
+
+
+def topk_slots(x, k):
+    """The k slots of tokenizer.c:219-253 after the last logit: (values, ids)."""
+    tv, ti = [float(v) for v in x[:k]], list(range(k))
+    mj = min(range(k), key=lambda j: (tv[j], j))
+    for i, v in enumerate(x.tolist()):
+        if i >= k and v > tv[mj]:
+            tv[mj], ti[mj] = v, i
+            mj = min(range(k), key=lambda j: (tv[j], j))
+    return np.array(tv, np.float32), np.array(ti)
+
+
+@pytest.mark.parametrize("V,k,kind", [
+    (41, 40, "normal"), (64, 1, "normal"), (65, 64, "normal"),      # one short slice, p0 = 64
+    (1023, 40, "normal"), (1024, 65, "normal"), (1025, 128, "normal"),  # the first slice's edge, p0 = 128
+    (2049, 64, "normal"), (5000, 128, "rising"), (70001, 100, "normal"), (33000, 256, "normal"), (14665, 195, "normal"),
+    (128256, 40, "normal"), (262144, 40, "normal"), (262145, 40, "normal"),  # the last runs the replay
+    (5000, 257, "normal"),                                          # replay: k above the lists'
+    (20000, 40, "few ties"), (20000, 200, "few ties"), (128256, 100, "few ties"),  # sorted by slot
+    (128256, 40, "ties"), (20000, 40, "ascending"),                 # replay from the third launch
+    (20000, 64, "descending"), (20000, 50, "masked"), (20000, 50, "nan"), (20000, 40, "zeros"),
+])
+def test_top_k_slots(ctx, orc, V, k, kind):
+    """Every kept token is drawn by a rnd in the middle of its share (so the
+    last bit of an exponential cannot move the draw), which pins the slots'
+    contents and order."""
+    import guanaco_amd.hip as H
+    x = logits_for(orc, V, kind, 5 + V + k)
+    if kind in ("ascending", "descending"):
+        x = np.ascontiguousarray(np.sort(x)[::1 if kind == "ascending" else -1])
+    elif kind == "few ties":  # 7, 16 and 5 groups of equal logits among the inserted
+        step = 512 if k == 40 else 4096
+        x = (np.round(x * step) / step).astype(np.float32)
+    elif kind == "masked":  # a vocabulary mask: most logits the lowest there are
+        x[np.arange(V) % 97 != 3] = -np.inf
+    elif kind == "nan":     # never above a minimum
+        x[[k, 999, 1024, V - 1]] = np.nan
+    elif kind == "zeros":   # -0 equals +0
+        x = np.where(x > 7, x, np.where(np.arange(V) % 2, np.float32(-0.0), np.float32(0.0))).astype(np.float32)
+    tv, ti = topk_slots(x, k)
+    xd, T = ctx.upload(x), 2.5
+    # larger logits first: nothing a call leaves in the workspace reaches the next one
+    yd = ctx.upload(np.where(np.isfinite(x), x + np.float32(50.0), np.float32(40.0)).astype(np.float32))
+    assert H.lib.gq_hip_sample_dev(ctx.h, yd.ptr, V, T, k, 1.0, 1 << 30) >= 0
+    p = np.exp((tv.astype(np.float64) - tv.max()) / T)
+    edge = np.concatenate([[0.0], np.cumsum(p)]) / p.sum()
+    wide = [j for j in range(k) if edge[j + 1] - edge[j] > 1e-4]
+    assert wide
+    for j in wide:
+        rnd = int((edge[j] + edge[j + 1]) / 2 * 2147483647.0)
+        assert H.lib.gq_hip_sample_dev(ctx.h, xd.ptr, V, T, k, 1.0, rnd) == ti[j], (j, k)
+    xd.free(), yd.free()
