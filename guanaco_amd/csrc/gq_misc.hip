@@ -136,10 +136,13 @@ __device__ __forceinline__ float embed_value(int dtype, const uint8_t *table, in
 
 /* Embedding row of `token`.  With tokens != NULL, row blockIdx.y holds
  * tokens[blockIdx.y] (out + blockIdx.y * hidden); blockIdx.x covers
- * 256-element slices of the row. */
+ * 256-element slices of the row.  With state != NULL the launch also sets
+ * the decode step's state (token, position, step, want) there, in place of a
+ * copy. */
 __global__ __launch_bounds__(kThreads) void embed_kernel(int dtype, const uint8_t *table, int hidden,
                                                         const int *token_dev, int token, const int *tokens,
-                                                        float *out) {
+                                                        float *out, int *state, int pos, int want) {
+  if (state && blockIdx.x == 0 && threadIdx.x == 0) state[0] = token, state[1] = pos, state[2] = 0, state[3] = want;
   const int tok = tokens ? tokens[blockIdx.y] : token_dev ? *token_dev : token;
   out += (size_t)blockIdx.y * hidden;
   for (int e = blockIdx.x * kThreads + threadIdx.x; e < hidden; e += gridDim.x * kThreads)
@@ -169,13 +172,15 @@ __device__ __forceinline__ void block_argmax(float &v, int &i) {
 
 constexpr int kArgmaxPerBlock = 1024; /* 126 workgroups for a 128256-entry vocabulary */
 
-__global__ __launch_bounds__(kThreads) void argmax_stage1(const float *x, int n, float *scratch) {
+__global__ __launch_bounds__(kThreads) void argmax_stage1(const float *x, int n, float *scratch, ArgmaxHost host) {
+  const bool copy = host.x && (!host.want || *host.want);
   const int base = blockIdx.x * kArgmaxPerBlock;
   const int end = min(n, base + kArgmaxPerBlock);
   float v = -INFINITY;
   int i = 0x7fffffff;
   for (int e = base + threadIdx.x; e < end; e += kThreads) {
     float xe = x[e];
+    if (copy) host.x[e] = xe;
     /* sample_greedy starts from logits[0] and only a strictly greater value
      * replaces it, so a NaN there is never replaced: index 0 wins.  As +inf
      * it does, since ties go to the lowest index.  A NaN elsewhere never
@@ -198,7 +203,8 @@ __global__ __launch_bounds__(kThreads) void argmax_stage1(const float *x, int n,
  * separate embedding after the argmax). */
 __global__ __launch_bounds__(kThreads) void argmax_stage2(const float *scratch, int nblk, int *out,
                                                          int *tokens, int *step_dev, int *pos_dev, int edt,
-                                                         const uint8_t *etab, int hidden, float *eout) {
+                                                         const uint8_t *etab, int hidden, float *eout,
+                                                         ArgmaxHost host) {
   float v = -INFINITY;
   int i = 0x7fffffff;
   for (int b = threadIdx.x; b < nblk; b += kThreads)
@@ -207,6 +213,7 @@ __global__ __launch_bounds__(kThreads) void argmax_stage2(const float *scratch, 
   if (i == 0x7fffffff) i = 0; /* all NaN: the reference keeps index 0 */
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     *out = i;
+    if (host.token) *host.token = i;
     if (step_dev) {
       tokens[*step_dev] = i;
       *step_dev += 1;
@@ -216,6 +223,8 @@ __global__ __launch_bounds__(kThreads) void argmax_stage2(const float *scratch, 
   if (eout)
     for (int e = blockIdx.x * kThreads + threadIdx.x; e < hidden; e += gridDim.x * kThreads)
       eout[e] = embed_value(edt, etab, hidden, i, e);
+  if (blockIdx.x == 0)
+    for (int e = threadIdx.x; e < host.row_n; e += kThreads) host.row_out[e] = host.row[e];
 }
 
 __global__ void silu_mul_kernel(float *gate, const float *up, int n) {
@@ -310,10 +319,10 @@ int gq_launch_rmsnorm_rows(const float *x, const float *w, float *out, int dim, 
 }
 
 int gq_launch_embed(int dtype, const void *table, int hidden, const int *token_dev, int token,
-                    float *out, hipStream_t s) {
+                    float *out, hipStream_t s, int *state, int pos, int want) {
   if (dtype != GQ_F32 && dtype != GQ_Q8_0 && dtype != GQ_Q4_K) return -1;
   hipLaunchKernelGGL(embed_kernel, dim3((hidden + kThreads - 1) / kThreads), dim3(kThreads), 0, s, dtype,
-                     (const uint8_t *)table, hidden, token_dev, token, (const int *)nullptr, out);
+                     (const uint8_t *)table, hidden, token_dev, token, (const int *)nullptr, out, state, pos, want);
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
@@ -321,7 +330,7 @@ int gq_launch_embed_rows(int dtype, const void *table, int hidden, const int *to
                          hipStream_t s) {
   if ((dtype != GQ_F32 && dtype != GQ_Q8_0 && dtype != GQ_Q4_K) || !tokens_dev || n <= 0) return -1;
   hipLaunchKernelGGL(embed_kernel, dim3((hidden + kThreads - 1) / kThreads, n), dim3(kThreads), 0, s, dtype,
-                     (const uint8_t *)table, hidden, (const int *)nullptr, 0, tokens_dev, out);
+                     (const uint8_t *)table, hidden, (const int *)nullptr, 0, tokens_dev, out, (int *)nullptr, 0, 0);
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
@@ -329,15 +338,15 @@ int gq_argmax_blocks(int n) { return (n + kArgmaxPerBlock - 1) / kArgmaxPerBlock
 
 int gq_launch_argmax(const float *x, int n, float *scratch, int nblk, int *out_index, int *tokens,
                      int *step_dev, int *pos_dev, hipStream_t s, int emb_dtype, const void *emb_table, int hidden,
-                     float *emb_out) {
+                     float *emb_out, const ArgmaxHost &host) {
   if (n <= 0 || nblk != gq_argmax_blocks(n)) return -1;
   if (emb_out && ((emb_dtype != GQ_F32 && emb_dtype != GQ_Q8_0 && emb_dtype != GQ_Q4_K) || !emb_table ||
                   hidden <= 0))
     return -1;
-  hipLaunchKernelGGL(argmax_stage1, dim3(nblk), dim3(kThreads), 0, s, x, n, scratch);
+  hipLaunchKernelGGL(argmax_stage1, dim3(nblk), dim3(kThreads), 0, s, x, n, scratch, host);
   hipLaunchKernelGGL(argmax_stage2, dim3(emb_out ? (hidden + kThreads - 1) / kThreads : 1), dim3(kThreads), 0, s,
                      scratch, nblk, out_index, tokens, step_dev, pos_dev, emb_dtype, (const uint8_t *)emb_table,
-                     hidden, emb_out);
+                     hidden, emb_out, host);
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 

@@ -44,7 +44,6 @@ struct PrefillWs {
   float *x = nullptr, *q = nullptr, *k = nullptr, *v = nullptr; /* fp32: hidden, q/k/v for RoPE */
   __bf16 *xn = nullptr, *att = nullptr, *act = nullptr;          /* bf16 GEMM inputs */
   __bf16 *xb = nullptr; /* op-level entry: bf16 copy of its fp32 x */
-  int *tok = nullptr;
   size_t xb_cap = 0;
   float *part = nullptr; /* the GEMM's K-part sums (PgArgs.part) */
   size_t part_cap = 0;
@@ -52,6 +51,9 @@ struct PrefillWs {
 
 /* tokens per prefill chunk */
 constexpr int kPrefillChunk = 512;
+/* prompt tokens that gq_ctx::h_in holds: a prompt is embedded in pieces of at
+ * most that many */
+constexpr int kPinnedTokens = 16 * kPrefillChunk;
 
 } // namespace
 
@@ -100,7 +102,16 @@ struct gq_ctx {
   void *stage[2] = {nullptr, nullptr};
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
   SampleWs sw;
-  int *h_sample = nullptr; /* sampled token: pinned, written by the kernels, read after the wait */
+  /* pinned host memory: the token that a step, a prompt or a sampler picked
+   * and the results a caller asked for (written by the argmax's or sampler's
+   * launches, read after the wait), and a prompt's tokens (read by the
+   * embedding kernel).  A copy to a caller's pageable buffer instead makes the
+   * host wait for it and wakes it up late: 13-29 us for four bytes. */
+  void *pinned = nullptr; /* one allocation: h_tok, h_in, h_out */
+  int *h_tok = nullptr;
+  int *h_in = nullptr; /* kPinnedTokens of them */
+  float *h_out = nullptr; /* logits, then a hidden state */
+  size_t h_out_cap = 0;
   /* graph */
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
@@ -108,7 +119,8 @@ struct gq_ctx {
    * the embedding of g_token, to be decoded at g_pos */
   bool g_valid = false;
   int g_token = -1, g_pos = -1;
-  int *st_pinned = nullptr; /* pinned (token, pos, step) for graph_step */
+  int g_step = 0;        /* replays since the device step was last set */
+  bool g_logits = false; /* the replays also write the logits to h_out */
   /* measurement hooks for eager steps */
   bool prof = false;
   std::vector<hipEvent_t> ev;
@@ -118,6 +130,7 @@ struct gq_ctx {
 
 static int fail(gq_ctx *c, int code, const char *fmt, ...) __attribute__((format(printf, 3, 4)));
 static void pf_release(gq_ctx *c);
+static int ensure_pinned(gq_ctx *c, size_t out);
 static int fail(gq_ctx *c, int code, const char *fmt, ...) {
   if (c) {
     va_list ap;
@@ -233,8 +246,7 @@ extern "C" void gq_hip_destroy(gq_ctx *c) {
   (void)hipSetDevice(c->dev);
   (void)hipStreamSynchronize(c->stream);
   free_graph(c);
-  if (c->st_pinned) (void)hipHostFree(c->st_pinned);
-  if (c->h_sample) (void)hipHostFree(c->h_sample);
+  if (c->pinned) (void)hipHostFree(c->pinned);
   for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
   for (void *p : c->allocs) (void)hipFree(p);
   for (int i = 0; i < 2; i++) {
@@ -924,6 +936,7 @@ extern "C" int gq_hip_model_bind(gq_ctx *c, const gq_model *m) {
     w.d_pos = w.d_token + 1;
     w.d_step = w.d_token + 2;
   }
+  if (int rc = ensure_pinned(c, (size_t)m->vocab + H)) return rc;
   c->bound = true;
   return 0;
 }
@@ -1115,10 +1128,12 @@ static int run_step(gq_ctx *c, int token, int pos, bool device_state, float *hid
                                hipMemcpyDeviceToHost, c->stream));
   }
   if ((rc = op_lm_head(c, w.hidden))) return rc;
+  ArgmaxHost host{};
+  if (device_state) host.token = c->h_tok, host.x = c->h_out, host.want = w.d_step + 1;
   if ((rc = gq_launch_argmax(w.logits, m.vocab, w.amax, w.amax_blocks, w.d_token,
                              device_state ? w.d_tokens : nullptr, device_state ? w.d_step : nullptr,
                              device_state ? w.d_pos : nullptr, c->stream, m.embed.dtype, m.embed.data, m.hidden,
-                             device_state ? w.hidden : nullptr)))
+                             device_state ? w.hidden : nullptr, host)))
     return rc;
   mark(c, PC_OTHER, 4.0 * m.vocab);
   return 0;
@@ -1177,42 +1192,42 @@ extern "C" int gq_hip_transformer_layer(gq_ctx *c, int layer, int pos, float *h_
 
 static int ensure_tokens(gq_ctx *c, int n);
 static int ensure_graph(gq_ctx *c);
+/* tokens a host-driven greedy loop's replays store before the device step is
+ * set back */
+constexpr int kStepTokens = 1024;
 
 /* One decode step of a host-driven loop (the generate and chat loops call
  * forward_token / forward_sample once per token) as a replay of the
  * captured step graph.  The graph expects the token's embedding in w.hidden
  * and token, position and step on the device, and leaves the argmax
  * token's embedding and the next position there.  When the caller's
- * (token, pos) is what the previous replay left (a greedy loop), only the
- * step counter is reset; otherwise the token is embedded first. */
-static int graph_step(gq_ctx *c, int token, int pos) {
+ * (token, pos) is what the previous replay left (a greedy loop), the graph is
+ * all there is to launch; otherwise the token is embedded first, by a launch
+ * that also sets token, position and step. */
+static int graph_step(gq_ctx *c, int token, int pos, bool want_logits) {
   Workspace &w = c->ws;
   int rc;
   if ((rc = ensure_tokens(c, 1)) || (rc = ensure_graph(c))) return rc;
-  if (!c->st_pinned && hipHostMalloc((void **)&c->st_pinned, 4 * sizeof(int)) != hipSuccess) {
-    c->st_pinned = nullptr;
-    return fail(c, -4, "pinned step state");
-  }
-  const bool same = c->g_valid && c->g_token == token && c->g_pos == pos;
-  c->st_pinned[0] = token, c->st_pinned[1] = pos, c->st_pinned[2] = 0;
-  HIPCHK(c, hipMemcpyAsync(w.d_token, c->st_pinned, 3 * sizeof(int), hipMemcpyHostToDevice, c->stream));
-  if (!same && (rc = gq_launch_embed(c->m.embed.dtype, c->m.embed.data, c->m.hidden, w.d_token, token, w.hidden,
-                                     c->stream)))
-    return fail(c, rc, "embed launch failed");
+  const bool same = c->g_valid && c->g_token == token && c->g_pos == pos && c->g_step < w.tokens_cap &&
+                    c->g_logits == want_logits;
   c->g_valid = false;
+  if (!same) {
+    if ((rc = gq_launch_embed(c->m.embed.dtype, c->m.embed.data, c->m.hidden, nullptr, token, w.hidden, c->stream,
+                              w.d_token, pos, want_logits)))
+      return fail(c, rc, "embed launch failed");
+    c->g_step = 0, c->g_logits = want_logits;
+  }
   HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
+  c->g_step++;
   return 0;
 }
 
 /* After graph_step: the argmax token to the host; the device state is then
  * (next, pos + 1). */
 static int graph_step_token(gq_ctx *c, int pos, float *logits) {
-  HIPCHK(c, hipMemcpyAsync(c->st_pinned + 3, c->ws.d_token, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  if (logits)
-    HIPCHK(c, hipMemcpyAsync(logits, c->ws.logits, sizeof(float) * c->m.vocab, hipMemcpyDeviceToHost,
-                             c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  const int next = c->st_pinned[3];
+  if (logits) memcpy(logits, c->h_out, sizeof(float) * c->m.vocab);
+  const int next = *c->h_tok;
   c->g_valid = true, c->g_token = next, c->g_pos = pos + 1;
   return next;
 }
@@ -1223,7 +1238,7 @@ extern "C" int gq_hip_forward_token(gq_ctx *c, int token, int pos, float *logits
   if (rc) return rc;
   if (token < 0 || token >= c->m.vocab) return fail(c, -1, "token %d out of range", token);
   if (!hidden_per_layer) { /* no per-layer copies: the captured step */
-    if ((rc = graph_step(c, token, pos))) return rc;
+    if ((rc = graph_step(c, token, pos, logits != nullptr))) return rc;
     return graph_step_token(c, pos, logits);
   }
   if ((rc = run_step(c, token, pos, false, hidden_per_layer))) return fail(c, rc, "step launch failed");
@@ -1236,8 +1251,24 @@ extern "C" int gq_hip_forward_token(gq_ctx *c, int token, int pos, float *logits
   return next;
 }
 
+/* the context's pinned memory, with out floats of results */
+static int ensure_pinned(gq_ctx *c, size_t out) {
+  if (c->pinned && c->h_out_cap >= out) return 0;
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  free_graph(c); /* it captured the old pointers */
+  if (c->pinned) (void)hipHostFree(c->pinned);
+  c->pinned = nullptr, c->h_tok = c->h_in = nullptr, c->h_out = nullptr, c->h_out_cap = 0;
+  void *p = nullptr;
+  if (hipHostMalloc(&p, sizeof(int) * (64 + kPinnedTokens) + sizeof(float) * out) != hipSuccess)
+    return fail(c, -4, "pinned memory for %zu floats", out);
+  c->pinned = p, c->h_tok = (int *)p, c->h_in = c->h_tok + 64, c->h_out = (float *)(c->h_in + kPinnedTokens);
+  c->h_out_cap = out;
+  return 0;
+}
+
 static int ensure_tokens(gq_ctx *c, int n) {
   Workspace &w = c->ws;
+  n = std::max(n, kStepTokens); /* a captured graph keeps the buffer */
   if (w.tokens_cap >= n) return 0;
   if (w.d_tokens) gq_hip_free(c, w.d_tokens);
   w.d_tokens = (int *)dev_alloc(c, sizeof(int) * n);
@@ -1276,7 +1307,7 @@ extern "C" int gq_hip_decode_loop(gq_ctx *c, int token, int pos, int n_steps, in
   if (token < 0 || token >= c->m.vocab) return fail(c, -1, "token out of range");
   if ((rc = ensure_tokens(c, n_steps))) return rc;
   Workspace &w = c->ws;
-  int st[3] = {token, pos, 0};
+  int st[4] = {token, pos, 0, 0};
   HIPCHK(c, hipMemcpyAsync(w.d_token, st, sizeof st, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (use_graph && (rc = ensure_graph(c))) return rc;
@@ -1321,12 +1352,11 @@ static int pf_ensure(gq_ctx *c, T *&p, size_t &cap, size_t n) {
  * the cache was re-made). */
 static void pf_release(gq_ctx *c) {
   PrefillWs &w = c->pf;
-  void *bufs[8] = {w.x, w.q, w.k, w.v, w.xn, w.att, w.act, w.tok};
+  void *bufs[7] = {w.x, w.q, w.k, w.v, w.xn, w.att, w.act};
   for (void *p : bufs)
     if (p) gq_hip_free(c, p);
   w.x = w.q = w.k = w.v = nullptr;
   w.xn = w.att = w.act = nullptr;
-  w.tok = nullptr;
   w.cap = w.H = w.F = w.kvd = 0;
 }
 
@@ -1345,7 +1375,6 @@ static int pf_alloc(gq_ctx *c) {
   const size_t nb[3] = {T * H, T * H, T * F};
   for (int i = 0; i < 3; i++)
     if (!(*b16[i] = (__bf16 *)dev_alloc(c, sizeof(__bf16) * nb[i]))) return -4;
-  if (!(w.tok = (int *)dev_alloc(c, sizeof(int) * T))) return -4;
   w.cap = kPrefillChunk;
   w.H = m.hidden, w.F = m.ff, w.kvd = kvd_m;
   return 0;
@@ -1471,29 +1500,42 @@ extern "C" int gq_hip_prefill(gq_ctx *c, const int32_t *tokens, int n_tokens, in
   } else {
     for (int t0 = 0; t0 < n_tokens; t0 += T) {
       T = std::min(kPrefillChunk, n_tokens - t0);
-      HIPCHK(c, hipMemcpyAsync(w.tok, tokens + t0, sizeof(int) * T, hipMemcpyHostToDevice, c->stream));
-      if ((rc = gq_launch_embed_rows(m.embed.dtype, m.embed.data, m.hidden, w.tok, T, w.x, c->stream)))
+      const int in = t0 % kPinnedTokens; /* the embedding kernel reads the tokens there */
+      if (in == 0) {
+        if (t0) HIPCHK(c, hipStreamSynchronize(c->stream)); /* the last piece has been read */
+        memcpy(c->h_in, tokens + t0, sizeof(int) * (size_t)std::min(kPinnedTokens, n_tokens - t0));
+      }
+      if ((rc = gq_launch_embed_rows(m.embed.dtype, m.embed.data, m.hidden, c->h_in + in, T, w.x, c->stream)))
         return fail(c, rc, "prefill: embed");
       int pending = 1;
       for (int l = 0; l < m.n_layers; l++)
         if ((rc = pf_layer(c, l, pos + t0, T, pending))) return fail(c, rc, "prefill: layer %d launch failed", l);
     }
     /* last token: final RMSNorm + LM head + argmax as in a decode step */
-    HIPCHK(c, hipMemcpyAsync(ws.hidden, w.x + (size_t)(T - 1) * m.hidden, sizeof(float) * m.hidden,
-                             hipMemcpyDeviceToDevice, c->stream));
-    if ((rc = op_lm_head(c, ws.hidden)) ||
+    float *last = w.x + (size_t)(T - 1) * m.hidden;
+    ArgmaxHost host{};
+    host.token = c->h_tok, host.x = logits ? c->h_out : nullptr;
+    if (hidden_last) host.row = last, host.row_out = c->h_out + m.vocab, host.row_n = m.hidden;
+    if ((rc = op_lm_head(c, last)) ||
         (rc = gq_launch_argmax(ws.logits, m.vocab, ws.amax, ws.amax_blocks, ws.d_token, nullptr, nullptr, nullptr,
-                               c->stream)))
+                               c->stream, 0, nullptr, 0, nullptr, host)))
       return fail(c, rc, "prefill: lm head");
   }
   if (ms) HIPCHK(c, hipEventRecord(ev.e1, c->stream));
   int next = -1;
-  HIPCHK(c, hipMemcpyAsync(&next, ws.d_token, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  if (logits)
-    HIPCHK(c, hipMemcpyAsync(logits, ws.logits, sizeof(float) * m.vocab, hipMemcpyDeviceToHost, c->stream));
-  if (hidden_last)
-    HIPCHK(c, hipMemcpyAsync(hidden_last, ws.hidden, sizeof(float) * m.hidden, hipMemcpyDeviceToHost, c->stream));
+  if (!gemm) {
+    HIPCHK(c, hipMemcpyAsync(&next, ws.d_token, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    if (logits)
+      HIPCHK(c, hipMemcpyAsync(logits, ws.logits, sizeof(float) * m.vocab, hipMemcpyDeviceToHost, c->stream));
+    if (hidden_last)
+      HIPCHK(c, hipMemcpyAsync(hidden_last, ws.hidden, sizeof(float) * m.hidden, hipMemcpyDeviceToHost, c->stream));
+  }
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (gemm) {
+    next = *c->h_tok;
+    if (logits) memcpy(logits, c->h_out, sizeof(float) * m.vocab);
+    if (hidden_last) memcpy(hidden_last, c->h_out + m.vocab, sizeof(float) * m.hidden);
+  }
   if (ms) *ms = ev.ms();
   return next;
 }
@@ -1743,10 +1785,7 @@ extern "C" int gq_hip_argmax_dev(gq_ctx *c, const float *x, int n, int *out_inde
 /* ---- on-device sampling (tokenizer.c:175-333, generate.c:302-311) ---- */
 static int sample_ensure(gq_ctx *c, int vocab, bool big, int top_k) {
   SampleWs &w = c->sw;
-  if (!c->h_sample && hipHostMalloc((void **)&c->h_sample, sizeof(int)) != hipSuccess) {
-    c->h_sample = nullptr;
-    return -4;
-  }
+  if (ensure_pinned(c, 0)) return -4;
   if (const size_t tb = top_k > 0 ? gq_sample_topk_bytes(vocab, top_k) : 0; tb && w.topk_cap < vocab) {
     void *p = dev_alloc(c, tb);
     if (p) { /* without it the one-workgroup replay runs */
@@ -1773,13 +1812,13 @@ static int sample_on_device(gq_ctx *c, const float *logits, int vocab, float tem
   const bool big = temperature > 0.0f && !(top_k > 0 && top_k < vocab) && top_p > 0.0f;
   int rc = sample_ensure(c, vocab, big, temperature > 0.0f && top_k < vocab ? top_k : 0);
   if (rc) return rc;
-  rc = gq_launch_sample(logits, vocab, temperature, top_k, top_p, rnd, c->sw, c->h_sample, c->stream);
+  rc = gq_launch_sample(logits, vocab, temperature, top_k, top_p, rnd, c->sw, c->h_tok, c->stream);
   if (rc == 1) { /* greedy */
     const int nblk = gq_argmax_blocks(vocab);
     float *scratch = c->ws.amax && c->ws.amax_blocks >= nblk ? c->ws.amax
                                                              : (float *)dev_alloc(c, sizeof(float) * 2 * nblk);
     if (!scratch) return -4;
-    rc = gq_launch_argmax(logits, vocab, scratch, nblk, c->h_sample, nullptr, nullptr, nullptr, c->stream);
+    rc = gq_launch_argmax(logits, vocab, scratch, nblk, c->h_tok, nullptr, nullptr, nullptr, c->stream);
     if (scratch != c->ws.amax) {
       (void)hipStreamSynchronize(c->stream);
       gq_hip_free(c, scratch);
@@ -1788,7 +1827,7 @@ static int sample_on_device(gq_ctx *c, const float *logits, int vocab, float tem
   if (rc == -2) return fail(c, -2, "top_k %d above the device limit %d", top_k, kMaxTopK);
   if (rc) return fail(c, rc, "sampling launch failed");
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  return *c->h_sample;
+  return *c->h_tok;
 }
 
 extern "C" int gq_hip_sample_dev(gq_ctx *c, const float *logits, int vocab, float temperature, int top_k,
@@ -1804,10 +1843,10 @@ extern "C" int gq_hip_forward_sample(gq_ctx *c, int token, int pos, float temper
   if (rc) return rc;
   if (token < 0 || token >= c->m.vocab) return fail(c, -1, "token %d out of range", token);
   if (temperature <= 0.0f) { /* greedy: the step's own argmax */
-    if ((rc = graph_step(c, token, pos))) return rc;
+    if ((rc = graph_step(c, token, pos, false))) return rc;
     return graph_step_token(c, pos, nullptr);
   }
-  if ((rc = graph_step(c, token, pos))) return rc;
+  if ((rc = graph_step(c, token, pos, false))) return rc;
   /* the sampled token generally differs from the argmax the replay embedded */
   const int next = sample_on_device(c, c->ws.logits, c->m.vocab, temperature, top_k, top_p, rnd);
   c->g_valid = false; /* the replay embedded its argmax, not the sampled token */
