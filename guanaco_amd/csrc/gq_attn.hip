@@ -370,21 +370,20 @@ typedef __bf16 gq_bf2a __attribute__((ext_vector_type(2)));
  * needed 312, one wave per SIMD, and ran 1.25-1.4x slower).  Same mathematics as the reference (engine.c:476-501:
  * scores * 1/sqrt(hd), -inf past the query position, softmax, P V) in fp32
  * throughout; only the summation order differs. */
+template <int HD>
+struct FlashLds { /* the waves' (max, sum, O) on their way to wave 0 */
+  float xm[3][64], xl[3][64], xo[3][HD / 16 * 4][64];
+};
+
 template <int HD, int G>
-__global__ __launch_bounds__(256) void flash_prefill_kernel(AttnArgs a) {
+__device__ __forceinline__ void flash_tile(const AttnArgs &a, int g, int t0, FlashLds<HD> &lds) {
   constexpr int TPT = 16 / G; /* tokens per tile */
   constexpr int NS = HD / 4;  /* QK^T MFMA steps */
   constexpr int ND = HD / 16; /* output tiles over the head dimension */
-  __shared__ float xm[3][64], xl[3][64], xo[3][ND * 4][64];
+  auto &xm = lds.xm, &xl = lds.xl;
+  auto &xo = lds.xo;
   const int lane = threadIdx.x & 63, c = lane & 15, j = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  /* One linear grid: workgroup L runs on XCD L mod 8, and takes KV head
-   * L mod n_kv, so a head's K/V stays in one XCD's L2 (n_kv = 8: one head
-   * per XCD; with tile-major ids every XCD read every head's K/V, 4 MB at
-   * 512 tokens: 49.3 -> 38.6 us per layer).  Heavy (late) tiles first. */
-  const int ntile = gridDim.x / a.n_kv;
-  const int g = blockIdx.x % a.n_kv, tile = ntile - 1 - blockIdx.x / a.n_kv;
-  const int t0 = tile * TPT;
   const int last = min(t0 + TPT, a.ntok) - 1;
   const int pmax = a.pos + last; /* last key any row of the tile needs */
   /* B operand of S^T: row c's query, dims NS j .. NS j + NS - 1 */
@@ -535,10 +534,303 @@ __global__ __launch_bounds__(256) void flash_prefill_kernel(AttnArgs a) {
   }
 }
 
+/* One linear grid: workgroup L runs on XCD L mod 8, and takes KV head
+ * L mod n_kv, so a head's K/V stays in one XCD's L2 (n_kv = 8: one head
+ * per XCD; with tile-major ids every XCD read every head's K/V, 4 MB at
+ * 512 tokens: 49.3 -> 38.6 us per layer).  Heavy (late) tiles first. */
+template <int HD, int G>
+__global__ __launch_bounds__(256) void flash_prefill_kernel(AttnArgs a) {
+  __shared__ FlashLds<HD> lds;
+  const int ntile = gridDim.x / a.n_kv;
+  const int g = blockIdx.x % a.n_kv, tile = ntile - 1 - blockIdx.x / a.n_kv;
+  flash_tile<HD, G>(a, g, tile * (16 / G), lds);
+}
+
+/* The same attention on the bf16 matrix cores without giving up fp32: every
+ * fp32 operand x is the sum of three bf16 numbers, hi = bf16(x), mid =
+ * bf16(x - hi), lo = bf16(x - hi - mid) (8 + 8 + 8 bits of a 24-bit
+ * significand), and a product keeps the six of the nine partial products that
+ * are not below 2^-24 of it: hi hi + (hi mid + mid hi) + (hi lo + lo hi + mid
+ * mid), each exact, summed in fp32.  bf16 products run 16 times as fast as
+ * fp32 ones (v_mfma_f32_16x16x4_f32), so six of them cost 0.38 of one.
+ *
+ * One workgroup of four waves takes 64 query rows = 64 / G tokens x the G
+ * query heads of a KV head, and streams the keys in blocks of 64: wave (rg,
+ * kh) rows 32 rg .. + 31 against keys 32 kh .. + 31 of every block, online
+ * softmax, the two halves of the keys combined at the end.  K and V are
+ * loaded once per workgroup a block ahead into registers, split, and put into
+ * LDS as three bf16 planes each (96 KB at head_dim 128):
+ *   S^T = K Q^T   A = K planes [key][dim], B = Q planes, in registers for the
+ *                 whole kernel; lane (r, h) = (lane % 32, lane / 32) gets row
+ *                 r's scores of keys 8 a + 4 h + c (a, c < 4)
+ *   O^T += V^T P^T  B = the probabilities straight from that layout: the 16
+ *                 keys of a step are taken in the order in which a lane holds
+ *                 them, and V is stored [dim][key] in the same order; lane
+ *                 (r, h) holds row r's output dims, so the softmax's rescale
+ *                 and the final division need no exchange between lanes.
+ * Octets (8 bf16, 16 bytes) are XOR-swizzled by the row, so operand reads
+ * are free of bank conflicts.
+ *
+ * 32 heads over 8, head_dim 128, 512 tokens at 3584: 383 -> 270 us with RoPE
+ * and append (118 TFLOP/s of fp32 products), the error against float64 6e-7
+ * -> 2.8e-7.  Bound by the vector work between the matrix instructions (one
+ * wave per SIMD: splitting 64 values and 16 exponentials a lane per block
+ * beside 96 MFMAs).
+ *
+ * An infinity or NaN among the operands leaves NaN in the splits and so in
+ * the outputs it reaches; a tile with such an output is computed again by
+ * flash_tile, which treats them as fp32 arithmetic does. */
+typedef __bf16 gq_bf8a __attribute__((ext_vector_type(8)));
+typedef float gq_f16a __attribute__((ext_vector_type(16)));
+
+constexpr int kFsKeys = 64, kFsRows = 64;
+/* Fewer workgroups than this leave most of the chip idle, and the fp32
+ * kernel's 16-row tiles win: at 77 tokens x 32 heads (40 workgroups, 378 keys)
+ * it takes 10 us where this one would take 6 blocks x 4.4. */
+constexpr int kFsMinWgs = 96;
+
+/* two floats to their (hi, mid, lo) bf16 pairs, each rounded to nearest even */
+__device__ __forceinline__ void split3(float x, float y, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2a){x, y}, gq_bf2a));
+  x -= __builtin_bit_cast(float, hi << 16), y -= __builtin_bit_cast(float, hi & 0xffff0000u);
+  mid = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2a){x, y}, gq_bf2a));
+  x -= __builtin_bit_cast(float, mid << 16), y -= __builtin_bit_cast(float, mid & 0xffff0000u);
+  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2a){x, y}, gq_bf2a));
+}
+
+struct Split8 {
+  uint4 p[3];
+};
+__device__ __forceinline__ Split8 split8(const float (&x)[8]) {
+  Split8 s;
+  split3(x[0], x[1], s.p[0].x, s.p[1].x, s.p[2].x);
+  split3(x[2], x[3], s.p[0].y, s.p[1].y, s.p[2].y);
+  split3(x[4], x[5], s.p[0].z, s.p[1].z, s.p[2].z);
+  split3(x[6], x[7], s.p[0].w, s.p[1].w, s.p[2].w);
+  return s;
+}
+
+/* the pairs of planes whose product is kept: the small ones, and last hi hi */
+constexpr int kFsA[6] = {1, 2, 0, 1, 0, 0}, kFsB[6] = {1, 0, 2, 0, 1, 0};
+
+template <int HD, int G>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void flash_split_kernel(AttnArgs a) {
+  constexpr int TPT = kFsRows / G;       /* tokens per workgroup */
+  constexpr int NO = HD / 8;             /* octets of a K row */
+  constexpr int NSL = HD / 16;           /* dim slices of S^T */
+  constexpr int ND = HD / 32;            /* dim tiles of O^T */
+  constexpr int KPL = kFsKeys * HD * 2;  /* bytes of one K (or V) plane */
+  constexpr int KT = kFsKeys * NO / 256; /* K octets per thread */
+  constexpr int VTH = kFsKeys / 8 * HD / 4; /* threads with a V task: 8 keys x 4 dims */
+  static_assert(6 * KPL >= (int)sizeof(FlashLds<HD>) && 6 * KPL >= 2 * 64 * 4 * (ND * 16 + 2), "exchanges fit the planes");
+  __shared__ __attribute__((aligned(16))) uint8_t smem_[6 * KPL];
+  __shared__ int s_nan;
+  GQ_LDS uint8_t *smem = (GQ_LDS uint8_t *)smem_;
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), rg = wv >> 1, kh = wv & 1;
+  const int ntile = gridDim.x / a.n_kv; /* heads and tiles as in flash_prefill_kernel */
+  const int g = blockIdx.x % a.n_kv, tile = ntile - 1 - blockIdx.x / a.n_kv, t0 = tile * TPT;
+  const int pmax = a.pos + min(t0 + TPT, a.ntok) - 1; /* last key any row of the tile needs */
+  const int nblk = pmax / kFsKeys + 1;
+  const float *K = a.k + (size_t)g * a.max_seq * HD;
+  const float *V = a.v + (size_t)g * a.max_seq * HD;
+  if (tid == 0) s_nan = 0;
+  /* this lane's query row: token t0 + row / G, head g G + row % G */
+  const int row = 32 * rg + r, qt = min(t0 + row / G, a.ntok - 1), qh = g * G + row % G;
+  const int cpos = a.pos + t0 + row / G;
+  Split8 q[NSL]; /* dims 16 s + 8 h .. + 7 */
+#pragma unroll
+  for (int s = 0; s < NSL; s++) {
+    const float *qp = a.q + (size_t)qt * a.q_stride + (size_t)qh * HD + 16 * s + 8 * h;
+    const float4 u = gld<float4>(qp), v = gld<float4>(qp + 4);
+    const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+    q[s] = split8(x);
+  }
+  /* K tasks: octet ko of keys tid / NO + (256 / NO) i; V task: dims 4 vd ..
+   * of the eight keys of octet vo, in P's order: key octet 4 kh + 2 t + h is
+   * keys 32 kh + 16 t + 4 h + {0..3, 8..11} */
+  const int ko = tid % NO, kk = tid / NO;
+  const int vd = tid % (HD / 4), vo = (tid / (HD / 4)) & 7;
+  const int vkey = 32 * (vo >> 2) + 16 * ((vo >> 1) & 1) + 4 * (vo & 1);
+  float4 kr[KT][2], vr[8];
+  auto load = [&](int b) {
+    const int key0 = b * kFsKeys;
+#pragma unroll
+    for (int i = 0; i < KT; i++) {
+      const float *kp = K + (size_t)min(key0 + kk + 256 / NO * i, pmax) * HD + 8 * ko;
+      kr[i][0] = gld<float4>(kp), kr[i][1] = gld<float4>(kp + 4);
+    }
+    if (VTH == 256 || tid < VTH) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) /* keys past pmax repeat it: their weight is 0 */
+        vr[e] = gld<float4>(V + (size_t)min(key0 + vkey + (e & 3) + 8 * (e >> 2), pmax) * HD + 4 * vd);
+    }
+  };
+  auto stage = [&]() {
+#pragma unroll
+    for (int i = 0; i < KT; i++) {
+      const float x[8] = {kr[i][0].x, kr[i][0].y, kr[i][0].z, kr[i][0].w, kr[i][1].x, kr[i][1].y, kr[i][1].z, kr[i][1].w};
+      const Split8 s = split8(x);
+      const int key = kk + 256 / NO * i;
+      const uint32_t at = (uint32_t)(key * HD * 2 + ((ko ^ (key & (NO - 1))) << 4));
+#pragma unroll
+      for (int p = 0; p < 3; p++) lst<uint4>(smem, (uint32_t)(p * KPL) + at, s.p[p]);
+    }
+    if (VTH == 256 || tid < VTH) {
+#pragma unroll
+      for (int d = 0; d < 4; d++) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[e] = d == 0 ? vr[e].x : d == 1 ? vr[e].y : d == 2 ? vr[e].z : vr[e].w;
+        const Split8 s = split8(x);
+        const int dim = 4 * vd + d;
+        const uint32_t at = (uint32_t)(3 * KPL + dim * kFsKeys * 2 + ((vo ^ ((dim ^ (dim >> 3)) & 7)) << 4));
+#pragma unroll
+        for (int p = 0; p < 3; p++) lst<uint4>(smem, (uint32_t)(p * KPL) + at, s.p[p]);
+      }
+    }
+  };
+  /* operand addresses: K row 32 kh + r, octet 2 s + h; V row 32 d + r, octet
+   * 4 kh + 2 t + h */
+  const int krow = 32 * kh + r;
+  float m = -INFINITY, l = 0.f;
+  gq_f16a o[ND];
+#pragma unroll
+  for (int d = 0; d < ND; d++) o[d] = gq_f16a{};
+  load(0);
+  for (int b = 0; b < nblk; b++) {
+    __syncthreads(); /* the planes are free */
+    stage();
+    __syncthreads();
+    if (b + 1 < nblk) load(b + 1);
+    const int key0 = b * kFsKeys + 32 * kh;
+    if (key0 > pmax) continue; /* none of this wave's keys (uniform in the wave) */
+    gq_f16a sa = gq_f16a{}, sb = gq_f16a{};
+#pragma unroll
+    for (int s = 0; s < NSL; s++) {
+      gq_bf8a kv[3];
+#pragma unroll
+      for (int p = 0; p < 3; p++)
+        kv[p] = lld<gq_bf8a>(smem, (uint32_t)(p * KPL + krow * HD * 2 + (((2 * s + h) ^ (krow & (NO - 1))) << 4)));
+#pragma unroll
+      for (int u = 0; u < 6; u++) {
+        const gq_bf8a qv = __builtin_bit_cast(gq_bf8a, q[s].p[kFsB[u]]);
+        if (u < 5) sb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kv[kFsA[u]], qv, sb, 0, 0, 0);
+        else sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kv[kFsA[u]], qv, sa, 0, 0, 0);
+      }
+    }
+    /* scores of keys key0 + 8 (e / 4) + 4 h + e % 4 */
+    float p[16], mb = -INFINITY;
+    if (key0 + 31 <= a.pos + t0) { /* every row sees every key of this half block */
+#pragma unroll
+      for (int e = 0; e < 16; e++) p[e] = (sa[e] + sb[e]) * a.scale;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 16; e++)
+        p[e] = key0 + 8 * (e >> 2) + 4 * h + (e & 3) <= cpos ? (sa[e] + sb[e]) * a.scale : -INFINITY;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; e++) mb = fmaxf(mb, p[e]);
+    mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
+    /* a half may hold no visible key of a row yet: m stays -inf, weight 0 */
+    const float mn = fmaxf(m, mb), ms = mn == -INFINITY ? 0.f : mn;
+    const float alpha = __expf(m - ms);
+    float lb = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      p[e] = __expf(p[e] - ms);
+      lb += p[e];
+    }
+    lb += __shfl_xor(lb, 32, 64);
+    l = __builtin_fmaf(l, alpha, lb);
+    m = mn;
+    Split8 ps[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      float x[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) x[e] = p[8 * t + e];
+      ps[t] = split8(x);
+    }
+    /* the half block's P V in accumulators of its own: O takes one rounding
+     * per 32 keys (twelve with O itself as the accumulator, and the error
+     * over 4096 keys was above the fp32 kernel's) */
+#pragma unroll
+    for (int d = 0; d < ND; d++) {
+      gq_f16a pv = gq_f16a{};
+      const int dim = 32 * d + r;
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        const int oct = 4 * kh + 2 * t + h;
+        gq_bf8a vv[3];
+#pragma unroll
+        for (int q3 = 0; q3 < 3; q3++)
+          vv[q3] = lld<gq_bf8a>(smem, (uint32_t)((3 + q3) * KPL + dim * kFsKeys * 2 + ((oct ^ ((dim ^ (dim >> 3)) & 7)) << 4)));
+#pragma unroll
+        for (int u = 0; u < 6; u++)
+          pv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv[kFsA[u]], __builtin_bit_cast(gq_bf8a, ps[t].p[kFsB[u]]), pv, 0, 0, 0);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; e++) o[d][e] = __builtin_fmaf(o[d][e], alpha, pv[e]);
+    }
+  }
+  /* the two halves of the keys: kh = 1 hands (m, l, O) to kh = 0, whose first
+   * block holds key 0, so its m is finite */
+  __syncthreads();
+  GQ_LDS float *x = (GQ_LDS float *)smem + rg * 64 * (ND * 16 + 2);
+  if (kh == 1) {
+    x[lane] = m, x[64 + lane] = l;
+#pragma unroll
+    for (int d = 0; d < ND; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) x[64 * (2 + 16 * d + e) + lane] = o[d][e];
+  }
+  __syncthreads();
+  if (kh == 0) {
+    const float m1 = x[lane], mt = fmaxf(m, m1), s0 = __expf(m - mt), s1 = __expf(m1 - mt);
+    const float inv = 1.0f / (l * s0 + x[64 + lane] * s1);
+    const int t = t0 + row / G;
+    bool nan = false;
+#pragma unroll
+    for (int d = 0; d < ND; d++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) { /* dims 32 d + 8 c + 4 h .. + 3 */
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          y[e] = (o[d][4 * c + e] * s0 + x[64 * (2 + 16 * d + 4 * c + e) + lane] * s1) * inv;
+          nan |= y[e] != y[e];
+        }
+        if (t < a.ntok) {
+          const size_t at = (size_t)t * a.out_stride + (size_t)qh * HD + 32 * d + 8 * c + 4 * h;
+          if (a.out16) {
+            uint2 u;
+            u.x = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2a){y[0], y[1]}, gq_bf2a));
+            u.y = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2a){y[2], y[3]}, gq_bf2a));
+            gst<uint2>(a.out16 + at, u);
+          } else {
+            gst<float4>(a.out + at, make_float4(y[0], y[1], y[2], y[3]));
+          }
+        }
+      }
+    if (__ballot(nan) && lane == 0) s_nan = 1;
+  }
+  __syncthreads();
+  if (!s_nan) return;
+  for (int t = t0; t < min(t0 + TPT, a.ntok); t += 16 / G) {
+    flash_tile<HD, G>(a, g, t, *(FlashLds<HD> *)smem_);
+    __syncthreads();
+  }
+}
+
 template <int HD, int G>
 int launch_flash(const AttnArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL((flash_prefill_kernel<HD, G>), dim3((a.ntok + 16 / G - 1) / (16 / G) * a.n_kv), dim3(256), 0, s,
-                     a);
+  const int wide = (a.ntok + kFsRows / G - 1) / (kFsRows / G) * a.n_kv;
+  if (wide >= kFsMinWgs)
+    hipLaunchKernelGGL((flash_split_kernel<HD, G>), dim3(wide), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((flash_prefill_kernel<HD, G>), dim3((a.ntok + 16 / G - 1) / (16 / G) * a.n_kv), dim3(256), 0, s,
+                       a);
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 

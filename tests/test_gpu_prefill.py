@@ -255,6 +255,12 @@ def test_prefill_gate_up_wide_tile(ctx, orc, T, N, K):
     (8, 8, 64, 0, 3, 16),          # G = 1, three tokens
     (64, 8, 128, 7, 33, 64),       # G = 8, two tokens per tile
     (16, 8, 64, 1, 21, 40),        # G = 2
+    # 96 workgroups of 64 rows and more: the split-bf16 kernel
+    (32, 4, 64, 77, 200, 277),     # G = 8, ragged last tile, ends at the cache end
+    (32, 32, 64, 3, 190, 200),     # G = 1, 64 tokens per tile
+    (32, 32, 128, 64, 129, 200),   # one token in the last tile
+    (64, 8, 128, 63, 97, 160),     # the first key of a block is the last one seen
+    (64, 32, 64, 0, 65, 65),       # G = 2, one token past a tile
 ])
 def test_prefill_attention(ctx, orc, nh, nkv, hd, pre, T, ms):
     from oracle import HostKV, fptr
@@ -297,6 +303,51 @@ def test_prefill_attention(ctx, orc, nh, nkv, hd, pre, T, ms):
             assert rel_l2(out[t], o1.download()) < 1e-5, t
     for b in (qb, kb, vb, ob, q1, o1):
         b.free()
+
+
+@pytest.mark.parametrize("bad", ["none", "k_inf", "v_inf", "v_nan", "q_nan", "huge"])
+def test_prefill_attention_wide_equals_narrow(ctx, bad):
+    """One launch over 256 tokens (the split-bf16 kernel) against the same
+    tokens in launches of 32 (the fp32 kernel): finite outputs to fp32
+    rounding, and exactly the same non-finite ones, for which the wide kernel
+    has to fall back to fp32 arithmetic."""
+    nh, nkv, hd, T, ms = 32, 8, 128, 256, 320
+    rng = np.random.default_rng(5)
+    q = rng.standard_normal((T, nh * hd)).astype(np.float32)
+    k = rng.standard_normal((T, nkv * hd)).astype(np.float32)
+    v = rng.standard_normal((T, nkv * hd)).astype(np.float32)
+    if bad == "k_inf":
+        k[70, 3 * hd + 6] = np.inf
+    elif bad == "v_inf":
+        v[131, 2 * hd + 5] = -np.inf
+    elif bad == "v_nan":
+        v[9, 7 * hd + 127] = np.nan
+    elif bad == "q_nan":
+        q[200, 11 * hd] = np.nan
+    elif bad == "huge":  # rounds to an infinite bf16
+        v[40, 0] = np.float32(3.4e38)
+    got = []
+    for step in (T, 32):
+        ctx.kv_init(1, nkv, hd, ms, 500000.0)
+        out = []
+        for t in range(0, T, step):
+            qb, kb, vb = (ctx.upload(a[t:t + step]) for a in (q, k, v))
+            ob = ctx.alloc(4 * step * nh * hd)
+            assert ctx.prefill_attention_dev(0, t, step, nh, qb, kb, vb, ob) == 0
+            out.append(ob.download(count=step * nh * hd).reshape(step, nh * hd))
+            for b in (qb, kb, vb, ob):
+                b.free()
+        got.append(np.concatenate(out))
+    wide, narrow = got
+    assert np.array_equal(np.isnan(wide), np.isnan(narrow))
+    fin = np.isfinite(narrow)
+    assert np.array_equal(np.isfinite(wide), fin) and np.array_equal(wide[~fin & ~np.isnan(wide)], narrow[~fin & ~np.isnan(wide)])
+    assert np.isnan(narrow).any() == (bad not in ("none", "huge"))
+    if bad != "huge":
+        assert rel_l2(wide[fin], narrow[fin]) < 2e-6
+    else:  # the column that holds it, and the rest
+        c = np.abs(narrow).max(axis=0) > 1e30
+        assert c.any() and rel_l2(wide[:, c] / 1e30, narrow[:, c] / 1e30) < 2e-6 and rel_l2(wide[:, ~c], narrow[:, ~c]) < 2e-6
 
 
 def test_prefill_attention_rejects_bad_positions(ctx):
