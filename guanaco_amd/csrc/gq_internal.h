@@ -300,13 +300,37 @@ struct PgArgs {
   int kparts, rows_total; /* set by the launcher */
   /* a launch with kparts_out set leaves the parts' sum (and for RESID the
    * residual add) to its caller when it splits, writing the number of parts
-   * there (1: not split, y is final) */
+   * there (0: y is final) */
   int *kparts_out;
 };
 int gq_launch_pgemm(int mode, const PgArgs &a, hipStream_t s);
 /* at most this many K parts in a split launch: PgArgs.part needs
  * kPgKParts * T * (all segments' rows) floats */
 constexpr int kPgKParts = 4;
+/* y = (y +) the sum of a split launch's parts, scattered to its segments
+ * (seg[].y / rows, nseg, T, part, kparts, rows_total) */
+int gq_launch_parts(const PgArgs &a, bool resid, hipStream_t s);
+
+/* The GEMM on a bf16 copy of the weights (gq_dense.hip): the outputs, K parts
+ * and workspace of PgArgs; rows[] with y[] per segment, or for MV_SWIGLU
+ * rows[0] rows of act. */
+struct DnArgs {
+  const __bf16 *x;
+  const uint8_t *w; /* gq_launch_dense_tile's copies of the segments, in order */
+  __bf16 *act;
+  float *y[3];
+  int rows[3];
+  int nseg, T, K;
+  float *part;
+  size_t part_cap;
+  int kparts, rows_total; /* set by the launcher */
+  bool to_parts;          /* likewise: the sums go to part */
+  int *kparts_out;
+};
+int gq_launch_dense(int mode, const DnArgs &a, int n_cu, hipStream_t s);
+/* bytes of the copy of rows x K weights (swiglu: of gate and up together) */
+size_t gq_dense_bytes(int rows, int K, bool swiglu);
+int gq_launch_dense_tile(void *dst, int dtype, const void *w0, const void *w1, int rows, int K, hipStream_t s);
 int gq_launch_to_bf16(const float *x, __bf16 *y, size_t n, hipStream_t s);
 /* RMSNorm of `rows` consecutive rows of dim floats, one workgroup per row;
  * out16 != NULL writes bf16 there instead of fp32 to out.  parts != NULL

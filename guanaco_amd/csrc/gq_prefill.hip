@@ -908,7 +908,7 @@ template <int MODE>
 int launch_mode(const PgArgs &a0, int row_tiles, hipStream_t s) {
   PgArgs a = a0;
   a.kparts = 1;
-  if (a.kparts_out) *a.kparts_out = 1;
+  if (a.kparts_out) *a.kparts_out = 0;
   /* Q4_K gate/up whose 128-row tiles alone give every CU a workgroup: the
    * wide tile */
   if (MODE == MV_SWIGLU && a.seg[0].dtype == GQ_Q4_K && a.seg[0].rows % 128 == 0 &&
@@ -959,10 +959,7 @@ int launch_mode(const PgArgs &a0, int row_tiles, hipStream_t s) {
       *a.kparts_out = KP;
       return 0;
     }
-    const size_t n4 = (size_t)a.T * a.rows_total / 4;
-    hipLaunchKernelGGL(pg_parts_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, a, n4,
-                       MODE == MV_RESID ? 1 : 0);
-    return hipGetLastError() == hipSuccess ? 0 : -4;
+    return gq_launch_parts(a, MODE == MV_RESID, s);
   }
   const int tt = !q6 && tiles4 >= n_cus() ? 4 : 2;
   const int wgs = row_tiles * ((a.T + 32 * tt - 1) / (32 * tt));
@@ -1017,6 +1014,12 @@ int gq_launch_pgemm(int mode, const PgArgs &a, hipStream_t s) {
   if (mode == MV_RESID) return launch_mode<MV_RESID>(a, tiles, s);
   if (mode == MV_STORE) return launch_mode<MV_STORE>(a, tiles, s);
   return -1;
+}
+
+int gq_launch_parts(const PgArgs &a, bool resid, hipStream_t s) {
+  const size_t n4 = (size_t)a.T * a.rows_total / 4;
+  hipLaunchKernelGGL(pg_parts_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, a, n4, resid ? 1 : 0);
+  return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
 int gq_launch_to_bf16(const float *x, __bf16 *y, size_t n, hipStream_t s) {

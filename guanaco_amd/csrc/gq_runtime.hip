@@ -49,11 +49,16 @@ struct PrefillWs {
   size_t part_cap = 0;
 };
 
-/* tokens per prefill chunk */
-constexpr int kPrefillChunk = 512;
+/* Tokens per prefill chunk, at most: the GEMMs' workgroups then come in more,
+ * fuller rounds and the weights are read once per chunk (1500 tokens of the
+ * 8B shape on the quantized weights: 41.0 ms in chunks of 512, 38.3 in one).
+ * The activations are sized for the longest chunk seen, in steps of 512. */
+constexpr int kPrefillChunk = 2048;
+/* chunks of at least this many tokens multiply by the bf16 copies */
+constexpr int kDenseTokens = 256;
 /* prompt tokens that gq_ctx::h_in holds: a prompt is embedded in pieces of at
  * most that many */
-constexpr int kPinnedTokens = 16 * kPrefillChunk;
+constexpr int kPinnedTokens = 4 * kPrefillChunk;
 
 } // namespace
 
@@ -92,6 +97,11 @@ struct gq_ctx {
     /* Q6_K projections in the same unit layout for the prefill GEMM (cols %
      * 2048): wq, wk, wv, wo, gate, up, down; ux[6] is dx itself */
     const uint8_t *ux[7] = {};
+    /* bf16 copies for prompts of many tokens (gq_launch_dense_tile), one
+     * allocation: q | k | v, o, gate + up, down; NULL: the quantized weights
+     * serve every prompt */
+    uint8_t *dn = nullptr;
+    size_t dn_at[4] = {};
   };
   std::vector<MmLayer> mm;
   const uint8_t *mm_lm = nullptr;
@@ -820,10 +830,40 @@ static void mm_free(gq_ctx *c) {
   for (auto &L : c->mm) {
     if (L.ux[6] == L.dx) L.ux[6] = nullptr; /* one allocation */
     rel(L.gu), rel(L.dx);
+    if (L.dn) gq_hip_free(c, L.dn);
+    L.dn = nullptr;
     for (auto &p : L.ux) rel(p);
   }
   c->mm.clear();
   rel(c->mm_lm);
+}
+
+static bool pf_gemm_ok(const gq_weight &w);
+
+/* The bf16 copy of layer l's projections for prompts of many tokens; left
+ * out (dn NULL) where the GEMM does not take the layer or memory is short. */
+static void dense_build(gq_ctx *c, int l) {
+  const gq_layer &L = c->layers[l];
+  const gq_weight *ws[7] = {&L.wq, &L.wk, &L.wv, &L.wo, &L.w_gate, &L.w_up, &L.w_down};
+  for (const gq_weight *w : ws)
+    if (!pf_gemm_ok(*w)) return;
+  if (L.w_gate.dtype != L.w_up.dtype) return;
+  auto &M = c->mm[l];
+  size_t at[8], n = 0; /* q, k, v, o, gate + up, (up), down */
+  for (int i = 0; i < 7; i++) {
+    at[i] = n;
+    if (i != 5) n += gq_dense_bytes(ws[i]->rows, ws[i]->cols, i == 4);
+  }
+  M.dn = (uint8_t *)dev_alloc(c, n);
+  if (!M.dn) return;
+  M.dn_at[0] = 0, M.dn_at[1] = at[3], M.dn_at[2] = at[4], M.dn_at[3] = at[6];
+  for (int i = 0; i < 7; i++)
+    if (i != 5 && gq_launch_dense_tile(M.dn + at[i], ws[i]->dtype, ws[i]->data, i == 4 ? L.w_up.data : nullptr,
+                                       ws[i]->rows, ws[i]->cols, c->stream)) {
+      gq_hip_free(c, M.dn);
+      M.dn = nullptr;
+      return;
+    }
 }
 
 extern "C" int gq_hip_model_bind(gq_ctx *c, const gq_model *m) {
@@ -909,6 +949,17 @@ extern "C" int gq_hip_model_bind(gq_ctx *c, const gq_model *m) {
       if (d && gq_launch_q6k_units(d, g.data, g.rows, g.cols, c->stream) == 0) c->mm[l].ux[i] = d;
       else if (d) gq_hip_free(c, d);
     }
+  }
+  /* bf16 copies for prompts of many tokens, only while they take less than a
+   * quarter of the memory that is free (2 bytes a weight: 14 GB at the 8B
+   * shape): a program that fills the card keeps the room it had */
+  if (c->whole) {
+    size_t need = 0, fr = 0, tot = 0;
+    for (int l = 0; l < m->n_layers; l++)
+      need += gq_dense_bytes(H, H, false) * 2 + gq_dense_bytes(kvd, H, false) * 2 + gq_dense_bytes(F, H, true) +
+              gq_dense_bytes(H, F, false);
+    if (hipMemGetInfo(&fr, &tot) == hipSuccess && need < fr / 4)
+      for (int l = 0; l < m->n_layers; l++) dense_build(c, l);
   }
   if (has_lm) {
     const gq_weight *lm[1] = {&m->lm_head};
@@ -1360,13 +1411,14 @@ static void pf_release(gq_ctx *c) {
   w.cap = w.H = w.F = w.kvd = 0;
 }
 
-static int pf_alloc(gq_ctx *c) {
+static int pf_alloc(gq_ctx *c, int tokens) {
   PrefillWs &w = c->pf;
   const gq_model &m = c->m;
   const int kvd_m = m.n_kv_heads * m.head_dim;
-  if (w.cap && w.H == m.hidden && w.F == m.ff && w.kvd == kvd_m) return 0;
+  if (w.cap >= tokens && w.H == m.hidden && w.F == m.ff && w.kvd == kvd_m) return 0;
   pf_release(c);
-  const size_t T = kPrefillChunk, H = m.hidden, F = m.ff, kvd = (size_t)kvd_m;
+  tokens = (tokens + 511) / 512 * 512;
+  const size_t T = tokens, H = m.hidden, F = m.ff, kvd = (size_t)kvd_m;
   float **f32[4] = {&w.x, &w.q, &w.k, &w.v};
   const size_t nf[4] = {T * H, T * H, T * kvd, T * kvd};
   for (int i = 0; i < 4; i++)
@@ -1375,7 +1427,7 @@ static int pf_alloc(gq_ctx *c) {
   const size_t nb[3] = {T * H, T * H, T * F};
   for (int i = 0; i < 3; i++)
     if (!(*b16[i] = (__bf16 *)dev_alloc(c, sizeof(__bf16) * nb[i]))) return -4;
-  w.cap = kPrefillChunk;
+  w.cap = tokens;
   w.H = m.hidden, w.F = m.ff, w.kvd = kvd_m;
   return 0;
 }
@@ -1408,11 +1460,11 @@ static PgSeg pg_seg(const gq_ctx *c, int l, int i, const gq_weight &w, float *y)
  * k/v: T x n_kv*hd), then causal attention of the T tokens into out (fp32)
  * or out16 (bf16), T x n_heads*hd */
 static int pf_attention(gq_ctx *c, int layer, int pos, int T, int n_heads, float *q, const float *k, const float *v,
-                        float *out, __bf16 *out16, int kparts = 1) {
+                        float *out, __bf16 *out16, int kparts = 0) {
   const int hd = c->kv_hd, kvd = c->kv_heads * hd, qd = n_heads * hd;
   RopeArgs ra{q, k, v, gq_hip_kv_k(c, layer), gq_hip_kv_v(c, layer), c->rope, nullptr, pos,
               n_heads, c->kv_heads, hd, c->kv_max_seq, T, qd, kvd, kvd};
-  if (kparts > 1) /* q, k, v are still the q/k/v GEMM's K parts */
+  if (kparts > 0) /* q, k, v are still the q/k/v GEMM's K parts */
     ra.parts = c->pf.part, ra.kparts = kparts, ra.prow = qd + 2 * kvd, ra.pstride = (size_t)T * (qd + 2 * kvd);
   int rc = gq_launch_rope_append(ra, c->stream);
   if (rc) return rc;
@@ -1437,7 +1489,7 @@ static void pf_parts(gq_ctx *c, PgArgs &a) {
 }
 
 /* pending: K parts of the previous layer's down launch still to be added
- * into the residual x (1: none); this layer's first RMSNorm adds them, and
+ * into the residual x (0: none); this layer's first RMSNorm adds them, and
  * this layer leaves its own down's parts the same way unless it is the
  * last */
 static int pf_layer(gq_ctx *c, int l, int pos, int T, int &pending) {
@@ -1445,31 +1497,41 @@ static int pf_layer(gq_ctx *c, int l, int pos, int T, int &pending) {
   const gq_layer &L = c->layers[l];
   PrefillWs &w = c->pf;
   int rc;
-  PgArgs qkv{}, o{}, gu{}, dn{};
-  qkv.T = o.T = gu.T = dn.T = T;
+  PgArgs qkv{}, o{}, gu{}, down{};
+  qkv.T = o.T = gu.T = down.T = T;
   qkv.x = w.xn, qkv.K = m.hidden, qkv.nseg = 3;
   qkv.seg[0] = pg_seg(c, l, 0, L.wq, w.q), qkv.seg[1] = pg_seg(c, l, 1, L.wk, w.k);
   qkv.seg[2] = pg_seg(c, l, 2, L.wv, w.v);
   o.x = w.att, o.K = m.hidden, o.nseg = 1, o.seg[0] = pg_seg(c, l, 3, L.wo, w.x);
   gu.x = w.xn, gu.K = m.hidden, gu.nseg = 2, gu.act = w.act;
   gu.seg[0] = pg_seg(c, l, 4, L.w_gate, nullptr), gu.seg[1] = pg_seg(c, l, 5, L.w_up, nullptr);
-  dn.x = w.act, dn.K = m.ff, dn.nseg = 1, dn.seg[0] = pg_seg(c, l, 6, L.w_down, w.x);
-  pf_parts(c, qkv), pf_parts(c, o), pf_parts(c, dn);
+  down.x = w.act, down.K = m.ff, down.nseg = 1, down.seg[0] = pg_seg(c, l, 6, L.w_down, w.x);
+  pf_parts(c, qkv), pf_parts(c, o), pf_parts(c, down);
   /* the q/k/v launch leaves its K parts' sum to the RoPE + append kernel,
    * o and down theirs to the next RMSNorm (the last layer's down sums its
    * own: the LM head reads x) */
-  int kq = 1, ko = 1, kd = 1;
+  int kq = 0, ko = 0, kd = 0;
   qkv.kparts_out = &kq;
   o.kparts_out = &ko;
-  if (l + 1 < m.n_layers) dn.kparts_out = &kd;
+  if (l + 1 < m.n_layers) down.kparts_out = &kd;
+  const uint8_t *dn = T >= kDenseTokens && (size_t)l < c->mm.size() && !gq_matvec_q6k_ref() ? c->mm[l].dn : nullptr;
+  auto gemm = [&](int mode, const PgArgs &p, int i) {
+    if (!dn) return gq_launch_pgemm(mode, p, c->stream);
+    DnArgs d{};
+    d.x = p.x, d.w = dn + c->mm[l].dn_at[i], d.act = p.act, d.T = p.T, d.K = p.K;
+    d.nseg = mode == MV_SWIGLU ? 1 : p.nseg;
+    for (int q = 0; q < d.nseg; q++) d.y[q] = p.seg[q].y, d.rows[q] = p.seg[q].rows;
+    d.part = p.part, d.part_cap = p.part_cap, d.kparts_out = p.kparts_out;
+    return gq_launch_dense(mode, d, c->n_cu, c->stream);
+  };
   auto norm = [&](const float *nw, int k) {
     return gq_launch_rmsnorm_rows(w.x, nw, nullptr, m.hidden, T, m.rms_eps, c->stream, w.xn,
-                                  k > 1 ? w.part : nullptr, k, w.x);
+                                  k > 0 ? w.part : nullptr, k, w.x);
   };
-  if ((rc = norm(L.rms_att, pending)) || (rc = gq_launch_pgemm(MV_STORE, qkv, c->stream)) ||
+  if ((rc = norm(L.rms_att, pending)) || (rc = gemm(MV_STORE, qkv, 0)) ||
       (rc = pf_attention(c, l, pos, T, m.n_heads, w.q, w.k, w.v, nullptr, w.att, kq)) ||
-      (rc = gq_launch_pgemm(MV_RESID, o, c->stream)) || (rc = norm(L.rms_ffn, ko)) ||
-      (rc = gq_launch_pgemm(MV_SWIGLU, gu, c->stream)) || (rc = gq_launch_pgemm(MV_RESID, dn, c->stream)))
+      (rc = gemm(MV_RESID, o, 1)) || (rc = norm(L.rms_ffn, ko)) || (rc = gemm(MV_SWIGLU, gu, 2)) ||
+      (rc = gemm(MV_RESID, down, 3)))
     return rc;
   pending = kd;
   return 0;
@@ -1484,7 +1546,9 @@ extern "C" int gq_hip_prefill(gq_ctx *c, const int32_t *tokens, int n_tokens, in
   for (int i = 0; i < n_tokens; i++)
     if (tokens[i] < 0 || tokens[i] >= m.vocab) return fail(c, -1, "prefill: token %d out of range", tokens[i]);
   const bool gemm = pf_model_ok(c);
-  if (gemm && (rc = pf_alloc(c))) return rc;
+  /* equal chunks */
+  const int nchunk = (n_tokens + kPrefillChunk - 1) / kPrefillChunk, chunk = (n_tokens + nchunk - 1) / nchunk;
+  if (gemm && (rc = pf_alloc(c, chunk))) return rc;
   c->g_valid = false;
   PrefillWs &w = c->pf;
   Workspace &ws = c->ws;
@@ -1493,21 +1557,23 @@ extern "C" int gq_hip_prefill(gq_ctx *c, const int32_t *tokens, int n_tokens, in
     HIPCHK(c, ev.create());
     HIPCHK(c, hipEventRecord(ev.e0, c->stream));
   }
-  int T = 0;
+  int T = 0, in = 0;
   if (!gemm) { /* token by token through the decode step */
     for (int t = 0; t < n_tokens; t++)
       if ((rc = run_step(c, tokens[t], pos + t, false, nullptr))) return fail(c, rc, "prefill: step launch failed");
   } else {
     for (int t0 = 0; t0 < n_tokens; t0 += T) {
-      T = std::min(kPrefillChunk, n_tokens - t0);
-      const int in = t0 % kPinnedTokens; /* the embedding kernel reads the tokens there */
-      if (in == 0) {
-        if (t0) HIPCHK(c, hipStreamSynchronize(c->stream)); /* the last piece has been read */
-        memcpy(c->h_in, tokens + t0, sizeof(int) * (size_t)std::min(kPinnedTokens, n_tokens - t0));
+      T = std::min(chunk, n_tokens - t0);
+      /* the embedding kernel reads the tokens there */
+      if (in + T > kPinnedTokens) {
+        HIPCHK(c, hipStreamSynchronize(c->stream)); /* what is there has been read */
+        in = 0;
       }
+      memcpy(c->h_in + in, tokens + t0, sizeof(int) * (size_t)T);
       if ((rc = gq_launch_embed_rows(m.embed.dtype, m.embed.data, m.hidden, c->h_in + in, T, w.x, c->stream)))
         return fail(c, rc, "prefill: embed");
-      int pending = 1;
+      in += T;
+      int pending = 0;
       for (int l = 0; l < m.n_layers; l++)
         if ((rc = pf_layer(c, l, pos + t0, T, pending))) return fail(c, rc, "prefill: layer %d launch failed", l);
     }

@@ -543,3 +543,35 @@ def test_prefill_model_rejects_bad_input(ctx):
         dm.prefill(np.arange(10, dtype=np.int32), 60)      # past the cache
     with pytest.raises(H.HipError):
         dm.prefill(np.array([1, 2, 5000], np.int32), 0)    # token out of range
+
+
+@pytest.mark.parametrize("T", [256, 257, 511, 700])
+@pytest.mark.parametrize("mix", ["q4_k_m", "q8_0"])
+def test_prefill_dense_copy_vs_quantized(orc, T, mix):
+    """Chunks of 256 tokens and more multiply by the bf16 copies of the
+    weights that model bind makes; matvec path 3 dequantizes the same weights
+    as it multiplies.  Layer 0's V rows are that GEMM's own output: the same
+    products in another order (1e-5).  After it the bf16 activations may round
+    apart: 2e-3, as between the layouts above.  128-row K and V segments (half
+    a tile), a gate/up of 10 tiles, ragged token tiles."""
+    import guanaco_amd.hip as H
+    dts = {k: S.Q8_0 for k in S.LAYER_WEIGHTS} if mix == "q8_0" else dict(wv=S.Q6_K, wd=S.Q6_K)
+    spec = S.ModelSpec("dense-test", n_layers=2, hidden=512, ff=1280 if mix == "q8_0" else 1536, n_heads=8, n_kv_heads=2,
+                       vocab=1000, layer_dtypes=dts, q4k_zero_mean=True, norm_shift=4)
+    c = H.Context(0)
+    try:
+        dm = H.DeviceModel(c, spec, 768)
+        toks = np.random.default_rng(T).integers(0, spec.vocab, T).astype(np.int32)
+        res = {}
+        for path in ("auto", "auto_q6k_ref"):
+            with H.matvec_path(path):
+                _, lg, hid, _ = dm.prefill(toks, 0, want_hidden=True)
+            k0, v0 = c.kv_read_layer(0)
+            res[path] = lg, hid, v0
+        a, b = res["auto"], res["auto_q6k_ref"]
+        v = [r[2].reshape(2, 768, 64)[:, :T] for r in (a, b)]
+        assert rel_l2(v[0], v[1]) < 1e-5  # the same bits where both take as many K parts
+        assert rel_l2(a[0], b[0]) < 2e-3 and rel_l2(a[1], b[1]) < 2e-3
+        print(f"dense copy vs quantized, T={T}: V rows {rel_l2(v[0], v[1]):.2e}, logits {rel_l2(a[0], b[0]):.2e}")
+    finally:
+        c.close()
