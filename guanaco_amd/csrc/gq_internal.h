@@ -304,9 +304,10 @@ struct PgArgs {
   int *kparts_out;
 };
 int gq_launch_pgemm(int mode, const PgArgs &a, hipStream_t s);
-/* at most this many K parts in a split launch: PgArgs.part needs
- * kPgKParts * T * (all segments' rows) floats */
-constexpr int kPgKParts = 4;
+/* at most this many K parts in a split launch (kPgFlatParts up to 64 tokens):
+ * PgArgs.part needs gq_parts_tokens(T) * (all segments' rows) floats */
+constexpr int kPgKParts = 4, kPgFlatParts = 8;
+constexpr size_t gq_parts_tokens(int T) { return T <= 64 ? (size_t)kPgFlatParts * T : (size_t)kPgKParts * T; }
 /* y = (y +) the sum of a split launch's parts, scattered to its segments
  * (seg[].y / rows, nseg, T, part, kparts, rows_total) */
 int gq_launch_parts(const PgArgs &a, bool resid, hipStream_t s);

@@ -392,14 +392,15 @@ struct PW<GQ_Q8_0> {
   }
 };
 
-/* KS = 1 or 2 K-splits per workgroup: with KS = 2, eight waves, the second
- * four running the upper half of K for the same tile; their sums are added
- * through LDS at the end.  Two waves per SIMD hide each other's LDS, DMA and
+/* KS = 1, 2 or 4 K-splits per workgroup, RW = 4 or 2 waves of 32 rows each
+ * in one: with KS = 2 and RW = 4, eight waves, the second four running the
+ * upper half of K for the same tile; the splits' sums are added through LDS
+ * at the end.  Two waves per SIMD hide each other's LDS, DMA and
  * MFMA latencies.  TT = 2 or 4 token tiles per wave: each dequantized B
  * operand feeds TT MFMAs. */
-template <int DT, int KS, int TT>
+template <int DT, int KS, int TT, int RW = 4>
 constexpr int stage_bytes() {
-  return KS * x_bytes<TT>() + 4 * KS * PW<DT>::kWaveLds;
+  return KS * x_bytes<TT>() + RW * KS * PW<DT>::kWaveLds;
 }
 
 /* Steps in the LDS ring: as deep as LDS (160 KB) and the 6-bit vmcnt allow
@@ -408,36 +409,42 @@ constexpr int stage_bytes() {
  * with 128-token tiles (KS 1, TT 4: 24 KB stages) takes 3 slots, 72 KB, so
  * two workgroups share a CU (two waves per SIMD): gate/up at 512 tokens ran
  * 265 -> 200 us against 4 slots and one workgroup per CU. */
-template <int DT, int KS, int TT>
+template <int DT, int KS, int TT, int RW = 4>
 constexpr int ring() {
-  return std::min(KS == 1 && TT == 4 ? 3 : 4, (160 * 1024) / stage_bytes<DT, KS, TT>());
+  return std::min(KS == 1 && TT == 4 ? 3 : 4, (160 * 1024) / stage_bytes<DT, KS, TT, RW>());
 }
-template <int DT, int KS, int TT>
+template <int DT, int KS, int TT, int RW = 4>
 constexpr int ring_bytes() {
-  return ring<DT, KS, TT>() * stage_bytes<DT, KS, TT>();
+  return ring<DT, KS, TT, RW>() * stage_bytes<DT, KS, TT, RW>();
 }
-template <int DT, int KS, int TT>
+template <int DT, int KS, int TT, int RW = 4>
 constexpr bool fits() {
-  return ring<DT, KS, TT>() >= 3 && (ring<DT, KS, TT>() - 2) * (TT + PW<DT>::kDma) < 64;
+  return ring<DT, KS, TT, RW>() >= 3 && (ring<DT, KS, TT, RW>() - 2) * (4 * TT / RW + PW<DT>::kDma) < 64;
 }
 static_assert(fits<GQ_Q4_K, 1, 2>() && fits<GQ_Q4_K, 2, 2>() && fits<GQ_Q6_K, 1, 2>() && fits<GQ_Q6_K, 2, 2>() &&
                   fits<GQ_Q6_KX, 1, 2>() && fits<GQ_Q6_KX, 2, 2>() &&
                   fits<GQ_Q4_K, 1, 4>() && fits<GQ_Q4_K, 2, 4>() && fits<GQ_Q8_0, 1, 2>() && fits<GQ_Q8_0, 2, 2>() &&
                   fits<GQ_Q8_0, 1, 4>() && fits<GQ_Q8_0, 2, 4>(),
               "ring shapes");
+static_assert(fits<GQ_Q4_K, 4, 1, 2>() && fits<GQ_Q4_K, 4, 2, 2>() && fits<GQ_Q6_KX, 4, 1, 2>() && fits<GQ_Q6_KX, 4, 2, 2>() &&
+                  fits<GQ_Q8_0, 4, 1, 2>() && fits<GQ_Q8_0, 4, 2, 2>() && fits<GQ_Q6_K, 4, 1, 2>(),
+              "flat ring shapes");
+static_assert(fits<GQ_Q4_K, 4, 1, 4>() && fits<GQ_Q6_KX, 4, 1, 4>() && fits<GQ_Q8_0, 4, 1, 4>() && !fits<GQ_Q6_K, 4, 1, 4>(),
+              "16-wave ring shapes (Q6_K in the reference layout takes two row waves)");
 
 /* One tile: tokens t0 .. t0 + 32 TT - 1 against this wave's 32 rows starting
  * at w, K-split kh of KS.  acc[i] holds tokens t0 + 32 i + (D layout rows)
  * for row (lane & 31). */
-template <int DT, int KS, int TT>
+template <int DT, int KS, int TT, int RW>
 __device__ __forceinline__ void tile_loop(const PgArgs &a, const uint8_t *w, uint32_t rowbytes, int t0,
                                           GQ_LDS uint8_t *smem, gq_f32x16 (&acc)[TT]) {
-  constexpr int SB = stage_bytes<DT, KS, TT>();
+  constexpr int SB = stage_bytes<DT, KS, TT, RW>();
   constexpr int XB = x_bytes<TT>();
-  constexpr int NPS = TT + PW<DT>::kDma; /* DMA instructions per wave and step */
-  constexpr int kRing = ring<DT, KS, TT>();
+  constexpr int NX = 4 * TT / RW;        /* a wave's share of its split's X instructions */
+  constexpr int NPS = NX + PW<DT>::kDma; /* DMA instructions per wave and step */
+  constexpr int kRing = ring<DT, KS, TT, RW>();
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kh = wave >> 2, rw = wave & 3;
+  const int kh = wave / RW, rw = wave % RW;
   /* this wave's steps s0 .. s0 + ns - 1: K part blockIdx.z of a.kparts,
    * then split kh of KS within the workgroup */
   const int nsp = a.K / kBK / a.kparts, ns = nsp / KS, s0 = (int)blockIdx.z * nsp + kh * ns;
@@ -445,13 +452,13 @@ __device__ __forceinline__ void tile_loop(const PgArgs &a, const uint8_t *w, uin
   PW<DT>::plan(pl, lane, rowbytes);
   const uint32_t sbase = (uint32_t)(uintptr_t)smem;
   const uint32_t xreg = (uint32_t)(kh * XB), wreg = (uint32_t)(KS * XB + wave * PW<DT>::kWaveLds);
-  /* X DMA: instruction j of wave rw covers tokens 8 (TT rw + j) + lane / 8;
+  /* X DMA: instruction j of wave rw covers tokens 8 (NX rw + j) + lane / 8;
    * lane position q = lane % 8 of the token's LDS row fetches octet
    * q ^ ((token / 2) % 8) */
-  const __bf16 *xsrc[TT];
+  const __bf16 *xsrc[NX];
 #pragma unroll
-  for (int j = 0; j < TT; j++) {
-    const int tl = 8 * (TT * rw + j) + (lane >> 3), q = lane & 7;
+  for (int j = 0; j < NX; j++) {
+    const int tl = 8 * (NX * rw + j) + (lane >> 3), q = lane & 7;
     const int oct = q ^ ((tl >> 1) & 7);
     /* the unit layout's steps take columns 64 s - 32 (s & 1) + 8 o (+32 for
      * o >= 4): PW<GQ_Q6_KX> */
@@ -461,8 +468,8 @@ __device__ __forceinline__ void tile_loop(const PgArgs &a, const uint8_t *w, uin
     const uint32_t slot = sbase + (uint32_t)((st % kRing) * SB);
     const int s = s0 + st, xs = DT == GQ_Q6_KX ? s * kBK - 32 * (s & 1) : s * kBK;
 #pragma unroll
-    for (int j = 0; j < TT; j++)
-      dma16(xsrc[j] + xs, __builtin_amdgcn_readfirstlane(slot + xreg + 1024u * (uint32_t)(TT * rw + j)));
+    for (int j = 0; j < NX; j++)
+      dma16(xsrc[j] + xs, __builtin_amdgcn_readfirstlane(slot + xreg + 1024u * (uint32_t)(NX * rw + j)));
     PW<DT>::issue(pl, w, s0 + st, slot + wreg);
   };
   for (int st = 0; st < kRing - 1 && st < ns; st++) issue(st);
@@ -474,7 +481,7 @@ __device__ __forceinline__ void tile_loop(const PgArgs &a, const uint8_t *w, uin
    * VALU work overlaps the matrix core.  A wave's copies of a step have
    * landed once only the copies of later steps remain in flight; the
    * barrier extends that to every wave's copies and frees the slot read in
-   * iteration s - 1 for step s + kRing - 1.  With TT = 2 the A operands of
+   * iteration s - 1 for step s + kRing - 1.  With TT <= 2 the A operands of
    * step s + 1 are read during step s too; with TT = 4 (twice the A
    * registers) they are read at the top of their own step. */
   /* A operand addresses within a slot: token tl = 32 i + lane % 32, octet
@@ -493,7 +500,7 @@ __device__ __forceinline__ void tile_loop(const PgArgs &a, const uint8_t *w, uin
   wait_groups<NPS, kRing - 2>(ns - 1);
   __syncthreads();
   PW<DT>::read(raw, wslot(0), lane, s0);
-  if (TT == 2) {
+  if (TT <= 2) {
 #pragma unroll
     for (int kk = 0; kk < 4; kk++)
 #pragma unroll
@@ -513,16 +520,16 @@ __device__ __forceinline__ void tile_loop(const PgArgs &a, const uint8_t *w, uin
     }
     /* LDS reads for step s + 1 first, so their latency hides behind the
      * MFMAs of step s */
-    gq_bf16x8 an[4][TT == 2 ? 2 : 1];
+    gq_bf16x8 an[4][TT];
     const bool more = s + 1 < ns;
     if (more) {
       PW<DT>::read(raw, wslot(s + 1), lane, s0 + s + 1);
-      if (TT == 2) {
+      if (TT <= 2) {
         const GQ_LDS uint8_t *xn = smem + ((s + 1) % kRing) * SB;
 #pragma unroll
         for (int kk = 0; kk < 4; kk++)
 #pragma unroll
-          for (int i = 0; i < 2; i++) an[kk][i] = lld<gq_bf16x8>(xn, aoff[kk][i]);
+          for (int i = 0; i < TT; i++) an[kk][i] = lld<gq_bf16x8>(xn, aoff[kk][i]);
       }
     }
 #pragma unroll
@@ -531,11 +538,11 @@ __device__ __forceinline__ void tile_loop(const PgArgs &a, const uint8_t *w, uin
       for (int i = 0; i < TT; i++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[kk][i], b[kk], acc[i], 0, 0, 0);
     if (more) {
       PW<DT>::dequant(raw, s0 + s + 1, b);
-      if (TT == 2) {
+      if (TT <= 2) {
 #pragma unroll
         for (int kk = 0; kk < 4; kk++)
 #pragma unroll
-          for (int i = 0; i < 2; i++) av[kk][i] = an[kk][i];
+          for (int i = 0; i < TT; i++) av[kk][i] = an[kk][i];
       }
     }
   }
@@ -545,64 +552,68 @@ __device__ __forceinline__ int tile_token(int i, int e, int lane) {
   return 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
 }
 
-/* Grid: x = row tiles over the segments (kBN rows each; MV_SWIGLU: 64 gate
- * rows with the same 64 up rows), y = token tiles of 32 TT; 256 KS threads. */
-template <int MODE, int KS, int TT>
-__global__ __launch_bounds__(kPThreads * KS) void pgemm_kernel(PgArgs a) {
+/* Grid: x = row tiles over the segments (32 RW rows each; MV_SWIGLU: 16 RW
+ * gate rows with the same up rows), y = token tiles of 32 TT; 64 RW KS
+ * threads. */
+template <int MODE, int KS, int TT, int RW>
+__global__ __launch_bounds__(64 * RW * KS) void pgemm_kernel(PgArgs a) {
+  constexpr int kBN = 32 * RW;
   extern __shared__ __attribute__((aligned(16))) uint8_t pg_smem[];
   GQ_LDS uint8_t *smem = (GQ_LDS uint8_t *)pg_smem;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kh = wave >> 2, rw = wave & 3;
+  const int kh = wave / RW, rw = wave % RW;
   const int t0 = blockIdx.y * 32 * TT;
   int sg = 0, tb = blockIdx.x, roff = 0; /* roff: the segment's first row among all segments' */
   if (MODE != MV_SWIGLU)
     while (sg + 1 < a.nseg && tb >= a.seg[sg].rows / kBN) tb -= a.seg[sg].rows / kBN, roff += a.seg[sg].rows, sg++;
   /* this wave's weights: rows r0 .. r0 + 31 of segment ws */
   int ws = sg, r0 = tb * kBN + 32 * rw;
-  if (MODE == MV_SWIGLU) ws = rw >> 1, r0 = tb * (kBN / 2) + 32 * (rw & 1);
+  if (MODE == MV_SWIGLU) ws = rw / (RW / 2), r0 = tb * (kBN / 2) + 32 * (rw % (RW / 2));
   const PgSeg &S = a.seg[ws];
   const int dt = a.seg[sg].dtype;
   const uint32_t rowbytes = dt == GQ_Q8_0 ? (uint32_t)(a.K / 32) * 34u : (uint32_t)(a.K / 256) * (dt == GQ_Q4_K ? 144u : 210u);
   const uint8_t *w = S.w + (size_t)r0 * rowbytes;
   gq_f32x16 acc[TT];
-  if constexpr (fits<GQ_Q6_K, KS, TT>() && fits<GQ_Q6_KX, KS, TT>()) {
+  if constexpr (fits<GQ_Q6_K, KS, TT, RW>() && fits<GQ_Q6_KX, KS, TT, RW>()) {
     if (dt == GQ_Q4_K)
-      tile_loop<GQ_Q4_K, KS, TT>(a, w, rowbytes, t0, smem, acc);
+      tile_loop<GQ_Q4_K, KS, TT, RW>(a, w, rowbytes, t0, smem, acc);
     else if (dt == GQ_Q6_KX)
-      tile_loop<GQ_Q6_KX, KS, TT>(a, w, rowbytes, t0, smem, acc);
+      tile_loop<GQ_Q6_KX, KS, TT, RW>(a, w, rowbytes, t0, smem, acc);
     else if (dt == GQ_Q8_0)
-      tile_loop<GQ_Q8_0, KS, TT>(a, w, rowbytes, t0, smem, acc);
+      tile_loop<GQ_Q8_0, KS, TT, RW>(a, w, rowbytes, t0, smem, acc);
     else
-      tile_loop<GQ_Q6_K, KS, TT>(a, w, rowbytes, t0, smem, acc);
-  } else if constexpr (fits<GQ_Q6_KX, KS, TT>()) { /* the launcher sends Q6_K to shapes that fit */
+      tile_loop<GQ_Q6_K, KS, TT, RW>(a, w, rowbytes, t0, smem, acc);
+  } else if constexpr (fits<GQ_Q6_KX, KS, TT, RW>()) { /* the launcher sends Q6_K to shapes that fit */
     if (dt == GQ_Q6_KX)
-      tile_loop<GQ_Q6_KX, KS, TT>(a, w, rowbytes, t0, smem, acc);
+      tile_loop<GQ_Q6_KX, KS, TT, RW>(a, w, rowbytes, t0, smem, acc);
     else if (dt == GQ_Q8_0)
-      tile_loop<GQ_Q8_0, KS, TT>(a, w, rowbytes, t0, smem, acc);
+      tile_loop<GQ_Q8_0, KS, TT, RW>(a, w, rowbytes, t0, smem, acc);
     else
-      tile_loop<GQ_Q4_K, KS, TT>(a, w, rowbytes, t0, smem, acc);
+      tile_loop<GQ_Q4_K, KS, TT, RW>(a, w, rowbytes, t0, smem, acc);
   } else {
     if (dt == GQ_Q8_0)
-      tile_loop<GQ_Q8_0, KS, TT>(a, w, rowbytes, t0, smem, acc);
+      tile_loop<GQ_Q8_0, KS, TT, RW>(a, w, rowbytes, t0, smem, acc);
     else
-      tile_loop<GQ_Q4_K, KS, TT>(a, w, rowbytes, t0, smem, acc);
+      tile_loop<GQ_Q4_K, KS, TT, RW>(a, w, rowbytes, t0, smem, acc);
   }
-  constexpr int XS = 4 * TT * 16 * 64 * 4; /* bytes of one K-half's tiles */
+  constexpr int XS = RW * TT * 16 * 64 * 4; /* bytes of one K-split's tiles */
   GQ_LDS float *xk = (GQ_LDS float *)smem;
-  if (KS == 2) { /* add the upper K half (waves 4..7) into waves 0..3, in a fixed order */
+  if (KS > 1) { /* add the other K splits into the first's waves, in order */
     __syncthreads(); /* every wave is done reading the ring */
-    if (kh == 1) {
+    if (kh > 0) {
 #pragma unroll
       for (int i = 0; i < TT; i++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) xk[((rw * TT + i) * 16 + e) * 64 + lane] = acc[i][e];
+        for (int e = 0; e < 16; e++) xk[(kh - 1) * (XS / 4) + ((rw * TT + i) * 16 + e) * 64 + lane] = acc[i][e];
     }
     __syncthreads();
     if (kh == 0) {
 #pragma unroll
-      for (int i = 0; i < TT; i++)
+      for (int k = 0; k < KS - 1; k++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) acc[i][e] += xk[((rw * TT + i) * 16 + e) * 64 + lane];
+        for (int i = 0; i < TT; i++)
+#pragma unroll
+          for (int e = 0; e < 16; e++) acc[i][e] += xk[k * (XS / 4) + ((rw * TT + i) * 16 + e) * 64 + lane];
     }
   }
   const int n = r0 + (lane & 31);
@@ -627,19 +638,19 @@ __global__ __launch_bounds__(kPThreads * KS) void pgemm_kernel(PgArgs a) {
     }
     return;
   }
-  /* SwiGLU: the up waves (rw 2, 3) hand their tiles to the gate waves (rw 0,
-   * 1) through LDS; act = (g * sigmoid(g)) * u as silu_inplace then
+  /* SwiGLU: the up waves (the upper half) hand their tiles to the gate waves
+   * through LDS; act = (g * sigmoid(g)) * u as silu_inplace then
    * elemwise_mul (kernels_cpu.c:312-389), rounded to bf16 */
-  __syncthreads(); /* the ring (and the K-half exchange) are free */
-  GQ_LDS float *xch = (GQ_LDS float *)(smem + (KS == 2 ? XS : 0));
-  if (kh == 0 && rw >= 2) {
+  __syncthreads(); /* the ring (and the K-split exchange) are free */
+  GQ_LDS float *xch = (GQ_LDS float *)(smem + (KS - 1) * XS);
+  if (kh == 0 && rw >= RW / 2) {
 #pragma unroll
     for (int i = 0; i < TT; i++)
 #pragma unroll
-      for (int e = 0; e < 16; e++) xch[(((rw - 2) * TT + i) * 16 + e) * 64 + lane] = acc[i][e];
+      for (int e = 0; e < 16; e++) xch[(((rw - RW / 2) * TT + i) * 16 + e) * 64 + lane] = acc[i][e];
   }
   __syncthreads();
-  if (kh == 0 && rw < 2) {
+  if (kh == 0 && rw < RW / 2) {
 #pragma unroll
     for (int i = 0; i < TT; i++)
 #pragma unroll
@@ -891,17 +902,42 @@ int n_cus() {
   return cus;
 }
 
-template <int MODE, int KS, int TT>
+template <int MODE, int KS, int TT, int RW = 4>
 int launch_shape(const PgArgs &a, int row_tiles, size_t lds, hipStream_t s) {
   static bool attr_done = false;
   if (!attr_done) {
-    (void)hipFuncSetAttribute((const void *)pgemm_kernel<MODE, KS, TT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    (void)hipFuncSetAttribute((const void *)pgemm_kernel<MODE, KS, TT, RW>, hipFuncAttributeMaxDynamicSharedMemorySize,
                               160 * 1024);
     attr_done = true;
   }
-  hipLaunchKernelGGL((pgemm_kernel<MODE, KS, TT>), dim3(row_tiles, (a.T + 32 * TT - 1) / (32 * TT), a.kparts),
-                     dim3(kPThreads * KS), lds, s, a);
+  hipLaunchKernelGGL((pgemm_kernel<MODE, KS, TT, RW>), dim3(row_tiles, (a.T + 32 * TT - 1) / (32 * TT), a.kparts),
+                     dim3(64 * RW * KS), lds, s, a);
   return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+/* Up to 64 tokens the weights are read and dequantized once however the
+ * launch is shaped, and what counts is how many steps run in a row: four K
+ * splits a workgroup, of two or four row waves, and as many K parts over the
+ * grid as fill the CUs.  Against 128-token tiles and four parts, us per
+ * launch at 37 tokens: 8B shape q/k/v 22 -> 20, o 21 -> 12, down 58 -> 32
+ * (Q4_K), gate/up at 8 tokens 39 -> 35; 1.1B Q8_0 15 -> 9, 15 -> 9, 27 -> 19,
+ * gate/up 26 -> 19.  A step of eight waves takes 1.25 us with 32-token tiles
+ * and 1.8 with 64, of sixteen waves 1.8: bound by the weights' DMA requests,
+ * 16 bytes each from rows kilobytes apart. */
+template <int MODE, int TT, int RW>
+int launch_flat(const PgArgs &a0, int rows, bool q4, bool q6, bool q6x, bool q8, int kp, hipStream_t s) {
+  PgArgs a = a0;
+  a.kparts = kp;
+  const size_t lds = std::max({q4 ? ring_bytes<GQ_Q4_K, 4, TT, RW>() : 0, q6x ? ring_bytes<GQ_Q6_KX, 4, TT, RW>() : 0,
+                               q8 ? ring_bytes<GQ_Q8_0, 4, TT, RW>() : 0,
+                               q6 && fits<GQ_Q6_K, 4, TT, RW>() ? ring_bytes<GQ_Q6_K, 4, TT, RW>() : 0});
+  int rc = launch_shape<MODE, 4, TT, RW>(a, rows / (MODE == MV_SWIGLU ? 16 * RW : 32 * RW), lds, s);
+  if (rc || kp == 1) return rc;
+  if (a.kparts_out) { /* the caller sums the parts */
+    *a.kparts_out = kp;
+    return 0;
+  }
+  return gq_launch_parts(a, MODE == MV_RESID, s);
 }
 
 template <int MODE>
@@ -930,6 +966,26 @@ int launch_mode(const PgArgs &a0, int row_tiles, hipStream_t s) {
   const int tiles4 = row_tiles * ((a.T + 127) / 128);
   a.rows_total = 0;
   for (int i = 0; i < a.nseg; i++) a.rows_total += a.seg[i].rows;
+  if (a.T <= 64 && (a.K / kBK) % 4 == 0 && (!q6 || a.T <= 32)) {
+    /* rounds of workgroups at a step's measured time and a round's start and
+     * end, and what the parts cost their reader; a gate/up launch may be
+     * better off as below (one part, two splits) */
+    const int rows = MODE == MV_SWIGLU ? a.seg[0].rows : a.rows_total, per = MODE == MV_SWIGLU ? 16 : 32;
+    const int steps = a.K / kBK / 4;
+    int kp = 0, rw = 2;
+    double best = MODE == MV_SWIGLU ? (rows / 64 + n_cus() - 1) / n_cus() * (2 * steps * 1.25 + 3.0) : 1e30;
+    for (int w = 2; w <= (a.T <= 32 && !q6 ? 4 : 2); w += 2)
+      for (int k = 1; k <= kPgFlatParts; k++) {
+        if (steps % k || (k > 1 && (MODE == MV_SWIGLU || !a.part || (size_t)k * a.T * a.rows_total > a.part_cap))) continue;
+        const double step = a.T > 32 || w == 4 ? 1.8 : 1.25;
+        const double us = (rows / (per * w) * k + n_cus() - 1) / n_cus() * (steps / k * step + 5.0) + (k > 1 ? 0.6 * k : 0.0);
+        if (us < best) best = us, kp = k, rw = w;
+      }
+    if (kp)
+      return a.T > 32   ? launch_flat<MODE, 2, 2>(a, rows, q4, q6, q6x, q8, kp, s)
+             : rw == 2 ? launch_flat<MODE, 1, 2>(a, rows, q4, q6, q6x, q8, kp, s)
+                       : launch_flat<MODE, 1, 4>(a, rows, q4, q6, q6x, q8, kp, s);
+  }
   /* as few parts as give 1.5 workgroups per CU: 2 for the fused q/k/v
    * launch at 512 tokens (forward 13.83 -> 13.62 ms against 4 parts'
    * 13.95), 4 for o, down and k/v alone */
@@ -1007,6 +1063,10 @@ int gq_launch_pgemm(int mode, const PgArgs &a, hipStream_t s) {
   static_assert(ring_bytes<GQ_Q4_K, 2, 2>() >= 6 * 2 * 16 * 64 * 4 && ring_bytes<GQ_Q6_K, 2, 2>() >= 6 * 2 * 16 * 64 * 4 &&
                     ring_bytes<GQ_Q4_K, 2, 4>() >= 6 * 4 * 16 * 64 * 4 && ring_bytes<GQ_Q8_0, 2, 2>() >= 6 * 2 * 16 * 64 * 4,
                 "exchanges fit the ring");
+  static_assert(ring_bytes<GQ_Q4_K, 4, 1, 2>() >= 7 * 16 * 64 * 4 && ring_bytes<GQ_Q4_K, 4, 2, 2>() >= 14 * 16 * 64 * 4 &&
+                    ring_bytes<GQ_Q6_K, 4, 1, 2>() >= 7 * 16 * 64 * 4,
+                "exchanges fit the flat rings (three splits' tiles, then the up tiles)");
+  static_assert(ring_bytes<GQ_Q4_K, 4, 1, 4>() >= 14 * 16 * 64 * 4, "and the 16-wave ring");
   if (mode == MV_SWIGLU) {
     if (a.nseg != 2 || !a.act) return -1;
     return launch_mode<MV_SWIGLU>(a, a.seg[0].rows / (kBN / 2), s);

@@ -1484,7 +1484,7 @@ static void pf_parts(gq_ctx *c, PgArgs &a) {
   PrefillWs &w = c->pf;
   size_t rows = 0;
   for (int i = 0; i < a.nseg; i++) rows += a.seg[i].rows;
-  const size_t n = (size_t)kPgKParts * a.T * rows;
+  const size_t n = gq_parts_tokens(a.T) * rows;
   if (pf_ensure(c, w.part, w.part_cap, n) == 0) a.part = w.part, a.part_cap = w.part_cap;
 }
 

@@ -208,6 +208,43 @@ def test_prefill_gate_up_swiglu(ctx, orc, dtype, T, N, K):
     H.lib.gq_hip_free(ctx.h, gd), H.lib.gq_hip_free(ctx.h, ud)
 
 
+@pytest.mark.parametrize("T", [1, 32, 33, 64])
+@pytest.mark.parametrize("dtype,N,K", [
+    (S.Q4_K, 128, 256),     # one step a split, one part
+    (S.Q4_K, 6144, 4096),   # the 8B q/k/v rows: 16 waves up to 32 tokens
+    (S.Q4_K, 384, 14336),   # 56 steps a split over 8 or 7 parts
+    (S.Q6_K, 256, 2048),    # unit layout
+    (S.Q6_K, 128, 1536),    # reference layout: past 32 tokens the 64-token tiles of longer chunks
+    (S.Q8_0, 640, 5632),    # 22 steps a split
+])
+def test_prefill_gemm_few_tokens(ctx, orc, dtype, N, K, T):
+    """The shapes of up to 64 tokens (four K splits a workgroup, parts over
+    the grid), stored and added to a residual, on up to 256 sampled rows
+    against the exact-input fp64 product (1e-5)."""
+    import guanaco_amd.hip as H
+    seed = (T << 20) ^ (N << 4) ^ K ^ (dtype << 28)
+    w = orc.synth_quant(dtype, seed, N, K)
+    x = orc.synth_normal(seed + 1, T * K).reshape(T, K)
+    r = orc.synth_normal(seed + 2, T * N).reshape(T, N)
+    idx = np.unique(np.concatenate([[0, N - 1], np.random.default_rng(seed).choice(N, min(N, 254), replace=False)]))
+    ws = np.ascontiguousarray(w.reshape(N, -1)[idx]).reshape(-1)
+    want = bf16_round(x).astype(np.float64) @ bf16_round(_kernel_weights(dtype, ws, idx.size, K)).astype(np.float64).T
+    wd, xd, yd = ctx.upload_weight(w), ctx.upload(x), ctx.upload(r)
+    assert H.lib.gq_hip_prefill_gemm_dev(ctx.h, dtype, 1, wd, N, K, xd.ptr, T, yd.ptr, yd.ptr) == 0
+    assert rel_l2(yd.download(count=T * N).reshape(T, N)[:, idx] - r[:, idx].astype(np.float64), want) < 1e-5
+    assert H.lib.gq_hip_prefill_gemm_dev(ctx.h, dtype, 0, wd, N, K, xd.ptr, T, yd.ptr, None) == 0
+    assert rel_l2(yd.download(count=T * N).reshape(T, N)[:, idx], want) < 1e-5
+    xd.free(), yd.free()
+    H.lib.gq_hip_free(ctx.h, wd)
+
+
+@pytest.mark.parametrize("dtype,T,N,K", [(S.Q4_K, 1, 64, 256), (S.Q4_K, 32, 10240, 2048), (S.Q4_K, 64, 192, 1024),
+                                         (S.Q8_0, 33, 320, 2048), (S.Q6_K, 32, 64, 512), (S.Q6_K, 64, 128, 2048)])
+def test_prefill_gate_up_few_tokens(ctx, orc, dtype, T, N, K):
+    """Gate/up + SwiGLU in those shapes (10240 rows: sixteen waves)."""
+    test_prefill_gate_up_swiglu(ctx, orc, dtype, T, N, K)
+
+
 @pytest.mark.parametrize("T,N,K", [(512, 14336, 4096), (300, 11008, 2048), (257, 11008, 1024)])
 def test_prefill_gate_up_wide_tile(ctx, orc, T, N, K):
     """The fused Q4_K gate/up launch on the wide tile (64 rows per wave),
