@@ -28,6 +28,7 @@
  * the fp32 matrix cores; see the kernel.
  */
 #include <algorithm>
+#include <cmath>
 
 #include "gq_device.h"
 #include "gq_internal.h"
@@ -376,14 +377,13 @@ struct FlashLds { /* the waves' (max, sum, O) on their way to wave 0 */
 };
 
 template <int HD, int G>
-__device__ __forceinline__ void flash_tile(const AttnArgs &a, int g, int t0, FlashLds<HD> &lds) {
+__device__ __forceinline__ void flash_tile(const AttnArgs &a, int g, int t0, int wv, FlashLds<HD> &lds) {
   constexpr int TPT = 16 / G; /* tokens per tile */
   constexpr int NS = HD / 4;  /* QK^T MFMA steps */
   constexpr int ND = HD / 16; /* output tiles over the head dimension */
   auto &xm = lds.xm, &xl = lds.xl;
   auto &xo = lds.xo;
   const int lane = threadIdx.x & 63, c = lane & 15, j = lane >> 4;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int last = min(t0 + TPT, a.ntok) - 1;
   const int pmax = a.pos + last; /* last key any row of the tile needs */
   /* B operand of S^T: row c's query, dims NS j .. NS j + NS - 1 */
@@ -543,7 +543,7 @@ __global__ __launch_bounds__(256) void flash_prefill_kernel(AttnArgs a) {
   __shared__ FlashLds<HD> lds;
   const int ntile = gridDim.x / a.n_kv;
   const int g = blockIdx.x % a.n_kv, tile = ntile - 1 - blockIdx.x / a.n_kv;
-  flash_tile<HD, G>(a, g, tile * (16 / G), lds);
+  flash_tile<HD, G>(a, g, tile * (16 / G), __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lds);
 }
 
 /* The same attention on the bf16 matrix cores without giving up fp32: every
@@ -554,8 +554,8 @@ __global__ __launch_bounds__(256) void flash_prefill_kernel(AttnArgs a) {
  * mid), each exact, summed in fp32.  bf16 products run 16 times as fast as
  * fp32 ones (v_mfma_f32_16x16x4_f32), so six of them cost 0.38 of one.
  *
- * One workgroup of four waves takes 64 query rows = 64 / G tokens x the G
- * query heads of a KV head, and streams the keys in blocks of 64: wave (rg,
+ * One workgroup of eight waves takes 128 query rows = 128 / G tokens x the
+ * G query heads of a KV head, and streams the keys in blocks of 64: wave (rg,
  * kh) rows 32 rg .. + 31 against keys 32 kh .. + 31 of every block, online
  * softmax, the two halves of the keys combined at the end.  K and V are
  * loaded once per workgroup a block ahead into registers, split, and put into
@@ -571,23 +571,55 @@ __global__ __launch_bounds__(256) void flash_prefill_kernel(AttnArgs a) {
  * Octets (8 bf16, 16 bytes) are XOR-swizzled by the row, so operand reads
  * are free of bank conflicts.
  *
- * 32 heads over 8, head_dim 128, 512 tokens at 3584: 383 -> 270 us with RoPE
- * and append (118 TFLOP/s of fp32 products), the error against float64 6e-7
- * -> 2.8e-7.  Bound by the vector work between the matrix instructions (one
- * wave per SIMD: splitting 64 values and 16 exponentials a lane per block
- * beside 96 MFMAs).
+ * Launches that would leave CUs idle split the keys over the grid
+ * (AttnArgs.fs_split): each part leaves its unnormalised O, maximum and sum
+ * to flash_merge_kernel.
+ *
+ * Microseconds with RoPE and append, 32 heads over 8, head_dim 128, beside
+ * the fp32 kernel's: 512 tokens at 3584 380 -> 226 (two parts; 270 with 64
+ * rows a workgroup), 2048 at 0 448 -> 267, 128 at 2000 74 -> 58 (six parts),
+ * 37 at 8000 246 -> 111 (eight).  The error against float64 of the first is
+ * 6e-7 -> 2.4e-7.  Bound by what comes between the matrix instructions, 2.6
+ * of a block's 6.2 us: splitting 32 values and 16 probabilities a lane, the
+ * exponentials, 56 KB of operands a wave from LDS.
  *
  * An infinity or NaN among the operands leaves NaN in the splits and so in
- * the outputs it reaches; a tile with such an output is computed again by
- * flash_tile, which treats them as fp32 arithmetic does. */
+ * the outputs it reaches; a tile with an output that is not finite is computed
+ * again by flash_tile, which treats them as fp32 arithmetic does. */
 typedef __bf16 gq_bf8a __attribute__((ext_vector_type(8)));
 typedef float gq_f16a __attribute__((ext_vector_type(16)));
 
-constexpr int kFsKeys = 64, kFsRows = 64;
-/* Fewer workgroups than this leave most of the chip idle, and the fp32
- * kernel's 16-row tiles win: at 77 tokens x 32 heads (40 workgroups, 378 keys)
- * it takes 10 us where this one would take 6 blocks x 4.4. */
-constexpr int kFsMinWgs = 96;
+constexpr int kFsKeys = 64, kFsRows = 128, kFsThreads = 512;
+
+/* The launch for ntok tokens at pos: the fp32 kernel (split 0), or the
+ * split-bf16 kernel with its keys in so many parts, whichever should take
+ * less.  Microseconds from measured launches at head_dim 128 (at 64 half of
+ * them): the fp32 kernel 2.8 per 64 keys when its 16-row workgroups fill the
+ * chip twice over, down to 1.5 when they leave it nearly empty; the other 6.2
+ * per block of 64 keys and workgroup, 4 at its ends, and 5 more plus the
+ * parts' way through memory where it splits the keys.  Measured over sixteen
+ * launches (head_dim 64 and 128, 37 to 2048 tokens at 0 to 8000): within 8% of
+ * the best choice for each. */
+struct FlashShape {
+  int split, wgs;
+};
+constexpr int kFsMaxSplit = 8;
+FlashShape flash_shape(int ntok, int pos, int n_heads, int n_kv, int hd, int n_cu, bool parts) {
+  const int G = n_heads / n_kv, tpt = kFsRows / G, wgs = (ntok + tpt - 1) / tpt * n_kv;
+  const int nblk = (pos + ntok - 1) / kFsKeys + 1; /* the longest tile's */
+  const double mean = (pos + 0.5 * ntok) / kFsKeys + 1, even = (double)pos / (pos + ntok);
+  /* tiles of one length run in whole rounds, causal ones fill each other's */
+  auto blocks = [&](double r) { return r <= 1 ? nblk : even * std::ceil(r) * nblk + (1 - even) * r * mean; };
+  const double narrow = (double)((ntok + 16 / G - 1) / (16 / G)) * n_kv / (2 * n_cu), scale = hd / 128.0;
+  double best = scale * blocks(narrow) * (1.5 + 1.3 * std::min(1.0, narrow));
+  FlashShape f{0, wgs};
+  for (int k = 1; k == 1 || (parts && k <= kFsMaxSplit && nblk / k >= 2); k++) {
+    const double us = scale * blocks((double)wgs * k / n_cu) / k * 6.2 + 4.0 +
+                      (k > 1 ? 5.0 + 8.0 * k * ntok * n_heads * hd / 4.0e6 : 0.0);
+    if (us < best) best = us, f.split = k;
+  }
+  return f;
+}
 
 /* two floats to their (hi, mid, lo) bf16 pairs, each rounded to nearest even */
 __device__ __forceinline__ void split3(float x, float y, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
@@ -596,6 +628,18 @@ __device__ __forceinline__ void split3(float x, float y, uint32_t &hi, uint32_t 
   mid = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2a){x, y}, gq_bf2a));
   x -= __builtin_bit_cast(float, mid << 16), y -= __builtin_bit_cast(float, mid & 0xffff0000u);
   lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2a){x, y}, gq_bf2a));
+}
+
+/* four consecutive outputs, fp32 or bf16 */
+__device__ __forceinline__ void flash_store(const AttnArgs &a, size_t at, const float (&y)[4]) {
+  if (a.out16) {
+    uint2 u;
+    u.x = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2a){y[0], y[1]}, gq_bf2a));
+    u.y = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2a){y[2], y[3]}, gq_bf2a));
+    gst<uint2>(a.out16 + at, u);
+  } else {
+    gst<float4>(a.out + at, make_float4(y[0], y[1], y[2], y[3]));
+  }
 }
 
 struct Split8 {
@@ -614,56 +658,65 @@ __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
 constexpr int kFsA[6] = {1, 2, 0, 1, 0, 0}, kFsB[6] = {1, 0, 2, 0, 1, 0};
 
 template <int HD, int G>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void flash_split_kernel(AttnArgs a) {
+__global__ __launch_bounds__(kFsThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void flash_split_kernel(AttnArgs a) {
   constexpr int TPT = kFsRows / G;       /* tokens per workgroup */
   constexpr int NO = HD / 8;             /* octets of a K row */
   constexpr int NSL = HD / 16;           /* dim slices of S^T */
   constexpr int ND = HD / 32;            /* dim tiles of O^T */
   constexpr int KPL = kFsKeys * HD * 2;  /* bytes of one K (or V) plane */
-  constexpr int KT = kFsKeys * NO / 256; /* K octets per thread */
-  constexpr int VTH = kFsKeys / 8 * HD / 4; /* threads with a V task: 8 keys x 4 dims */
-  static_assert(6 * KPL >= (int)sizeof(FlashLds<HD>) && 6 * KPL >= 2 * 64 * 4 * (ND * 16 + 2), "exchanges fit the planes");
-  __shared__ __attribute__((aligned(16))) uint8_t smem_[6 * KPL];
-  __shared__ int s_nan;
+  constexpr int KT = kFsKeys * NO / kFsThreads; /* K octets per thread */
+  constexpr int VTH = kFsKeys / 8 * HD / 2; /* threads with a V task: 8 keys x 2 dims */
+  static_assert(6 * KPL >= 2 * (int)sizeof(FlashLds<HD>) && 6 * KPL >= 4 * 64 * 4 * (ND * 16 + 2), "exchanges fit the planes");
+  /* K's planes, V's planes, and Q's third plane [slice][row group][lane]: in
+   * registers it did not fit beside the other two */
+  __shared__ __attribute__((aligned(16))) uint8_t smem_[6 * KPL + NSL * 4096];
+  __shared__ int s_bad;
   GQ_LDS uint8_t *smem = (GQ_LDS uint8_t *)smem_;
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), rg = wv >> 1, kh = wv & 1;
-  const int ntile = gridDim.x / a.n_kv; /* heads and tiles as in flash_prefill_kernel */
+  /* heads and tiles as in flash_prefill_kernel */
+  const int ntile = gridDim.x / a.n_kv;
   const int g = blockIdx.x % a.n_kv, tile = ntile - 1 - blockIdx.x / a.n_kv, t0 = tile * TPT;
   const int pmax = a.pos + min(t0 + TPT, a.ntok) - 1; /* last key any row of the tile needs */
   const int nblk = pmax / kFsKeys + 1;
+  /* this part's key blocks b0 .. b1 - 1 */
+  const int b0 = nblk * (int)blockIdx.y / a.fs_split, b1 = nblk * ((int)blockIdx.y + 1) / a.fs_split;
   const float *K = a.k + (size_t)g * a.max_seq * HD;
   const float *V = a.v + (size_t)g * a.max_seq * HD;
-  if (tid == 0) s_nan = 0;
+  if (tid == 0) s_bad = 0;
   /* this lane's query row: token t0 + row / G, head g G + row % G */
   const int row = 32 * rg + r, qt = min(t0 + row / G, a.ntok - 1), qh = g * G + row % G;
   const int cpos = a.pos + t0 + row / G;
-  Split8 q[NSL]; /* dims 16 s + 8 h .. + 7 */
+  uint4 q[NSL][2]; /* dims 16 s + 8 h .. + 7 */
+  const uint32_t qlo = (uint32_t)(6 * KPL + (rg * 64 + lane) * 16);
 #pragma unroll
   for (int s = 0; s < NSL; s++) {
     const float *qp = a.q + (size_t)qt * a.q_stride + (size_t)qh * HD + 16 * s + 8 * h;
     const float4 u = gld<float4>(qp), v = gld<float4>(qp + 4);
     const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-    q[s] = split8(x);
+    const Split8 p = split8(x);
+    q[s][0] = p.p[0], q[s][1] = p.p[1];
+    if (kh == 0) lst<uint4>(smem, qlo + 4096 * s, p.p[2]);
   }
-  /* K tasks: octet ko of keys tid / NO + (256 / NO) i; V task: dims 4 vd ..
+  /* K tasks: octet ko of keys tid / NO + (512 / NO) i; V task: dims 2 vd ..
    * of the eight keys of octet vo, in P's order: key octet 4 kh + 2 t + h is
    * keys 32 kh + 16 t + 4 h + {0..3, 8..11} */
   const int ko = tid % NO, kk = tid / NO;
-  const int vd = tid % (HD / 4), vo = (tid / (HD / 4)) & 7;
+  const int vd = tid % (HD / 2), vo = (tid / (HD / 2)) & 7;
   const int vkey = 32 * (vo >> 2) + 16 * ((vo >> 1) & 1) + 4 * (vo & 1);
-  float4 kr[KT][2], vr[8];
+  float4 kr[KT][2];
+  float2 vr[8];
   auto load = [&](int b) {
     const int key0 = b * kFsKeys;
 #pragma unroll
     for (int i = 0; i < KT; i++) {
-      const float *kp = K + (size_t)min(key0 + kk + 256 / NO * i, pmax) * HD + 8 * ko;
+      const float *kp = K + (size_t)min(key0 + kk + kFsThreads / NO * i, pmax) * HD + 8 * ko;
       kr[i][0] = gld<float4>(kp), kr[i][1] = gld<float4>(kp + 4);
     }
-    if (VTH == 256 || tid < VTH) {
+    if (VTH == kFsThreads || tid < VTH) {
 #pragma unroll
       for (int e = 0; e < 8; e++) /* keys past pmax repeat it: their weight is 0 */
-        vr[e] = gld<float4>(V + (size_t)min(key0 + vkey + (e & 3) + 8 * (e >> 2), pmax) * HD + 4 * vd);
+        vr[e] = gld<float2>(V + (size_t)min(key0 + vkey + (e & 3) + 8 * (e >> 2), pmax) * HD + 2 * vd);
     }
   };
   auto stage = [&]() {
@@ -671,19 +724,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     for (int i = 0; i < KT; i++) {
       const float x[8] = {kr[i][0].x, kr[i][0].y, kr[i][0].z, kr[i][0].w, kr[i][1].x, kr[i][1].y, kr[i][1].z, kr[i][1].w};
       const Split8 s = split8(x);
-      const int key = kk + 256 / NO * i;
+      const int key = kk + kFsThreads / NO * i;
       const uint32_t at = (uint32_t)(key * HD * 2 + ((ko ^ (key & (NO - 1))) << 4));
 #pragma unroll
       for (int p = 0; p < 3; p++) lst<uint4>(smem, (uint32_t)(p * KPL) + at, s.p[p]);
     }
-    if (VTH == 256 || tid < VTH) {
+    if (VTH == kFsThreads || tid < VTH) {
 #pragma unroll
-      for (int d = 0; d < 4; d++) {
+      for (int d = 0; d < 2; d++) {
         float x[8];
 #pragma unroll
-        for (int e = 0; e < 8; e++) x[e] = d == 0 ? vr[e].x : d == 1 ? vr[e].y : d == 2 ? vr[e].z : vr[e].w;
+        for (int e = 0; e < 8; e++) x[e] = d == 0 ? vr[e].x : vr[e].y;
         const Split8 s = split8(x);
-        const int dim = 4 * vd + d;
+        const int dim = 2 * vd + d;
         const uint32_t at = (uint32_t)(3 * KPL + dim * kFsKeys * 2 + ((vo ^ ((dim ^ (dim >> 3)) & 7)) << 4));
 #pragma unroll
         for (int p = 0; p < 3; p++) lst<uint4>(smem, (uint32_t)(p * KPL) + at, s.p[p]);
@@ -693,30 +746,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   /* operand addresses: K row 32 kh + r, octet 2 s + h; V row 32 d + r, octet
    * 4 kh + 2 t + h */
   const int krow = 32 * kh + r;
+  const uint32_t kbase = (uint32_t)(krow * HD * 2 + ((h ^ (krow & (NO - 1))) << 4));
+  const uint32_t vbase = (uint32_t)(r * kFsKeys * 2 + (((4 * kh + h) ^ ((r ^ (r >> 3)) & 7)) << 4));
   float m = -INFINITY, l = 0.f;
   gq_f16a o[ND];
 #pragma unroll
   for (int d = 0; d < ND; d++) o[d] = gq_f16a{};
-  load(0);
-  for (int b = 0; b < nblk; b++) {
+  if (b0 < b1) load(b0);
+  for (int b = b0; b < b1; b++) {
     __syncthreads(); /* the planes are free */
     stage();
     __syncthreads();
-    if (b + 1 < nblk) load(b + 1);
+    if (b + 1 < b1) load(b + 1);
     const int key0 = b * kFsKeys + 32 * kh;
     if (key0 > pmax) continue; /* none of this wave's keys (uniform in the wave) */
+    /* addresses from these, one XOR each, anew in every block: kept across
+     * blocks they cost the registers that O needs */
+    uint32_t kb = kbase, vb = vbase, qb = qlo;
+    asm volatile("" : "+v"(kb), "+v"(vb), "+v"(qb));
     gq_f16a sa = gq_f16a{}, sb = gq_f16a{};
 #pragma unroll
     for (int s = 0; s < NSL; s++) {
       gq_bf8a kv[3];
+      const gq_bf8a qv[3] = {__builtin_bit_cast(gq_bf8a, q[s][0]), __builtin_bit_cast(gq_bf8a, q[s][1]),
+                             lld<gq_bf8a>(smem, qb + 4096 * s)};
 #pragma unroll
       for (int p = 0; p < 3; p++)
-        kv[p] = lld<gq_bf8a>(smem, (uint32_t)(p * KPL + krow * HD * 2 + (((2 * s + h) ^ (krow & (NO - 1))) << 4)));
+        kv[p] = lld<gq_bf8a>(smem, (kb ^ (32 * s)) + p * KPL);
 #pragma unroll
       for (int u = 0; u < 6; u++) {
-        const gq_bf8a qv = __builtin_bit_cast(gq_bf8a, q[s].p[kFsB[u]]);
-        if (u < 5) sb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kv[kFsA[u]], qv, sb, 0, 0, 0);
-        else sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kv[kFsA[u]], qv, sa, 0, 0, 0);
+        if (u < 5) sb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kv[kFsA[u]], qv[kFsB[u]], sb, 0, 0, 0);
+        else sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kv[kFsA[u]], qv[kFsB[u]], sa, 0, 0, 0);
       }
     }
     /* scores of keys key0 + 8 (e / 4) + 4 h + e % 4 */
@@ -757,15 +817,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
      * over 4096 keys was above the fp32 kernel's) */
 #pragma unroll
     for (int d = 0; d < ND; d++) {
+      if (HD > 64) __builtin_amdgcn_sched_barrier(0); /* no operands read further ahead: registers */
       gq_f16a pv = gq_f16a{};
-      const int dim = 32 * d + r;
 #pragma unroll
       for (int t = 0; t < 2; t++) {
-        const int oct = 4 * kh + 2 * t + h;
         gq_bf8a vv[3];
 #pragma unroll
         for (int q3 = 0; q3 < 3; q3++)
-          vv[q3] = lld<gq_bf8a>(smem, (uint32_t)((3 + q3) * KPL + dim * kFsKeys * 2 + ((oct ^ ((dim ^ (dim >> 3)) & 7)) << 4)));
+          vv[q3] = lld<gq_bf8a>(smem, (vb ^ (((4 * d & 7) ^ (2 * t)) << 4)) + (3 + q3) * KPL + 32 * d * kFsKeys * 2);
 #pragma unroll
         for (int u = 0; u < 6; u++)
           pv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv[kFsA[u]], __builtin_bit_cast(gq_bf8a, ps[t].p[kFsB[u]]), pv, 0, 0, 0);
@@ -774,8 +833,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       for (int e = 0; e < 16; e++) o[d][e] = __builtin_fmaf(o[d][e], alpha, pv[e]);
     }
   }
-  /* the two halves of the keys: kh = 1 hands (m, l, O) to kh = 0, whose first
-   * block holds key 0, so its m is finite */
+  /* the two halves of the keys: kh = 1 hands (m, l, O) to kh = 0 */
   __syncthreads();
   GQ_LDS float *x = (GQ_LDS float *)smem + rg * 64 * (ND * 16 + 2);
   if (kh == 1) {
@@ -787,10 +845,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   }
   __syncthreads();
   if (kh == 0) {
-    const float m1 = x[lane], mt = fmaxf(m, m1), s0 = __expf(m - mt), s1 = __expf(m1 - mt);
-    const float inv = 1.0f / (l * s0 + x[64 + lane] * s1);
+    /* a half (or a whole part of the keys) that holds no visible key of a
+     * row weighs 0; of an unsplit launch kh = 0 holds key 0 */
+    const float m1 = x[lane], mt = fmaxf(m, m1), mf = mt == -INFINITY ? 0.f : mt;
+    const float s0 = __expf(m - mf), s1 = __expf(m1 - mf), lt = l * s0 + x[64 + lane] * s1;
+    const bool parts = a.fs_split > 1;
+    const float inv = parts ? 1.0f : 1.0f / lt;
     const int t = t0 + row / G;
-    bool nan = false;
+    bool bad = false;
+    float *po = a.part_o + ((size_t)blockIdx.y * a.ntok + t) * (a.n_heads * HD) + qh * HD;
+    if (parts && t < a.ntok && h == 0) {
+      float *ml = a.part_ml + (((size_t)blockIdx.y * a.ntok + t) * a.n_heads + qh) * 2;
+      ml[0] = mt, ml[1] = lt;
+    }
 #pragma unroll
     for (int d = 0; d < ND; d++)
 #pragma unroll
@@ -799,54 +866,100 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           y[e] = (o[d][4 * c + e] * s0 + x[64 * (2 + 16 * d + 4 * c + e) + lane] * s1) * inv;
-          nan |= y[e] != y[e];
+          bad |= !(__builtin_fabsf(y[e]) < INFINITY);
         }
+        const int dim = 32 * d + 8 * c + 4 * h;
         if (t < a.ntok) {
-          const size_t at = (size_t)t * a.out_stride + (size_t)qh * HD + 32 * d + 8 * c + 4 * h;
-          if (a.out16) {
-            uint2 u;
-            u.x = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2a){y[0], y[1]}, gq_bf2a));
-            u.y = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2a){y[2], y[3]}, gq_bf2a));
-            gst<uint2>(a.out16 + at, u);
-          } else {
-            gst<float4>(a.out + at, make_float4(y[0], y[1], y[2], y[3]));
-          }
+          const size_t at = (size_t)t * a.out_stride + (size_t)qh * HD + dim;
+          if (parts) gst<float4>(po + dim, make_float4(y[0], y[1], y[2], y[3]));
+          else flash_store(a, at, y);
         }
       }
-    if (__ballot(nan) && lane == 0) s_nan = 1;
+    if (!parts && __ballot(bad) && lane == 0) s_bad = 1;
   }
   __syncthreads();
-  if (!s_nan) return;
-  for (int t = t0; t < min(t0 + TPT, a.ntok); t += 16 / G) {
-    flash_tile<HD, G>(a, g, t, *(FlashLds<HD> *)smem_);
+  if (!s_bad) return;
+  /* two 16-row tiles at a time, four waves each */
+  for (int t = t0; t < min(t0 + TPT, a.ntok); t += 32 / G) {
+    flash_tile<HD, G>(a, g, min(t + (wv >> 2) * (16 / G), (a.ntok - 1) / (16 / G) * (16 / G)), wv & 3, ((FlashLds<HD> *)smem_)[wv >> 2]);
     __syncthreads();
   }
 }
 
+/* The parts of a key-split launch: out = sum_s O_s e^(m_s - M) / sum_s l_s
+ * e^(m_s - M), a workgroup per 16 query rows (16 / G tokens x G heads),
+ * sixteen lanes a row; a tile with a result that is not finite goes through
+ * flash_tile. */
 template <int HD, int G>
-int launch_flash(const AttnArgs &a, hipStream_t s) {
-  const int wide = (a.ntok + kFsRows / G - 1) / (kFsRows / G) * a.n_kv;
-  if (wide >= kFsMinWgs)
-    hipLaunchKernelGGL((flash_split_kernel<HD, G>), dim3(wide), dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL((flash_prefill_kernel<HD, G>), dim3((a.ntok + 16 / G - 1) / (16 / G) * a.n_kv), dim3(256), 0, s,
-                       a);
+__global__ __launch_bounds__(256) void flash_merge_kernel(AttnArgs a) {
+  __shared__ FlashLds<HD> lds;
+  __shared__ int s_bad;
+  const int ntile = gridDim.x / a.n_kv;
+  const int g = blockIdx.x % a.n_kv, tile = ntile - 1 - blockIdx.x / a.n_kv, t0 = tile * (16 / G);
+  const int row = threadIdx.x >> 4, sub = threadIdx.x & 15, t = t0 + row / G, qh = g * G + row % G;
+  if (threadIdx.x == 0) s_bad = 0;
+  __syncthreads();
+  if (t < a.ntok) {
+    const float *ml = a.part_ml + ((size_t)t * a.n_heads + qh) * 2, *po = a.part_o + (size_t)t * (a.n_heads * HD) + qh * HD;
+    const size_t mls = (size_t)a.ntok * a.n_heads * 2, pos = (size_t)a.ntok * a.n_heads * HD;
+    float M = -INFINITY, L = 0.f;
+    for (int s = 0; s < a.fs_split; s++) M = fmaxf(M, ml[s * mls]);
+    for (int s = 0; s < a.fs_split; s++) L += ml[s * mls + 1] * __expf(ml[s * mls] - M);
+    const float inv = 1.0f / L;
+    bool bad = false;
+#pragma unroll
+    for (int d = 0; d < HD / 64; d++) {
+      const int dim = 64 * d + 4 * sub;
+      float y[4] = {0.f, 0.f, 0.f, 0.f};
+      for (int s = 0; s < a.fs_split; s++) {
+        const float w = __expf(ml[s * mls] - M);
+        const float4 u = gld<float4>(po + s * pos + dim);
+        y[0] = __builtin_fmaf(u.x, w, y[0]), y[1] = __builtin_fmaf(u.y, w, y[1]);
+        y[2] = __builtin_fmaf(u.z, w, y[2]), y[3] = __builtin_fmaf(u.w, w, y[3]);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; e++) y[e] *= inv, bad |= !(__builtin_fabsf(y[e]) < INFINITY);
+      flash_store(a, (size_t)t * a.out_stride + (size_t)qh * HD + dim, y);
+    }
+    if (bad) s_bad = 1;
+  }
+  __syncthreads();
+  if (s_bad) flash_tile<HD, G>(a, g, t0, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lds);
+}
+
+template <int HD, int G>
+int launch_flash(const AttnArgs &a0, int n_cu, hipStream_t s) {
+  AttnArgs a = a0;
+  const FlashShape f = flash_shape(a.ntok, a.pos, a.n_heads, a.n_kv, HD, n_cu, a.part_o != nullptr);
+  a.fs_split = f.split;
+  const int narrow = (a.ntok + 16 / G - 1) / (16 / G) * a.n_kv;
+  if (!f.split) {
+    hipLaunchKernelGGL((flash_prefill_kernel<HD, G>), dim3(narrow), dim3(256), 0, s, a);
+  } else {
+    hipLaunchKernelGGL((flash_split_kernel<HD, G>), dim3(f.wgs, f.split), dim3(kFsThreads), 0, s, a);
+    if (f.split > 1) hipLaunchKernelGGL((flash_merge_kernel<HD, G>), dim3(narrow), dim3(256), 0, s, a);
+  }
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
 } // namespace
 
-int gq_launch_flash_prefill(const AttnArgs &a, hipStream_t s) {
+size_t gq_flash_parts(int ntok, int pos, int n_heads, int n_kv, int hd, int n_cu) {
+  const FlashShape f = flash_shape(ntok, pos, n_heads, n_kv, hd, n_cu, true);
+  return f.split > 1 ? (size_t)f.split * ntok * n_heads : 0;
+}
+
+int gq_launch_flash_prefill(const AttnArgs &a, int n_cu, hipStream_t s) {
   if (a.n_kv <= 0 || a.n_heads % a.n_kv || a.ntok < 1 || a.pos < 0 || a.pos + a.ntok > a.max_seq) return -1;
   const int G = a.n_heads / a.n_kv;
-  if (a.hd == 128 && G == 4) return launch_flash<128, 4>(a, s);
-  if (a.hd == 128 && G == 8) return launch_flash<128, 8>(a, s);
-  if (a.hd == 128 && G == 1) return launch_flash<128, 1>(a, s);
-  if (a.hd == 128 && G == 2) return launch_flash<128, 2>(a, s);
-  if (a.hd == 64 && G == 4) return launch_flash<64, 4>(a, s);
-  if (a.hd == 64 && G == 8) return launch_flash<64, 8>(a, s);
-  if (a.hd == 64 && G == 1) return launch_flash<64, 1>(a, s);
-  if (a.hd == 64 && G == 2) return launch_flash<64, 2>(a, s);
+  if (a.hd == 128 && G == 4) return launch_flash<128, 4>(a, n_cu, s);
+  if (a.hd == 128 && G == 8) return launch_flash<128, 8>(a, n_cu, s);
+  if (a.hd == 128 && G == 1) return launch_flash<128, 1>(a, n_cu, s);
+  if (a.hd == 128 && G == 2) return launch_flash<128, 2>(a, n_cu, s);
+  if (a.hd == 64 && G == 4) return launch_flash<64, 4>(a, n_cu, s);
+  if (a.hd == 64 && G == 8) return launch_flash<64, 8>(a, n_cu, s);
+  if (a.hd == 64 && G == 1) return launch_flash<64, 1>(a, n_cu, s);
+  if (a.hd == 64 && G == 2) return launch_flash<64, 2>(a, n_cu, s);
   return -1;
 }
 

@@ -185,15 +185,21 @@ struct AttnArgs {
    * of fp32 to out.  Decode launches leave these zero. */
   int ntok, q_stride, out_stride;
   __bf16 *out16;
+  /* prefill: parts of the keys (set by the launcher; part_o and part_ml then
+   * hold gq_flash_parts() rows of hd and of 2 floats) */
+  int fs_split;
 };
 int gq_attn_nch(int n_kv, int max_seq);
 int gq_attn_smax(int max_seq, int nch);
 int gq_launch_attention(const AttnArgs &a, hipStream_t s, hipEvent_t mid);
 /* Causal attention of a prefill chunk (a.ntok tokens at a.pos, their keys
- * already appended) by the fp32-MFMA flash kernel: q, q_stride, k, v, out
+ * already appended) by the flash kernels: q, q_stride, k, v, out
  * or out16, out_stride, pos, ntok, n_heads, n_kv, hd (64 or 128), max_seq
  * and scale are used. */
-int gq_launch_flash_prefill(const AttnArgs &a, hipStream_t s);
+int gq_launch_flash_prefill(const AttnArgs &a, int n_cu, hipStream_t s);
+/* query rows of partial results the launch wants in part_o / part_ml (0:
+ * none); without them it does not split the keys */
+size_t gq_flash_parts(int ntok, int pos, int n_heads, int n_kv, int hd, int n_cu);
 
 struct RopeArgs {
   float *q;

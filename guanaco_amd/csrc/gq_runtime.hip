@@ -45,6 +45,8 @@ struct PrefillWs {
   __bf16 *xn = nullptr, *att = nullptr, *act = nullptr;          /* bf16 GEMM inputs */
   __bf16 *xb = nullptr; /* op-level entry: bf16 copy of its fp32 x */
   size_t xb_cap = 0;
+  float *fs = nullptr; /* partial results of the key-split attention */
+  size_t fs_cap = 0;
   float *part = nullptr; /* the GEMM's K-part sums (PgArgs.part) */
   size_t part_cap = 0;
 };
@@ -1473,7 +1475,10 @@ static int pf_attention(gq_ctx *c, int layer, int pos, int T, int n_heads, float
   aa.out = out, aa.out16 = out16, aa.out_stride = qd, aa.pos = pos, aa.ntok = T;
   aa.n_heads = n_heads, aa.n_kv = c->kv_heads, aa.hd = hd, aa.max_seq = c->kv_max_seq;
   aa.scale = 1.0f / sqrtf((float)hd);
-  return gq_launch_flash_prefill(aa, c->stream);
+  PrefillWs &w = c->pf;
+  if (const size_t rows = gq_flash_parts(T, pos, n_heads, c->kv_heads, hd, c->n_cu))
+    if (pf_ensure(c, w.fs, w.fs_cap, rows * (hd + 2)) == 0) aa.part_o = w.fs, aa.part_ml = w.fs + rows * hd;
+  return gq_launch_flash_prefill(aa, c->n_cu, c->stream);
 }
 
 /* one layer over the chunk (engine.c:352-554 with T tokens): 7 launches of

@@ -292,12 +292,23 @@ def test_prefill_gate_up_wide_tile(ctx, orc, T, N, K):
     (8, 8, 64, 0, 3, 16),          # G = 1, three tokens
     (64, 8, 128, 7, 33, 64),       # G = 8, two tokens per tile
     (16, 8, 64, 1, 21, 40),        # G = 2
-    # 96 workgroups of 64 rows and more: the split-bf16 kernel
+    # ragged tiles of the fp32 kernel
     (32, 4, 64, 77, 200, 277),     # G = 8, ragged last tile, ends at the cache end
     (32, 32, 64, 3, 190, 200),     # G = 1, 64 tokens per tile
     (32, 32, 128, 64, 129, 200),   # one token in the last tile
     (64, 8, 128, 63, 97, 160),     # the first key of a block is the last one seen
     (64, 32, 64, 0, 65, 65),       # G = 2, one token past a tile
+    # the split-bf16 kernel: its keys whole
+    (64, 64, 64, 0, 515, 515),     # G = 1, ragged last tile, ends at the cache end
+    (64, 32, 64, 0, 1025, 1025),   # G = 2, one token past a tile
+    (64, 64, 128, 0, 512, 640),    # whole tiles
+    # and in parts, merged
+    (32, 8, 128, 256, 512, 768),   # G = 4, two parts
+    (32, 8, 128, 0, 1000, 1000),   # two parts, the first tile with keys in one alone
+    (32, 4, 64, 2000, 257, 2257),  # G = 8, seven parts, one token past a tile
+    (64, 32, 128, 1300, 130, 1430),  # G = 2, five parts
+    (64, 8, 128, 1535, 33, 1600),  # eight parts, the first key of a block is the last one seen
+    (32, 8, 128, 8100, 1, 8160),   # one token
 ])
 def test_prefill_attention(ctx, orc, nh, nkv, hd, pre, T, ms):
     from oracle import HostKV, fptr
@@ -342,38 +353,42 @@ def test_prefill_attention(ctx, orc, nh, nkv, hd, pre, T, ms):
         b.free()
 
 
+@pytest.mark.parametrize("nh,nkv,pre,T", [(64, 64, 0, 512), (32, 8, 256, 768)])
 @pytest.mark.parametrize("bad", ["none", "k_inf", "v_inf", "v_nan", "q_nan", "huge"])
-def test_prefill_attention_wide_equals_narrow(ctx, bad):
-    """One launch over 256 tokens (the split-bf16 kernel) against the same
-    tokens in launches of 32 (the fp32 kernel): finite outputs to fp32
-    rounding, and exactly the same non-finite ones, for which the wide kernel
-    has to fall back to fp32 arithmetic."""
-    nh, nkv, hd, T, ms = 32, 8, 128, 256, 320
+def test_prefill_attention_wide_equals_narrow(ctx, bad, nh, nkv, pre, T):
+    """One launch over 512 tokens (the split-bf16 kernel; after a prefix its
+    keys in two parts) against the same tokens in launches of 32 (the fp32
+    kernel): finite outputs to fp32 rounding, and exactly the same non-finite
+    ones, for which the wide kernel has to fall back to fp32 arithmetic."""
+    hd, ms = 128, T + 64
     rng = np.random.default_rng(5)
     q = rng.standard_normal((T, nh * hd)).astype(np.float32)
     k = rng.standard_normal((T, nkv * hd)).astype(np.float32)
     v = rng.standard_normal((T, nkv * hd)).astype(np.float32)
     if bad == "k_inf":
-        k[70, 3 * hd + 6] = np.inf
+        k[70 + pre // 2, 3 * hd + 6] = np.inf
     elif bad == "v_inf":
         v[131, 2 * hd + 5] = -np.inf
     elif bad == "v_nan":
         v[9, 7 * hd + 127] = np.nan
     elif bad == "q_nan":
-        q[200, 11 * hd] = np.nan
+        q[T - 56, 11 * hd] = np.nan
     elif bad == "huge":  # rounds to an infinite bf16
         v[40, 0] = np.float32(3.4e38)
     got = []
-    for step in (T, 32):
+    for wide_step in (True, False):
         ctx.kv_init(1, nkv, hd, ms, 500000.0)
         out = []
-        for t in range(0, T, step):
+        t = 0
+        while t < T:
+            step = T - pre if wide_step and t >= pre else 32
             qb, kb, vb = (ctx.upload(a[t:t + step]) for a in (q, k, v))
             ob = ctx.alloc(4 * step * nh * hd)
             assert ctx.prefill_attention_dev(0, t, step, nh, qb, kb, vb, ob) == 0
             out.append(ob.download(count=step * nh * hd).reshape(step, nh * hd))
             for b in (qb, kb, vb, ob):
                 b.free()
+            t += step
         got.append(np.concatenate(out))
     wide, narrow = got
     assert np.array_equal(np.isnan(wide), np.isnan(narrow))
