@@ -285,9 +285,15 @@ extern "C" int gq_hip_device_info(gq_ctx *c, int *n_cu, char *name, int name_len
 }
 
 /* ------------------------------------------------------------ memory */
-static void *dev_alloc(gq_ctx *c, size_t bytes) {
+static bool dense_drop(gq_ctx *c);
+/* keep_copies: fail rather than take back the bf16 copies of the weights,
+ * which prompts can do without */
+static void *dev_alloc(gq_ctx *c, size_t bytes, bool keep_copies = false) {
   void *p = nullptr;
-  if (hipMalloc(&p, bytes + kPad) != hipSuccess) {
+  hipError_t e = hipMalloc(&p, bytes + kPad);
+  if (e != hipSuccess && !keep_copies && dense_drop(c)) e = hipMalloc(&p, bytes + kPad);
+  if (e != hipSuccess) {
+    (void)hipGetLastError(); /* not for the next launch's check: a caller may go on without */
     fail(c, -4, "hipMalloc(%zu) failed", bytes + kPad);
     return nullptr;
   }
@@ -308,6 +314,18 @@ extern "C" void gq_hip_free(gq_ctx *c, void *p) {
   (void)hipStreamSynchronize(c->stream);
   (void)hipFree(p);
   c->allocs.erase(it);
+}
+
+/* Give the bf16 copies back; false: there are none.  Prompts multiply by the
+ * quantized weights from then on, as models without copies do. */
+static bool dense_drop(gq_ctx *c) {
+  bool any = false;
+  for (auto &L : c->mm) {
+    if (!L.dn) continue;
+    gq_hip_free(c, L.dn);
+    L.dn = nullptr, any = true;
+  }
+  return any;
 }
 
 extern "C" int gq_hip_h2d(gq_ctx *c, void *dev, const void *host, size_t bytes) {
@@ -856,7 +874,7 @@ static void dense_build(gq_ctx *c, int l) {
     at[i] = n;
     if (i != 5) n += gq_dense_bytes(ws[i]->rows, ws[i]->cols, i == 4);
   }
-  M.dn = (uint8_t *)dev_alloc(c, n);
+  M.dn = (uint8_t *)dev_alloc(c, n, true);
   if (!M.dn) return;
   M.dn_at[0] = 0, M.dn_at[1] = at[3], M.dn_at[2] = at[4], M.dn_at[3] = at[6];
   for (int i = 0; i < 7; i++)
@@ -1387,7 +1405,7 @@ extern "C" int gq_hip_decode_loop(gq_ctx *c, int token, int pos, int n_steps, in
 
 /* ------------------------------------------------------------ prefill
  * forward(model, kv, scr, tokens, n, pos) for n > 1 (engine.c:559-595 with
- * transformer_layer's T-token path, engine.c:352-509): chunks of up to 512
+ * transformer_layer's T-token path, engine.c:352-509): chunks of up to 2048
  * tokens; per layer and chunk one GEMM launch per projection on the matrix
  * cores, RoPE + append of every token of the chunk, then causal attention
  * (token t sees positions 0 .. pos + t). */
@@ -1519,9 +1537,13 @@ static int pf_layer(gq_ctx *c, int l, int pos, int T, int &pending) {
   qkv.kparts_out = &kq;
   o.kparts_out = &ko;
   if (l + 1 < m.n_layers) down.kparts_out = &kd;
-  const uint8_t *dn = T >= kDenseTokens && (size_t)l < c->mm.size() && !gq_matvec_q6k_ref() ? c->mm[l].dn : nullptr;
   auto gemm = [&](int mode, const PgArgs &p, int i) {
-    if (!dn) return gq_launch_pgemm(mode, p, c->stream);
+    /* asked for at each launch: an allocation since the last may have taken
+     * the copies back */
+    const uint8_t *dn = T >= kDenseTokens && (size_t)l < c->mm.size() && !gq_matvec_q6k_ref() ? c->mm[l].dn : nullptr;
+    /* the bf16 launch needs a workspace to add into x; without one (out of
+     * memory) the other does it in place */
+    if (!dn || (mode == MV_RESID && !p.part)) return gq_launch_pgemm(mode, p, c->stream);
     DnArgs d{};
     d.x = p.x, d.w = dn + c->mm[l].dn_at[i], d.act = p.act, d.T = p.T, d.K = p.K;
     d.nseg = mode == MV_SWIGLU ? 1 : p.nseg;
@@ -1551,9 +1573,17 @@ extern "C" int gq_hip_prefill(gq_ctx *c, const int32_t *tokens, int n_tokens, in
   for (int i = 0; i < n_tokens; i++)
     if (tokens[i] < 0 || tokens[i] >= m.vocab) return fail(c, -1, "prefill: token %d out of range", tokens[i]);
   const bool gemm = pf_model_ok(c);
-  /* equal chunks */
-  const int nchunk = (n_tokens + kPrefillChunk - 1) / kPrefillChunk, chunk = (n_tokens + nchunk - 1) / nchunk;
-  if (gemm && (rc = pf_alloc(c, chunk))) return rc;
+  /* equal chunks; smaller ones where the activations of such a chunk find no
+   * memory */
+  auto chunks = [&](int most) {
+    const int n = (n_tokens + most - 1) / most;
+    return (n_tokens + n - 1) / n;
+  };
+  int chunk = chunks(kPrefillChunk);
+  if (gemm && (rc = pf_alloc(c, chunk))) {
+    chunk = chunks(512);
+    if ((rc = pf_alloc(c, chunk))) return rc;
+  }
   c->g_valid = false;
   PrefillWs &w = c->pf;
   Workspace &ws = c->ws;

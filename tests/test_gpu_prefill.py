@@ -627,3 +627,25 @@ def test_prefill_dense_copy_vs_quantized(orc, T, mix):
         print(f"dense copy vs quantized, T={T}: V rows {rel_l2(v[0], v[1]):.2e}, logits {rel_l2(a[0], b[0]):.2e}")
     finally:
         c.close()
+
+
+def test_prefill_dense_copy_given_back(orc):
+    """An allocation that the card has no room for takes the bf16 copies back
+    before it fails; prompts then multiply by the quantized weights, bit for
+    bit as on the layouts that have no copy."""
+    import guanaco_amd.hip as H
+    spec = S.ModelSpec("dense-back", n_layers=2, hidden=512, ff=1536, n_heads=8, n_kv_heads=2, vocab=1000,
+                       layer_dtypes=dict(wv=S.Q6_K, wd=S.Q6_K), q4k_zero_mean=True, norm_shift=4)
+    c = H.Context(0)
+    try:
+        dm = H.DeviceModel(c, spec, 512)
+        toks = np.random.default_rng(3).integers(0, spec.vocab, 300).astype(np.int32)
+        with H.matvec_path("auto_q6k_ref"):
+            ref = dm.prefill(toks, 0)[1]
+        with_copy = dm.prefill(toks, 0)[1]
+        with pytest.raises(H.HipError):
+            c.alloc(1 << 46)
+        after = dm.prefill(toks, 0)[1]
+        assert np.array_equal(bits(after), bits(ref)) and rel_l2(with_copy, ref) < 2e-3
+    finally:
+        c.close()
