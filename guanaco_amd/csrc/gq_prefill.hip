@@ -29,6 +29,11 @@
  * row, its k-octets), so a weight is converted once per token tile and never
  * round-trips through LDS in bf16.  One barrier per step.
  *
+ * Launches of up to 64 tokens take two (or four) row waves x four K splits
+ * a workgroup and up to eight K parts over the grid (launch_flat).  Chunks of
+ * 256 tokens and more of a bound model multiply by bf16 copies of the weights
+ * instead (gq_dense.hip).
+ *
  * The fused Q4_K gate/up launch runs a wide variant of the tile when its grid
  * fills the GPU: 64 rows per wave, so each A operand read feeds two MFMAs
  * (pgemm_wide_swiglu_kernel).

@@ -305,7 +305,7 @@ int gq_hip_argmax_dev(gq_ctx *ctx, const float *x, int n, int *out_index_dev);
  * per sampled token; unused for greedy).  logits: vocab floats in device
  * memory.  Returns the token, or -1 bad argument, -2 top_k above 1024, -4 HIP
  * error.  Every mode follows the reference's arithmetic order (plain
- * temperature sampling sums on one device thread, ~0.3 ms at 128256
+ * temperature sampling sums on one device thread, 0.8 ms at 128256
  * entries); exponentials come from the device's expf. */
 int gq_hip_sample_dev(gq_ctx *ctx, const float *logits, int vocab, float temperature, int top_k, float top_p,
                       int rnd);
@@ -368,7 +368,7 @@ int gq_hip_chat_turn(gq_ctx *ctx, const int32_t *tokens, int n_tokens, int *curr
                      int eos_token, float temperature, int top_k, float top_p, const int *rnd, int32_t *reply);
 /* forward(model, kv, scr, tokens, n_tokens, pos) of the bound model
  * (engine.c:559-595): the whole prompt through every layer in chunks of
- * up to 512 tokens, filling the device KV cache at pos .. pos+n_tokens-1;
+ * up to 2048 tokens, filling the device KV cache at pos .. pos+n_tokens-1;
  * the slot of gpu_prefill (gpu_prefill.h:13-20).  tokens and the optional
  * outputs are host pointers: logits (vocab floats) and hidden_last (the
  * last token's final hidden state before the final RMSNorm) of the last
