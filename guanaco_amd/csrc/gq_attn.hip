@@ -576,10 +576,10 @@ __global__ __launch_bounds__(256) void flash_prefill_kernel(AttnArgs a) {
  * to flash_merge_kernel.
  *
  * Microseconds with RoPE and append, 32 heads over 8, head_dim 128, beside
- * the fp32 kernel's: 512 tokens at 3584 380 -> 226 (two parts; 270 with 64
- * rows a workgroup), 2048 at 0 448 -> 267, 128 at 2000 74 -> 58 (six parts),
+ * the fp32 kernel's: 512 tokens at 3584 382 -> 216 (two parts; 270 with 64
+ * rows a workgroup), 2048 at 0 448 -> 256, 128 at 2000 74 -> 58 (six parts),
  * 37 at 8000 246 -> 111 (eight).  The error against float64 of the first is
- * 6e-7 -> 2.4e-7.  Bound by what comes between the matrix instructions, 2.6
+ * 6e-7 -> 2.6e-7.  Bound by what comes between the matrix instructions, 2.6
  * of a block's 6.2 us: splitting 32 values and 16 probabilities a lane, the
  * exponentials, 56 KB of operands a wave from LDS.
  *
