@@ -1413,6 +1413,7 @@ template <class T>
 static int pf_ensure(gq_ctx *c, T *&p, size_t &cap, size_t n) {
   if (cap >= n && p) return 0;
   if (p) gq_hip_free(c, p);
+  cap = 0;
   p = (T *)dev_alloc(c, sizeof(T) * n);
   if (!p) return -4;
   cap = n;
@@ -1499,19 +1500,17 @@ static int pf_attention(gq_ctx *c, int layer, int pos, int T, int n_heads, float
   return gq_launch_flash_prefill(aa, c->n_cu, c->stream);
 }
 
-/* one layer over the chunk (engine.c:352-554 with T tokens): 7 launches of
- * the GEMM (q/k/v together, gate/up together with SwiGLU), RMSNorms writing
- * bf16, RoPE + append + attention writing bf16 */
-/* the K-part workspace for a launch of T x (its segments' rows) */
-static void pf_parts(gq_ctx *c, PgArgs &a) {
-  PrefillWs &w = c->pf;
-  size_t rows = 0;
-  for (int i = 0; i < a.nseg; i++) rows += a.seg[i].rows;
-  const size_t n = gq_parts_tokens(a.T) * rows;
-  if (pf_ensure(c, w.part, w.part_cap, n) == 0) a.part = w.part, a.part_cap = w.part_cap;
+/* The K-part workspace of launches over T tokens and `rows` weight rows.  A
+ * prompt asks for it before its first layer: a request in between could free
+ * sums that a launch has left to the next. */
+static int pf_parts(gq_ctx *c, int T, size_t rows) {
+  return pf_ensure(c, c->pf.part, c->pf.part_cap, gq_parts_tokens(T) * rows);
 }
 
-/* pending: K parts of the previous layer's down launch still to be added
+/* One layer over the chunk (engine.c:352-554 with T tokens): 4 launches of
+ * the GEMM (q/k/v together, gate/up together with SwiGLU), RMSNorms writing
+ * bf16, RoPE + append + attention writing bf16.
+ * pending: K parts of the previous layer's down launch still to be added
  * into the residual x (0: none); this layer's first RMSNorm adds them, and
  * this layer leaves its own down's parts the same way unless it is the
  * last */
@@ -1529,7 +1528,8 @@ static int pf_layer(gq_ctx *c, int l, int pos, int T, int &pending) {
   gu.x = w.xn, gu.K = m.hidden, gu.nseg = 2, gu.act = w.act;
   gu.seg[0] = pg_seg(c, l, 4, L.w_gate, nullptr), gu.seg[1] = pg_seg(c, l, 5, L.w_up, nullptr);
   down.x = w.act, down.K = m.ff, down.nseg = 1, down.seg[0] = pg_seg(c, l, 6, L.w_down, w.x);
-  pf_parts(c, qkv), pf_parts(c, o), pf_parts(c, down);
+  /* a launch that needs more splits less, or not at all */
+  for (PgArgs *a : {&qkv, &o, &down}) a->part = w.part, a->part_cap = w.part_cap;
   /* the q/k/v launch leaves its K parts' sum to the RoPE + append kernel,
    * o and down theirs to the next RMSNorm (the last layer's down sums its
    * own: the LM head reads x) */
@@ -1584,6 +1584,9 @@ extern "C" int gq_hip_prefill(gq_ctx *c, const int32_t *tokens, int n_tokens, in
     chunk = chunks(512);
     if ((rc = pf_alloc(c, chunk))) return rc;
   }
+  /* for every launch of a chunk, or for o and down alone, or none: the
+   * launches do with what there is */
+  if (gemm && pf_parts(c, chunk, m.hidden + 2 * (size_t)m.n_kv_heads * m.head_dim)) (void)pf_parts(c, chunk, m.hidden);
   c->g_valid = false;
   PrefillWs &w = c->pf;
   Workspace &ws = c->ws;
@@ -2031,7 +2034,7 @@ extern "C" int gq_hip_prefill_gemm_dev(gq_ctx *c, int dtype, int mode, const voi
   if (!(a.x = pf_x16(c, x, (size_t)t * k))) return fail(c, -4, "prefill GEMM: x conversion");
   const uint8_t *ps = op_units(c, dtype, w, n, k);
   a.T = t, a.K = k, a.nseg = 1, a.seg[0] = op_seg(ps, w, y, n, dtype);
-  pf_parts(c, a);
+  if (pf_parts(c, t, n) == 0) a.part = c->pf.part, a.part_cap = c->pf.part_cap;
   if (mode == 1 && r != y)
     HIPCHK(c, hipMemcpyAsync(y, r, sizeof(float) * (size_t)t * n, hipMemcpyDeviceToDevice, c->stream));
   const int rc = gq_launch_pgemm(mode == 1 ? MV_RESID : MV_STORE, a, c->stream);
@@ -2049,7 +2052,7 @@ extern "C" float gq_hip_time_prefill_gemm(gq_ctx *c, int dtype, const void *w, i
   if (!(a.x = pf_x16(c, x, (size_t)t * k))) return fail(c, -4, "time GEMM: x conversion"), -1.f;
   const uint8_t *ps = op_units(c, dtype, w, n, k);
   a.T = t, a.K = k, a.nseg = 1, a.seg[0] = op_seg(ps, w, y, n, dtype);
-  pf_parts(c, a);
+  if (pf_parts(c, t, n) == 0) a.part = c->pf.part, a.part_cap = c->pf.part_cap;
   EventPair ev;
   int rc = ev.create() == hipSuccess ? 0 : -4;
   if (!rc) rc = gq_launch_pgemm(MV_STORE, a, c->stream); /* untimed first launch */

@@ -1,0 +1,87 @@
+"""The host side of the library on a CPU: gq_runtime.hip linked with
+tests/native/fake_device.cpp, which stands for the HIP runtime and the kernel
+launchers.  It gives device memory a size, refuses allocations on request, and
+follows what the launchers are handed: that workspaces are alive and large
+enough, and that the K-part sums one launch leaves reach the launch that adds
+them.  What the kernels compute is not part of it."""
+import ctypes as C
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+import guanaco_amd.hip as H
+from guanaco_amd import spec as S
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+GB = 1 << 30
+SMALL = S.ModelSpec("host-test", n_layers=4, hidden=512, ff=1024, n_heads=8, n_kv_heads=2, vocab=1000,
+                    layer_dtypes={k: S.Q8_0 for k in S.LAYER_WEIGHTS}, embed_dtype=S.Q8_0, lm_head_dtype=S.Q8_0)
+
+
+@pytest.fixture(scope="module")
+def built(tmp_path_factory):
+    if not os.path.exists(HIPCC):
+        pytest.skip("no hipcc")
+    d = tmp_path_factory.mktemp("fake")
+    flags = ["--offload-arch=gfx950", "--offload-host-only", "-O1", "-fPIC", "-std=c++17", "-I",
+             os.path.join(ROOT, "guanaco_amd", "csrc")]
+    objs = []
+    for src in (os.path.join(ROOT, "guanaco_amd", "csrc", "gq_runtime.hip"),
+                os.path.join(ROOT, "tests", "native", "fake_device.cpp")):
+        objs.append(str(d / (os.path.basename(src) + ".o")))
+        subprocess.run([HIPCC, *flags, "-x", "hip", "-c", src, "-o", objs[-1]], check=True)
+    # the device code that the host object registers is not there
+    nm = subprocess.run(["nm", "-u", objs[0]], capture_output=True, text=True, check=True).stdout
+    fat = [w for w in nm.split() if w.startswith("__hip_fatbin")]
+    stub = d / "fatbin.c"
+    stub.write_text("".join(f"char {w}[64];\n" for w in fat))
+    so = str(d / "libfake.so")
+    subprocess.run(["g++", "-shared", "-fPIC", "-Wl,-Bsymbolic", "-o", so, *objs, "-x", "c++", str(stub)], check=True)
+    lib = C.CDLL(so)
+    for n in (n for n in H.EXPORTS if hasattr(lib, n)):
+        f, g = getattr(lib, n), getattr(H.lib, n)
+        f.restype, f.argtypes = g.restype, g.argtypes
+    lib.fake_errors.restype = C.c_char_p
+    lib.fake_count.restype, lib.fake_count.argtypes = C.c_long, [C.c_char_p]
+    lib.fake_used.restype = C.c_size_t
+    lib.fake_reset.argtypes = lib.fake_refuse_from.argtypes = [C.c_size_t]
+    return lib
+
+
+@pytest.fixture
+def dev(built, monkeypatch):
+    """The fake library in place of the real one, 288 GB free; no launch may
+    have been handed dead memory or lost sums by the end."""
+    built.fake_reset(288 * GB)
+    monkeypatch.setattr(H, "lib", built)
+    built.n = lambda what: built.fake_count(what.encode())
+    yield built
+    assert built.fake_errors() == b""
+
+
+def prompt(dm, T, pos=0):
+    return dm.prefill(np.arange(T) % 1000, pos)[0]
+
+
+@pytest.mark.parametrize("T", [40, 100, 300])
+@pytest.mark.parametrize("room", ["all", "o_down", "none"])
+def test_prompt_sums_survive_short_workspaces(dev, T, room):
+    """K-part sums of one layer's down projection are still owed when the next
+    layer starts.  Where the card has room for the workspace of o and down but
+    not for the larger one of q/k/v (or for none), no request of that next
+    layer may free or replace it before they are added."""
+    kvd, hid = SMALL.n_kv_heads * SMALL.head_dim, SMALL.hidden
+    tokens = 8 * T if T <= 64 else 4 * T
+    with H.Context(0) as ctx:
+        dm = H.DeviceModel(ctx, SMALL, 512)
+        first = prompt(dm, 2)  # the activations of up to 512 tokens are there
+        if room != "all":
+            assert 4 * tokens * hid < 4 * tokens * (hid + 2 * kvd)
+            dev.fake_refuse_from(4 * tokens * ((hid + 2 * kvd) if room == "o_down" else 1))
+        for _ in range(2):
+            assert prompt(dm, T) == first
+        assert dev.n("refused") > 0 or room == "all"
