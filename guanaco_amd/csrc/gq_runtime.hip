@@ -328,8 +328,29 @@ static bool dense_drop(gq_ctx *c) {
   return any;
 }
 
+/* The copies hold the weights as they were: a write to a bound projection's
+ * own memory, in place, gives them back. */
+static size_t block_bytes(int dtype, int *qk);
+static void weights_written(gq_ctx *c, const void *dst, size_t bytes) {
+  const uintptr_t a = (uintptr_t)dst, b = a + bytes;
+  for (size_t l = 0; l < c->mm.size() && l < c->layers.size(); l++) {
+    if (!c->mm[l].dn) continue;
+    const gq_layer &L = c->layers[l];
+    for (const gq_weight *w : {&L.wq, &L.wk, &L.wv, &L.wo, &L.w_gate, &L.w_up, &L.w_down}) {
+      int qk;
+      const size_t bb = block_bytes(w->dtype, &qk);
+      const uintptr_t p = (uintptr_t)w->data;
+      if (a < p + (size_t)w->rows * (w->cols / qk) * bb && p < b) {
+        (void)dense_drop(c);
+        return;
+      }
+    }
+  }
+}
+
 extern "C" int gq_hip_h2d(gq_ctx *c, void *dev, const void *host, size_t bytes) {
   if (!c || !dev || !host) return -1;
+  weights_written(c, dev, bytes);
   HIPCHK(c, hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return 0;
@@ -411,6 +432,8 @@ extern "C" int gq_hip_synth_quant(gq_ctx *c, void *dev, int dtype, int rows, int
   if (!c || !dev || rows <= 0 || cols <= 0) return -1;
   int rc = gq_launch_synth_quant(dev, dtype, rows, cols, seed, c->stream);
   if (rc) return fail(c, rc, "synth_quant: bad dtype/shape");
+  int qk;
+  if (const size_t bb = block_bytes(dtype & 0xff, &qk)) weights_written(c, dev, (size_t)rows * (cols / qk) * bb);
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -2116,6 +2139,7 @@ extern "C" float gq_hip_time_read(gq_ctx *c, const void *src, size_t bytes, size
 
 extern "C" int gq_hip_copy_dev(gq_ctx *c, void *dst, const void *src, size_t bytes) {
   if (!c || !dst || !src) return -1;
+  weights_written(c, dst, bytes);
   const int rc = gq_launch_copy(dst, src, bytes, c->n_cu, c->stream);
   return rc ? fail(c, rc, "copy: sizes and pointers must be multiples of 16 bytes") : 0;
 }

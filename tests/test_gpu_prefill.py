@@ -23,6 +23,8 @@ sequential oracle steps (bit-exact with the reference's forward()): the
 projections see bf16 inputs, so the last token's logits and the new cache
 rows are held to 3e-2 relative L2 (observed about 5e-3) and the next greedy
 token must agree."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -647,5 +649,30 @@ def test_prefill_dense_copy_given_back(orc):
             c.alloc(1 << 46)
         after = dm.prefill(toks, 0)[1]
         assert np.array_equal(bits(after), bits(ref)) and rel_l2(with_copy, ref) < 2e-3
+    finally:
+        c.close()
+
+
+def test_prefill_weights_rewritten_in_place(orc):
+    """A Q8_0 model whose weights are written again in place after it was
+    bound: a prompt of 300 tokens sees the new ones, as a model bound after the
+    write does (2e-3, as between the kernels above), and not the copy of the
+    old ones."""
+    import guanaco_amd.hip as H
+    spec = S.ModelSpec("dense-rewrite", n_layers=2, hidden=512, ff=1024, n_heads=8, n_kv_heads=2, vocab=1000,
+                       layer_dtypes={k: S.Q8_0 for k in S.LAYER_WEIGHTS}, embed_dtype=S.Q8_0, lm_head_dtype=S.Q8_0)
+    toks = np.random.default_rng(4).integers(0, spec.vocab, 300).astype(np.int32)
+    c = H.Context(0)
+    try:
+        dm = H.DeviceModel(c, spec, 512)
+        old = dm.prefill(toks, 0)[1]
+        for l, k in ((0, "wv"), (1, "wd")):
+            w = dm.weight(l, k)
+            new = orc.synth_quant(S.Q8_0, 99 + l, w.rows, w.cols)
+            c.check(H.lib.gq_hip_h2d(c.h, w.data, new.ctypes.data, new.nbytes), "h2d")
+        got = dm.prefill(toks, 0)[1]
+        c.check(H.lib.gq_hip_model_bind(c.h, C.byref(dm.model)), "model_bind")
+        ref = dm.prefill(toks, 0)[1]
+        assert rel_l2(got, ref) < 2e-3 and rel_l2(old, ref) > 0.1
     finally:
         c.close()

@@ -85,3 +85,28 @@ def test_prompt_sums_survive_short_workspaces(dev, T, room):
         for _ in range(2):
             assert prompt(dm, T) == first
         assert dev.n("refused") > 0 or room == "all"
+
+
+@pytest.mark.parametrize("how", ["h2d", "synth", "copy", "elsewhere"])
+def test_weights_written_in_place(dev, how):
+    """A bound projection's memory written in place through the context: later
+    prompts do not multiply by a bf16 copy of what was there before."""
+    with H.Context(0) as ctx:
+        dm = H.DeviceModel(ctx, SMALL, 512)
+        w = dm.weight(2, "wu")
+        prompt(dm, 300)
+        assert dev.n("dense") == 4 * SMALL.n_layers
+        src = ctx.alloc(4096)
+        if how == "h2d":  # its last block
+            n = S.qbytes(w.dtype, w.rows, w.cols)
+            ctx.check(dev.gq_hip_h2d(ctx.h, w.data + n - 34, np.zeros(34, np.uint8).ctypes.data, 34), "h2d")
+        elif how == "synth":
+            ctx.check(dev.gq_hip_synth_quant(ctx.h, w.data, w.dtype, w.rows, w.cols, 77), "synth")
+        elif how == "copy":
+            ctx.check(dev.gq_hip_copy_dev(ctx.h, w.data, src.ptr, 4096), "copy")
+        else:
+            src.upload(np.zeros(1024, np.float32))
+        before = dev.n("dense_tile")
+        prompt(dm, 300)
+        stale = dev.n("dense") == 8 * SMALL.n_layers and dev.n("dense_tile") == before
+        assert stale == (how == "elsewhere")
