@@ -944,13 +944,20 @@ int launch_flash(const AttnArgs &a0, int n_cu, hipStream_t s) {
 
 } // namespace
 
+bool gq_flash_takes(int n_heads, int n_kv, int hd) {
+  if (n_kv <= 0 || n_heads <= 0 || n_heads % n_kv || (hd != 64 && hd != 128)) return false;
+  const int G = n_heads / n_kv;
+  return G == 1 || G == 2 || G == 4 || G == 8;
+}
+
 size_t gq_flash_parts(int ntok, int pos, int n_heads, int n_kv, int hd, int n_cu) {
+  if (!gq_flash_takes(n_heads, n_kv, hd)) return 0; /* flash_shape divides by 16 / G */
   const FlashShape f = flash_shape(ntok, pos, n_heads, n_kv, hd, n_cu, true);
   return f.split > 1 ? (size_t)f.split * ntok * n_heads : 0;
 }
 
 int gq_launch_flash_prefill(const AttnArgs &a, int n_cu, hipStream_t s) {
-  if (a.n_kv <= 0 || a.n_heads % a.n_kv || a.ntok < 1 || a.pos < 0 || a.pos + a.ntok > a.max_seq) return -1;
+  if (!gq_flash_takes(a.n_heads, a.n_kv, a.hd) || a.ntok < 1 || a.pos < 0 || a.pos + a.ntok > a.max_seq) return -1;
   const int G = a.n_heads / a.n_kv;
   if (a.hd == 128 && G == 4) return launch_flash<128, 4>(a, n_cu, s);
   if (a.hd == 128 && G == 8) return launch_flash<128, 8>(a, n_cu, s);

@@ -197,6 +197,9 @@ int gq_launch_attention(const AttnArgs &a, hipStream_t s, hipEvent_t mid);
  * or out16, out_stride, pos, ntok, n_heads, n_kv, hd (64 or 128), max_seq
  * and scale are used. */
 int gq_launch_flash_prefill(const AttnArgs &a, int n_cu, hipStream_t s);
+/* the head geometries that it takes: head_dim 64 or 128, 1, 2, 4 or 8 query
+ * heads per KV head */
+bool gq_flash_takes(int n_heads, int n_kv, int hd);
 /* query rows of partial results the launch wants in part_o / part_ml (0:
  * none); without them it does not split the keys */
 size_t gq_flash_parts(int ntok, int pos, int n_heads, int n_kv, int hd, int n_cu);

@@ -1506,6 +1506,7 @@ static PgSeg pg_seg(const gq_ctx *c, int l, int i, const gq_weight &w, float *y)
 static int pf_attention(gq_ctx *c, int layer, int pos, int T, int n_heads, float *q, const float *k, const float *v,
                         float *out, __bf16 *out16, int kparts = 0) {
   const int hd = c->kv_hd, kvd = c->kv_heads * hd, qd = n_heads * hd;
+  if (!gq_flash_takes(n_heads, c->kv_heads, hd)) return -1; /* before q and the cache are written */
   RopeArgs ra{q, k, v, gq_hip_kv_k(c, layer), gq_hip_kv_v(c, layer), c->rope, nullptr, pos,
               n_heads, c->kv_heads, hd, c->kv_max_seq, T, qd, kvd, kvd};
   if (kparts > 0) /* q, k, v are still the q/k/v GEMM's K parts */

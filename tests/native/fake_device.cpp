@@ -159,6 +159,7 @@ size_t gq_mm_tile_bytes(int, int rows, int cols, bool swiglu) { return (size_t)r
 size_t gq_q6k_units_bytes(int rows, int cols) { return (size_t)rows * cols; }
 size_t gq_sample_ws_bytes(int vocab) { return 16 * (size_t)vocab; }
 size_t gq_sample_topk_bytes(int vocab, int k) { return k <= 256 ? 12 * (size_t)vocab : 0; }
+bool gq_flash_takes(int n_heads, int n_kv, int hd) { return (hd == 64 || hd == 128) && n_heads / n_kv <= 8; }
 size_t gq_flash_parts(int ntok, int pos, int n_heads, int, int, int) { return pos ? (size_t)2 * ntok * n_heads : 0; }
 bool gq_matvec_mm_forced() { return false; }
 bool gq_matvec_q6k_ref() { return false; }

@@ -37,6 +37,25 @@ def test_no_device_means_null_context():
         H.Context(0)
 
 
+def test_prompt_attention_rule_for_unsupported_groups():
+    """The workspace rule of the prompt attention (plain host code) for head
+    geometries that no kernel takes: no rows, where it had divided by 16 / G =
+    0 for more than 16 query heads per KV head and ended the process."""
+    import subprocess
+    import sys
+    code = """
+import ctypes, guanaco_amd.hip as H
+f = ctypes.CDLL(H.LIB_PATH)._Z14gq_flash_partsiiiiii  # gq_flash_parts(ntok, pos, n_heads, n_kv, hd, n_cu)
+f.restype = ctypes.c_size_t
+for nh, nkv, hd in ((32, 1, 64), (96, 2, 128), (17, 1, 64), (16, 1, 64), (24, 8, 128), (32, 8, 96), (0, 8, 64)):
+    for ntok, pos in ((1, 0), (37, 8000), (512, 3584)):
+        assert f(ntok, pos, nh, nkv, hd, 256) == 0, (nh, nkv, hd)
+assert f(37, 8000, 32, 8, 128, 256) > 0
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT)
+    assert r.returncode == 0, (r.returncode, r.stderr[-500:])
+
+
 def test_reference_patch_applies_and_builds(tmp_path):
     """The drop-in as a maintainer applies it: guanaco_amd/host/reference-hip.patch
     applies to the reference's src/ tree as it is, and with hip_backend.c /

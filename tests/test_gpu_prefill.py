@@ -414,6 +414,21 @@ def test_prefill_attention_rejects_bad_positions(ctx):
     b.free()
 
 
+@pytest.mark.parametrize("nh,nkv,hd", [(32, 1, 64), (6, 2, 64), (32, 2, 128), (8, 4, 96)])
+def test_prefill_attention_rejects_unsupported_heads(ctx, nh, nkv, hd):
+    """Head geometries that no kernel takes (more than 8 query heads per KV
+    head, 3, or head_dim 96) are refused, and the cache is left as it was."""
+    ctx.kv_init(1, nkv, hd, 64, 500000.0)
+    ctx.kv_prefill_synth(5, 6, 64)
+    before = ctx.kv_read_layer(0)
+    b = ctx.alloc(4 * 40 * nh * hd)
+    for T, pos in ((1, 0), (37, 20)):
+        assert ctx.prefill_attention_dev(0, pos, T, nh, b, b, b, b) == -1
+    for d, e in zip(ctx.kv_read_layer(0), before):
+        assert np.array_equal(bits(d), bits(e))
+    b.free()
+
+
 PF_TOL = 3e-2
 
 
