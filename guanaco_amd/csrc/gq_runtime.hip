@@ -951,6 +951,7 @@ extern "C" int gq_hip_model_bind(gq_ctx *c, const gq_model *m) {
                     (m->embed.dtype != GQ_F32 && m->embed.dtype != GQ_Q8_0 && m->embed.dtype != GQ_Q4_K)))
     return fail(c, -1, "embed: F32, Q8_0 or Q4_K (vocab x hidden)");
   if (has_lm && !m->rms_final) return fail(c, -1, "rms_final");
+  c->bound = c->whole = false; /* until everything below is there */
   free_graph(c);
   pf_release(c); /* sized for the previous model */
   c->m = *m;

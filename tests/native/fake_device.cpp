@@ -22,6 +22,7 @@ struct Block {
 };
 std::map<char *, Block> live; /* device memory */
 size_t used, capacity = (size_t)288 << 30, refuse_from = ~(size_t)0;
+bool refuse_pinned;
 std::map<std::string, long> counts;
 std::string errors;
 
@@ -75,8 +76,9 @@ void take(Owed &o, const char *what, const float *part, int n, size_t floats) {
 
 extern "C" {
 /* what the tests ask for and see */
-void fake_reset(size_t total) { capacity = total, refuse_from = ~(size_t)0, counts.clear(), errors.clear(), owed_qkv = owed_x = Owed(); }
+void fake_reset(size_t total) { capacity = total, refuse_from = ~(size_t)0, refuse_pinned = false, counts.clear(), errors.clear(), owed_qkv = owed_x = Owed(); }
 void fake_refuse_from(size_t bytes) { refuse_from = bytes; } /* allocations of so many bytes and more fail */
+void fake_refuse_pinned(int on) { refuse_pinned = on != 0; }
 const char *fake_errors() { return errors.c_str(); }
 long fake_count(const char *what) { return counts[what]; }
 size_t fake_used() { return used; }
@@ -109,7 +111,7 @@ hipError_t hipFree(void *p) {
 hipError_t hipMemGetInfo(size_t *f, size_t *t) { return *f = capacity - used, *t = capacity, hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
   counts["host_malloc"]++;
-  if (n >= refuse_from) return hipErrorOutOfMemory;
+  if (refuse_pinned) return hipErrorOutOfMemory;
   return (*p = calloc(1, n)) ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }

@@ -5,6 +5,7 @@ follows what the launchers are handed: that workspaces are alive and large
 enough, and that the K-part sums one launch leaves reach the launch that adds
 them.  What the kernels compute is not part of it."""
 import ctypes as C
+import dataclasses
 import os
 import shutil
 import subprocess
@@ -110,3 +111,32 @@ def test_weights_written_in_place(dev, how):
         prompt(dm, 300)
         stale = dev.n("dense") == 8 * SMALL.n_layers and dev.n("dense_tile") == before
         assert stale == (how == "elsewhere")
+
+
+@pytest.mark.parametrize("what", ["pinned", "workspace"])
+def test_failed_bind_leaves_no_model(dev, what):
+    """A bind that fails for memory after it has begun to replace the bound
+    model leaves none: the entry points say so instead of running on buffers
+    that are gone."""
+    with H.Context(0) as ctx:
+        dm = H.DeviceModel(ctx, SMALL, 512)
+        prompt(dm, 40)
+        emb = ctx.alloc(S.qbytes(S.Q8_0, 2000, SMALL.hidden))
+        dm.spec = dataclasses.replace(SMALL, vocab=2000)  # larger results: the pinned memory is made anew
+        dm.model.vocab = 2000
+        dm.model.embed = dm.model.lm_head = H.GqWeight(emb.ptr, S.Q8_0, 2000, SMALL.hidden)
+        if what == "pinned":
+            dev.fake_refuse_pinned(1)
+        else:
+            dev.fake_refuse_from(4 * SMALL.hidden)
+        assert dev.gq_hip_model_bind(ctx.h, C.byref(dm.model)) == -4
+        dev.fake_refuse_pinned(0)
+        dev.fake_refuse_from(1 << 60)
+        whole = C.c_int(9)
+        assert dev.gq_hip_bound_layers(ctx.h, C.byref(whole)) == 0 and whole.value == 0
+        assert dev.gq_hip_forward_token(ctx.h, 1, 0, None, None) == -1
+        with pytest.raises(H.HipError, match="no model bound"):
+            prompt(dm, 40)
+        assert dev.gq_hip_model_bind(ctx.h, C.byref(dm.model)) == 0  # and it can be bound again
+        prompt(dm, 300)
+        assert dev.gq_hip_forward_token(ctx.h, 1, 300, None, None) >= 0
