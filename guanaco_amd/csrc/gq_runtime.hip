@@ -1365,11 +1365,12 @@ static int ensure_tokens(gq_ctx *c, int n) {
   Workspace &w = c->ws;
   n = std::max(n, kStepTokens); /* a captured graph keeps the buffer */
   if (w.tokens_cap >= n) return 0;
-  if (w.d_tokens) gq_hip_free(c, w.d_tokens);
-  w.d_tokens = (int *)dev_alloc(c, sizeof(int) * n);
-  if (!w.d_tokens) return -4;
-  w.tokens_cap = n;
+  int *p = (int *)dev_alloc(c, sizeof(int) * n);
+  if (!p) return -4;
   free_graph(c); /* the graph captured the old pointer */
+  if (w.d_tokens) gq_hip_free(c, w.d_tokens);
+  w.d_tokens = p;
+  w.tokens_cap = n;
   return 0;
 }
 

@@ -48,6 +48,7 @@ struct Owed {
   int n = 0;
 } owed_qkv, owed_x;
 float serial;
+const int *captured_tokens; /* the token log of the captured step */
 
 /* a launch whose sums its caller adds; n parts of tokens x rows */
 void leave(Owed &o, float *part, int n, size_t floats) {
@@ -138,7 +139,11 @@ hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { return *g = (hipGraph_t)&live, hipSuccess; }
 hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t) { return *e = (hipGraphExec_t)&live, hipSuccess; }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return counts["graph"]++, hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) {
+  counts["graph"]++;
+  need("captured token log", captured_tokens, sizeof(int));
+  return hipSuccess;
+}
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t *e) { return *e = (hipEvent_t)&live, hipSuccess; }
@@ -214,7 +219,7 @@ int gq_launch_flash_prefill(const AttnArgs &a, int, hipStream_t) {
 int gq_launch_argmax(const float *x, int n, float *, int, int *out, int *tokens, int *, int *, hipStream_t, int, const void *, int,
                      float *, const ArgmaxHost &h) {
   need("logits", x, sizeof(float) * n);
-  if (tokens) need("token log", tokens, sizeof(int));
+  if (tokens) need("token log", captured_tokens = tokens, sizeof(int));
   if (h.token) *h.token = 3;
   else *out = 3;
   return 0;

@@ -140,3 +140,19 @@ def test_failed_bind_leaves_no_model(dev, what):
         assert dev.gq_hip_model_bind(ctx.h, C.byref(dm.model)) == 0  # and it can be bound again
         prompt(dm, 300)
         assert dev.gq_hip_forward_token(ctx.h, 1, 300, None, None) >= 0
+
+
+def test_refused_token_log(dev):
+    """A decode loop whose token log finds no memory fails, and single steps
+    go on with the log that their captured graph writes."""
+    with H.Context(0) as ctx:
+        dm = H.DeviceModel(ctx, SMALL, 8192)
+        step = lambda: dev.gq_hip_forward_token(ctx.h, 1, 0, None, None)  # noqa: E731
+        assert step() == 3
+        dev.fake_refuse_from(4 * 5000)
+        with pytest.raises(H.HipError):
+            dm.decode_loop(1, 0, 5000)
+        assert step() == 3 and step() == 3
+        dev.fake_refuse_from(1 << 60)
+        dm.decode_loop(1, 0, 5000)
+        assert step() == 3
