@@ -1860,6 +1860,7 @@ extern "C" int gq_hip_attention_dev(gq_ctx *c, int layer, int pos, int n_heads, 
     if (w.part_cap < need_o || w.part_ml_cap < need_ml || !w.part_o) {
       if (w.part_o) gq_hip_free(c, w.part_o);
       if (w.part_ml) gq_hip_free(c, w.part_ml);
+      w.part_cap = w.part_ml_cap = 0;
       w.part_o = (float *)dev_alloc(c, sizeof(float) * need_o);
       w.part_ml = (float *)dev_alloc(c, sizeof(float) * need_ml);
       if (!w.part_o || !w.part_ml) return -4;

@@ -22,6 +22,7 @@ struct Block {
 };
 std::map<char *, Block> live; /* device memory */
 size_t used, capacity = (size_t)288 << 30, refuse_from = ~(size_t)0;
+long refuse_after = -1; /* allocations granted before all are refused; -1: no such limit */
 bool refuse_pinned;
 std::map<std::string, long> counts;
 std::string errors;
@@ -77,8 +78,9 @@ void take(Owed &o, const char *what, const float *part, int n, size_t floats) {
 
 extern "C" {
 /* what the tests ask for and see */
-void fake_reset(size_t total) { capacity = total, refuse_from = ~(size_t)0, refuse_pinned = false, counts.clear(), errors.clear(), owed_qkv = owed_x = Owed(); }
+void fake_reset(size_t total) { capacity = total, refuse_from = ~(size_t)0, refuse_after = -1, refuse_pinned = false, counts.clear(), errors.clear(), owed_qkv = owed_x = Owed(); }
 void fake_refuse_from(size_t bytes) { refuse_from = bytes; } /* allocations of so many bytes and more fail */
+void fake_refuse_after(long n) { refuse_after = n; }
 void fake_refuse_pinned(int on) { refuse_pinned = on != 0; }
 const char *fake_errors() { return errors.c_str(); }
 long fake_count(const char *what) { return counts[what]; }
@@ -87,6 +89,8 @@ size_t fake_used() { return used; }
 /* ---- the HIP runtime ---- */
 hipError_t hipMalloc(void **p, size_t n) {
   counts["malloc"]++;
+  if (refuse_after > 0) refuse_after--;
+  else if (refuse_after == 0) n = ~(size_t)0;
   if (n >= refuse_from || n > capacity - used) {
     counts["refused"]++;
     return hipErrorOutOfMemory;

@@ -49,6 +49,7 @@ def built(tmp_path_factory):
     lib.fake_errors.restype = C.c_char_p
     lib.fake_count.restype, lib.fake_count.argtypes = C.c_long, [C.c_char_p]
     lib.fake_used.restype = C.c_size_t
+    lib.fake_refuse_after.argtypes = [C.c_long]
     lib.fake_reset.argtypes = lib.fake_refuse_from.argtypes = [C.c_size_t]
     return lib
 
@@ -156,3 +157,20 @@ def test_refused_token_log(dev):
         dev.fake_refuse_from(1 << 60)
         dm.decode_loop(1, 0, 5000)
         assert step() == 3
+
+
+@pytest.mark.parametrize("granted", [0, 1])
+def test_refused_attention_partials(dev, granted):
+    """Decode attention without a bound model grows its own partials: when one
+    of the two finds no memory the call fails, and a smaller one afterwards
+    has both again."""
+    with H.Context(0) as ctx:
+        q = ctx.alloc(4 * 8 * 64)
+        ctx.kv_init(1, 2, 64, 64, 500000.0)
+        assert ctx.attention_dev(0, 3, 8, q, q) == 0
+        ctx.kv_init(1, 2, 64, 4096, 500000.0)
+        dev.fake_refuse_after(granted)
+        assert ctx.attention_dev(0, 3, 8, q, q) == -4
+        dev.fake_refuse_after(-1)
+        ctx.kv_init(1, 2, 64, 64, 500000.0)
+        assert ctx.attention_dev(0, 3, 8, q, q) == 0
