@@ -6,9 +6,9 @@
  * once per 128 tokens and weight, about as many vector-ALU cycles as its
  * MFMAs take.  That is right for few tokens, where the quantized bytes are
  * what there is to read; for many tokens the same weights are converted over
- * and over.  gq_hip_model_bind therefore keeps a bf16 copy of the
- * projections beside the quantized ones (2 bytes a weight, the values that
- * pgemm_kernel rounds to) and launches of enough tokens multiply by that.
+ * and over.  The first prompt of enough tokens therefore makes a bf16 copy
+ * of the projections beside the quantized ones (2 bytes a weight, the values
+ * that pgemm_kernel rounds to), and such prompts multiply by that.
  *
  * The copy is laid out as the kernel's LDS tiles: for each 256-row tile and
  * 32-column step one contiguous 16 KB block, row r's four octets (8 weights,

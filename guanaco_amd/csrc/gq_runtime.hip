@@ -56,7 +56,8 @@ struct PrefillWs {
  * 8B shape on the quantized weights: 41.0 ms in chunks of 512, 38.3 in one).
  * The activations are sized for the longest chunk seen, in steps of 512. */
 constexpr int kPrefillChunk = 2048;
-/* chunks of at least this many tokens multiply by the bf16 copies */
+/* chunks of at least this many tokens multiply by the bf16 copies of the
+ * weights (dense_build) */
 constexpr int kDenseTokens = 256;
 /* prompt tokens that gq_ctx::h_in holds: a prompt is embedded in pieces of at
  * most that many */
@@ -106,6 +107,7 @@ struct gq_ctx {
     size_t dn_at[4] = {};
   };
   std::vector<MmLayer> mm;
+  bool dense_short = false; /* no room for the copies when last asked; any free asks again */
   const uint8_t *mm_lm = nullptr;
   Workspace ws;
   PrefillWs pf;
@@ -314,10 +316,12 @@ extern "C" void gq_hip_free(gq_ctx *c, void *p) {
   (void)hipStreamSynchronize(c->stream);
   (void)hipFree(p);
   c->allocs.erase(it);
+  c->dense_short = false;
 }
 
-/* Give the bf16 copies back; false: there are none.  Prompts multiply by the
- * quantized weights from then on, as models without copies do. */
+/* Give the bf16 copies back; false: there are none.  A later prompt of many
+ * tokens makes them again if there is room (dense_build), and multiplies by
+ * the quantized weights if not. */
 static bool dense_drop(gq_ctx *c) {
   bool any = false;
   for (auto &L : c->mm) {
@@ -881,34 +885,6 @@ static void mm_free(gq_ctx *c) {
   rel(c->mm_lm);
 }
 
-static bool pf_gemm_ok(const gq_weight &w);
-
-/* The bf16 copy of layer l's projections for prompts of many tokens; left
- * out (dn NULL) where the GEMM does not take the layer or memory is short. */
-static void dense_build(gq_ctx *c, int l) {
-  const gq_layer &L = c->layers[l];
-  const gq_weight *ws[7] = {&L.wq, &L.wk, &L.wv, &L.wo, &L.w_gate, &L.w_up, &L.w_down};
-  for (const gq_weight *w : ws)
-    if (!pf_gemm_ok(*w)) return;
-  if (L.w_gate.dtype != L.w_up.dtype) return;
-  auto &M = c->mm[l];
-  size_t at[8], n = 0; /* q, k, v, o, gate + up, (up), down */
-  for (int i = 0; i < 7; i++) {
-    at[i] = n;
-    if (i != 5) n += gq_dense_bytes(ws[i]->rows, ws[i]->cols, i == 4);
-  }
-  M.dn = (uint8_t *)dev_alloc(c, n, true);
-  if (!M.dn) return;
-  M.dn_at[0] = 0, M.dn_at[1] = at[3], M.dn_at[2] = at[4], M.dn_at[3] = at[6];
-  for (int i = 0; i < 7; i++)
-    if (i != 5 && gq_launch_dense_tile(M.dn + at[i], ws[i]->dtype, ws[i]->data, i == 4 ? L.w_up.data : nullptr,
-                                       ws[i]->rows, ws[i]->cols, c->stream)) {
-      gq_hip_free(c, M.dn);
-      M.dn = nullptr;
-      return;
-    }
-}
-
 extern "C" int gq_hip_model_bind(gq_ctx *c, const gq_model *m) {
   if (!c || !m || !m->layers) return fail(c, -1, "model_bind: NULL");
   if (!c->kslab) return fail(c, -1, "model_bind: call gq_hip_kv_init first");
@@ -965,6 +941,7 @@ extern "C" int gq_hip_model_bind(gq_ctx *c, const gq_model *m) {
    * the stream after whatever wrote the weights */
   mm_free(c);
   c->mm.resize(m->n_layers);
+  c->dense_short = false;
   for (int l = 0; l < m->n_layers; l++) {
     if (!on[l]) continue;
     const gq_layer &L = c->layers[l];
@@ -993,17 +970,6 @@ extern "C" int gq_hip_model_bind(gq_ctx *c, const gq_model *m) {
       if (d && gq_launch_q6k_units(d, g.data, g.rows, g.cols, c->stream) == 0) c->mm[l].ux[i] = d;
       else if (d) gq_hip_free(c, d);
     }
-  }
-  /* bf16 copies for prompts of many tokens, only while they take less than a
-   * quarter of the memory that is free (2 bytes a weight: 14 GB at the 8B
-   * shape): a program that fills the card keeps the room it had */
-  if (c->whole) {
-    size_t need = 0, fr = 0, tot = 0;
-    for (int l = 0; l < m->n_layers; l++)
-      need += gq_dense_bytes(H, H, false) * 2 + gq_dense_bytes(kvd, H, false) * 2 + gq_dense_bytes(F, H, true) +
-              gq_dense_bytes(H, F, false);
-    if (hipMemGetInfo(&fr, &tot) == hipSuccess && need < fr / 4)
-      for (int l = 0; l < m->n_layers; l++) dense_build(c, l);
   }
   if (has_lm) {
     const gq_weight *lm[1] = {&m->lm_head};
@@ -1495,6 +1461,42 @@ static bool pf_model_ok(const gq_ctx *c) {
   return true;
 }
 
+/* The bf16 copies of the projections (pf_model_ok) for prompts of many
+ * tokens, made by the first such prompt: 2 bytes a weight, 14 GB at the 8B
+ * shape, where they take 8.4 ms once and a 1500-token prompt gains 10 (made at
+ * bind, programs that only decode paid 8 of its 26 ms and the memory).  Only
+ * while they take less than a quarter of the memory that is free: a program
+ * that fills the card keeps the room it had.  All of them or none. */
+static void dense_build(gq_ctx *c) {
+  size_t at[8], need = 0, fr = 0, tot = 0; /* q, k, v, o, gate + up, (up), down */
+  if (c->dense_short || c->layers.empty() || c->mm.size() != c->layers.size() || c->mm[0].dn) return;
+  const gq_layer &L0 = c->layers[0];
+  const gq_weight *shape[7] = {&L0.wq, &L0.wk, &L0.wv, &L0.wo, &L0.w_gate, &L0.w_up, &L0.w_down};
+  for (int i = 0; i < 7; i++) {
+    at[i] = need;
+    if (i != 5) need += gq_dense_bytes(shape[i]->rows, shape[i]->cols, i == 4);
+  }
+  c->dense_short = hipMemGetInfo(&fr, &tot) != hipSuccess || need * c->layers.size() >= fr / 4;
+  if (c->dense_short) return;
+  for (size_t l = 0; l < c->layers.size(); l++) {
+    const gq_layer &L = c->layers[l];
+    const gq_weight *ws[7] = {&L.wq, &L.wk, &L.wv, &L.wo, &L.w_gate, &L.w_up, &L.w_down};
+    auto &M = c->mm[l];
+    M.dn = (uint8_t *)dev_alloc(c, need, true);
+    M.dn_at[0] = 0, M.dn_at[1] = at[3], M.dn_at[2] = at[4], M.dn_at[3] = at[6];
+    bool ok = M.dn != nullptr;
+    for (int i = 0; i < 7 && ok; i++)
+      if (i != 5)
+        ok = gq_launch_dense_tile(M.dn + at[i], ws[i]->dtype, ws[i]->data, i == 4 ? L.w_up.data : nullptr, ws[i]->rows,
+                                  ws[i]->cols, c->stream) == 0;
+    if (!ok) {
+      (void)dense_drop(c);
+      c->dense_short = true;
+      return;
+    }
+  }
+}
+
 /* weight i (wq, wk, wv, wo, gate, up, down) of layer l as a GEMM segment:
  * its unit-layout copy where model bind made one */
 static PgSeg pg_seg(const gq_ctx *c, int l, int i, const gq_weight &w, float *y) {
@@ -1610,6 +1612,7 @@ extern "C" int gq_hip_prefill(gq_ctx *c, const int32_t *tokens, int n_tokens, in
     chunk = chunks(512);
     if ((rc = pf_alloc(c, chunk))) return rc;
   }
+  if (gemm && chunk >= kDenseTokens && !gq_matvec_q6k_ref()) dense_build(c);
   /* for every launch of a chunk, or for o and down alone, or none: the
    * launches do with what there is */
   if (gemm && pf_parts(c, chunk, m.hidden + 2 * (size_t)m.n_kv_heads * m.head_dim)) (void)pf_parts(c, chunk, m.hidden);

@@ -617,8 +617,8 @@ def test_prefill_model_rejects_bad_input(ctx):
 @pytest.mark.parametrize("T", [256, 257, 511, 700])
 @pytest.mark.parametrize("mix", ["q4_k_m", "q8_0"])
 def test_prefill_dense_copy_vs_quantized(orc, T, mix):
-    """Chunks of 256 tokens and more multiply by the bf16 copies of the
-    weights that model bind makes; matvec path 3 dequantizes the same weights
+    """Chunks of 256 tokens and more multiply by bf16 copies of the weights,
+    made by the first such prompt; matvec path 3 dequantizes the same weights
     as it multiplies.  Layer 0's V rows are that GEMM's own output: the same
     products in another order (1e-5).  After it the bf16 activations may round
     apart: 2e-3, as between the layouts above.  128-row K and V segments (half
@@ -646,10 +646,9 @@ def test_prefill_dense_copy_vs_quantized(orc, T, mix):
         c.close()
 
 
-def test_prefill_dense_copy_given_back(orc):
-    """An allocation that the card has no room for takes the bf16 copies back
-    before it fails; prompts then multiply by the quantized weights, bit for
-    bit as on the layouts that have no copy."""
+def test_prefill_dense_copy_after_a_failed_allocation(orc):
+    """An allocation that the card has no room for changes no prompt's bits:
+    copies that it took back before it failed are made again."""
     import guanaco_amd.hip as H
     spec = S.ModelSpec("dense-back", n_layers=2, hidden=512, ff=1536, n_heads=8, n_kv_heads=2, vocab=1000,
                        layer_dtypes=dict(wv=S.Q6_K, wd=S.Q6_K), q4k_zero_mean=True, norm_shift=4)
@@ -663,7 +662,7 @@ def test_prefill_dense_copy_given_back(orc):
         with pytest.raises(H.HipError):
             c.alloc(1 << 46)
         after = dm.prefill(toks, 0)[1]
-        assert np.array_equal(bits(after), bits(ref)) and rel_l2(with_copy, ref) < 2e-3
+        assert np.array_equal(bits(after), bits(with_copy)) and rel_l2(with_copy, ref) < 2e-3
     finally:
         c.close()
 

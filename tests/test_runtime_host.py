@@ -174,3 +174,53 @@ def test_refused_attention_partials(dev, granted):
         dev.fake_refuse_after(-1)
         ctx.kv_init(1, 2, 64, 64, 500000.0)
         assert ctx.attention_dev(0, 3, 8, q, q) == 0
+
+
+def copies(spec):
+    """bytes of the bf16 copies as the stand-in lays them out"""
+    per = sum(2 * np.prod(spec.shape(k)) for k in ("wq", "wk", "wv", "wo", "wd")) + 4 * np.prod(spec.shape("wg"))
+    return int(per) * spec.n_layers
+
+
+def test_copies_are_made_by_the_first_long_prompt(dev):
+    """The bf16 copies of the weights cost time and 2 bytes a weight, so only a
+    prompt that uses them makes them: not a bind, a step, a short prompt, or
+    any prompt in the mode that runs token by token."""
+    with H.Context(0) as ctx:
+        dm = H.DeviceModel(ctx, SMALL, 4096)
+        dm.forward(1, 0)
+        prompt(dm, 200)
+        assert dev.gq_hip_set_prefill_mode(ctx.h, 1) == 0
+        prompt(dm, 600)
+        assert dev.n("dense_tile") == 0
+        assert dev.gq_hip_set_prefill_mode(ctx.h, 0) == 1
+        used = dev.fake_used()
+        prompt(dm, 300)
+        made = dev.n("dense_tile")
+        assert made == 6 * SMALL.n_layers and dev.fake_used() >= used + copies(SMALL)
+        prompt(dm, 3000)  # once
+        assert dev.n("dense_tile") == made and dev.n("dense") == 4 * SMALL.n_layers * 3
+
+
+def test_copies_only_where_there_is_room(dev):
+    """A card of which the copies would take a quarter or more of what is free
+    runs prompts without them, and asks again once something is given back."""
+    dev.fake_reset(GB)
+    with H.Context(0) as ctx:
+        dm = H.DeviceModel(ctx, SMALL, 512)
+        prompt(dm, 200)  # the activations
+        held = ctx.alloc(GB - 256 - dev.fake_used() - 4 * copies(SMALL))
+        prompt(dm, 300)
+        prompt(dm, 300)
+        assert dev.n("dense") == dev.n("dense_tile") == 0
+        held.free()
+        prompt(dm, 300)
+        assert dev.n("dense") == 4 * SMALL.n_layers
+        # not even a layer's copy can be had: all go, and nothing is asked for
+        # again until something is given back
+        dev.gq_hip_model_bind(ctx.h, C.byref(dm.model))
+        dev.fake_refuse_from(copies(SMALL) // SMALL.n_layers)
+        prompt(dm, 300)
+        n = dev.n("refused")
+        prompt(dm, 300)
+        assert n > 0 and dev.n("dense") == 4 * SMALL.n_layers and dev.n("refused") == n
