@@ -104,7 +104,7 @@ struct gq_ctx {
      * allocation: q | k | v, o, gate + up, down; NULL: the quantized weights
      * serve every prompt */
     uint8_t *dn = nullptr;
-    size_t dn_at[4] = {};
+    size_t dn_at[4] = {}, dn_bytes = 0;
   };
   std::vector<MmLayer> mm;
   bool dense_short = false; /* no room for the copies when last asked; any free asks again */
@@ -288,12 +288,17 @@ extern "C" int gq_hip_device_info(gq_ctx *c, int *n_cu, char *name, int name_len
 
 /* ------------------------------------------------------------ memory */
 static bool dense_drop(gq_ctx *c);
-/* keep_copies: fail rather than take back the bf16 copies of the weights,
- * which prompts can do without */
-static void *dev_alloc(gq_ctx *c, size_t bytes, bool keep_copies = false) {
+static size_t dense_held(const gq_ctx *c);
+/* A request that finds no room takes back the bf16 copies of the weights,
+ * which prompts can do without, if it fits then.  optional: the caller can do
+ * without too; the copies stay. */
+static void *dev_alloc(gq_ctx *c, size_t bytes, bool optional = false) {
   void *p = nullptr;
   hipError_t e = hipMalloc(&p, bytes + kPad);
-  if (e != hipSuccess && !keep_copies && dense_drop(c)) e = hipMalloc(&p, bytes + kPad);
+  if (e != hipSuccess && !optional && dense_held(c)) {
+    size_t fr = 0, tot = 0;
+    if (hipMemGetInfo(&fr, &tot) == hipSuccess && bytes <= fr + dense_held(c) && dense_drop(c)) e = hipMalloc(&p, bytes + kPad);
+  }
   if (e != hipSuccess) {
     (void)hipGetLastError(); /* not for the next launch's check: a caller may go on without */
     fail(c, -4, "hipMalloc(%zu) failed", bytes + kPad);
@@ -322,6 +327,9 @@ extern "C" void gq_hip_free(gq_ctx *c, void *p) {
 /* Give the bf16 copies back; false: there are none.  A later prompt of many
  * tokens makes them again if there is room (dense_build), and multiplies by
  * the quantized weights if not. */
+static size_t dense_held(const gq_ctx *c) {
+  return c->mm.empty() || !c->mm[0].dn ? 0 : c->mm.size() * c->mm[0].dn_bytes;
+}
 static bool dense_drop(gq_ctx *c) {
   bool any = false;
   for (auto &L : c->mm) {
@@ -1401,11 +1409,11 @@ extern "C" int gq_hip_decode_loop(gq_ctx *c, int token, int pos, int n_steps, in
  * cores, RoPE + append of every token of the chunk, then causal attention
  * (token t sees positions 0 .. pos + t). */
 template <class T>
-static int pf_ensure(gq_ctx *c, T *&p, size_t &cap, size_t n) {
+static int pf_ensure(gq_ctx *c, T *&p, size_t &cap, size_t n, bool optional = false) {
   if (cap >= n && p) return 0;
   if (p) gq_hip_free(c, p);
   cap = 0;
-  p = (T *)dev_alloc(c, sizeof(T) * n);
+  p = (T *)dev_alloc(c, sizeof(T) * n, optional);
   if (!p) return -4;
   cap = n;
   return 0;
@@ -1423,7 +1431,7 @@ static void pf_release(gq_ctx *c) {
   w.cap = w.H = w.F = w.kvd = 0;
 }
 
-static int pf_alloc(gq_ctx *c, int tokens) {
+static int pf_alloc(gq_ctx *c, int tokens, bool optional = false) {
   PrefillWs &w = c->pf;
   const gq_model &m = c->m;
   const int kvd_m = m.n_kv_heads * m.head_dim;
@@ -1434,11 +1442,11 @@ static int pf_alloc(gq_ctx *c, int tokens) {
   float **f32[4] = {&w.x, &w.q, &w.k, &w.v};
   const size_t nf[4] = {T * H, T * H, T * kvd, T * kvd};
   for (int i = 0; i < 4; i++)
-    if (!(*f32[i] = (float *)dev_alloc(c, sizeof(float) * nf[i]))) return -4;
+    if (!(*f32[i] = (float *)dev_alloc(c, sizeof(float) * nf[i], optional))) return -4;
   __bf16 **b16[3] = {&w.xn, &w.att, &w.act};
   const size_t nb[3] = {T * H, T * H, T * F};
   for (int i = 0; i < 3; i++)
-    if (!(*b16[i] = (__bf16 *)dev_alloc(c, sizeof(__bf16) * nb[i]))) return -4;
+    if (!(*b16[i] = (__bf16 *)dev_alloc(c, sizeof(__bf16) * nb[i], optional))) return -4;
   w.cap = tokens;
   w.H = m.hidden, w.F = m.ff, w.kvd = kvd_m;
   return 0;
@@ -1483,7 +1491,7 @@ static void dense_build(gq_ctx *c) {
     const gq_weight *ws[7] = {&L.wq, &L.wk, &L.wv, &L.wo, &L.w_gate, &L.w_up, &L.w_down};
     auto &M = c->mm[l];
     M.dn = (uint8_t *)dev_alloc(c, need, true);
-    M.dn_at[0] = 0, M.dn_at[1] = at[3], M.dn_at[2] = at[4], M.dn_at[3] = at[6];
+    M.dn_bytes = need, M.dn_at[0] = 0, M.dn_at[1] = at[3], M.dn_at[2] = at[4], M.dn_at[3] = at[6];
     bool ok = M.dn != nullptr;
     for (int i = 0; i < 7 && ok; i++)
       if (i != 5)
@@ -1524,7 +1532,7 @@ static int pf_attention(gq_ctx *c, int layer, int pos, int T, int n_heads, float
   aa.scale = 1.0f / sqrtf((float)hd);
   PrefillWs &w = c->pf;
   if (const size_t rows = gq_flash_parts(T, pos, n_heads, c->kv_heads, hd, c->n_cu))
-    if (pf_ensure(c, w.fs, w.fs_cap, rows * (hd + 2)) == 0) aa.part_o = w.fs, aa.part_ml = w.fs + rows * hd;
+    if (pf_ensure(c, w.fs, w.fs_cap, rows * (hd + 2), true) == 0) aa.part_o = w.fs, aa.part_ml = w.fs + rows * hd;
   return gq_launch_flash_prefill(aa, c->n_cu, c->stream);
 }
 
@@ -1532,7 +1540,7 @@ static int pf_attention(gq_ctx *c, int layer, int pos, int T, int n_heads, float
  * prompt asks for it before its first layer: a request in between could free
  * sums that a launch has left to the next. */
 static int pf_parts(gq_ctx *c, int T, size_t rows) {
-  return pf_ensure(c, c->pf.part, c->pf.part_cap, gq_parts_tokens(T) * rows);
+  return pf_ensure(c, c->pf.part, c->pf.part_cap, gq_parts_tokens(T) * rows, true);
 }
 
 /* One layer over the chunk (engine.c:352-554 with T tokens): 4 launches of
@@ -1608,7 +1616,7 @@ extern "C" int gq_hip_prefill(gq_ctx *c, const int32_t *tokens, int n_tokens, in
     return (n_tokens + n - 1) / n;
   };
   int chunk = chunks(kPrefillChunk);
-  if (gemm && (rc = pf_alloc(c, chunk))) {
+  if (gemm && (rc = pf_alloc(c, chunk, true))) {
     chunk = chunks(512);
     if ((rc = pf_alloc(c, chunk))) return rc;
   }
@@ -1921,7 +1929,7 @@ static int sample_ensure(gq_ctx *c, int vocab, bool big, int top_k) {
   SampleWs &w = c->sw;
   if (ensure_pinned(c, 0)) return -4;
   if (const size_t tb = top_k > 0 ? gq_sample_topk_bytes(vocab, top_k) : 0; tb && w.topk_cap < vocab) {
-    void *p = dev_alloc(c, tb);
+    void *p = dev_alloc(c, tb, true);
     if (p) { /* without it the one-workgroup replay runs */
       if (w.topk) gq_hip_free(c, w.topk);
       w.topk = p, w.topk_cap = vocab;
@@ -2033,7 +2041,7 @@ extern "C" int gq_hip_chat_turn(gq_ctx *c, const int32_t *tokens, int n_tokens, 
  * matvec path 3 keeps the reference layout.  Freed by the caller. */
 static const uint8_t *op_units(gq_ctx *c, int dtype, const void *w, int rows, int cols) {
   if (dtype != GQ_Q6_K || cols % 2048 || gq_matvec_q6k_ref()) return nullptr;
-  uint8_t *d = (uint8_t *)dev_alloc(c, gq_q6k_units_bytes(rows, cols));
+  uint8_t *d = (uint8_t *)dev_alloc(c, gq_q6k_units_bytes(rows, cols), true);
   if (d && gq_launch_q6k_units(d, w, rows, cols, c->stream)) {
     gq_hip_free(c, d);
     return nullptr;

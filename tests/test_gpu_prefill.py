@@ -647,8 +647,8 @@ def test_prefill_dense_copy_vs_quantized(orc, T, mix):
 
 
 def test_prefill_dense_copy_after_a_failed_allocation(orc):
-    """An allocation that the card has no room for changes no prompt's bits:
-    copies that it took back before it failed are made again."""
+    """An allocation that the card could not hold even without the bf16 copies
+    leaves them, and the bits of later prompts, as they were."""
     import guanaco_amd.hip as H
     spec = S.ModelSpec("dense-back", n_layers=2, hidden=512, ff=1536, n_heads=8, n_kv_heads=2, vocab=1000,
                        layer_dtypes=dict(wv=S.Q6_K, wd=S.Q6_K), q4k_zero_mean=True, norm_shift=4)

@@ -224,3 +224,41 @@ def test_copies_only_where_there_is_room(dev):
         n = dev.n("refused")
         prompt(dm, 300)
         assert n > 0 and dev.n("dense") == 4 * SMALL.n_layers and dev.n("refused") == n
+
+
+def test_what_takes_the_copies_back(dev):
+    """A request that needs their room takes the copies back; one that could
+    not be met even so, or that its caller can do without (K parts, the
+    attention's key parts, the sampler's lists, a longer chunk), does not."""
+    dev.fake_reset(GB)
+    with H.Context(0) as ctx:
+        dm = H.DeviceModel(ctx, SMALL, 8192)
+        x = ctx.alloc(4 * 200000)
+        prompt(dm, 300)
+        made = dev.n("dense_tile")
+        assert made == 6 * SMALL.n_layers
+
+        def fill(rest):
+            return ctx.alloc(GB - 256 - dev.fake_used() - rest)
+
+        def kept():
+            n = dev.n("dense")
+            prompt(dm, 300)
+            return dev.n("dense") == n + 4 * SMALL.n_layers and dev.n("dense_tile") == made
+
+        with pytest.raises(H.HipError):
+            ctx.alloc(GB)
+        assert kept()
+        held = fill(1 << 20)
+        n = dev.n("refused")
+        chunks = dev.n("chunk")
+        prompt(dm, 4000, 4000)  # two chunks of 2000, or in 512 tokens at most
+        assert dev.n("refused") > n and dev.n("chunk") == chunks + 8
+        n = dev.n("refused")
+        assert dev.gq_hip_sample_dev(ctx.h, x.ptr, 200000, 1.0, 40, 1.0, 7) == 5
+        assert dev.n("refused") > n and dev.n("topk_replay") == 1
+        assert kept()
+        more = ctx.alloc(copies(SMALL) // 2)  # fits where the copies were
+        assert not kept() and dev.n("dense_tile") == made
+        more.free()
+        held.free()
