@@ -107,6 +107,7 @@ struct gq_ctx {
     size_t dn_at[4] = {}, dn_bytes = 0;
   };
   std::vector<MmLayer> mm;
+  bool dense_off = false;   /* gq_hip_set_prefill_copies */
   bool dense_short = false; /* no room for the copies when last asked; any free asks again */
   const uint8_t *mm_lm = nullptr;
   Workspace ws;
@@ -1477,7 +1478,7 @@ static bool pf_model_ok(const gq_ctx *c) {
  * that fills the card keeps the room it had.  All of them or none. */
 static void dense_build(gq_ctx *c) {
   size_t at[8], need = 0, fr = 0, tot = 0; /* q, k, v, o, gate + up, (up), down */
-  if (c->dense_short || c->layers.empty() || c->mm.size() != c->layers.size() || c->mm[0].dn) return;
+  if (c->dense_off || c->dense_short || c->layers.empty() || c->mm.size() != c->layers.size() || c->mm[0].dn) return;
   const gq_layer &L0 = c->layers[0];
   const gq_weight *shape[7] = {&L0.wq, &L0.wk, &L0.wv, &L0.wo, &L0.w_gate, &L0.w_up, &L0.w_down};
   for (int i = 0; i < 7; i++) {
@@ -1696,6 +1697,16 @@ extern "C" int gq_hip_set_prefill_mode(gq_ctx *c, int mode) {
   c->prefill_mode = mode;
   return prev;
 }
+
+extern "C" int gq_hip_set_prefill_copies(gq_ctx *c, int on) {
+  if (!c || (on != 0 && on != 1)) return -1;
+  const int prev = !c->dense_off;
+  c->dense_off = !on;
+  if (!on) (void)dense_drop(c);
+  return prev;
+}
+
+extern "C" size_t gq_hip_prefill_copy_bytes(gq_ctx *c) { return c ? dense_held(c) : 0; }
 
 /* ------------------------------------------------------------ measurement */
 extern "C" int gq_hip_profile_step(gq_ctx *c, int token, int pos, double ms[GQ_NCLASS],

@@ -69,6 +69,8 @@ def _load():
         "gq_hip_model_bind": (C.c_int, [_vp, _vp]),
         "gq_hip_bound_layers": (C.c_int, [_vp, _vp]),
         "gq_hip_set_prefill_mode": (C.c_int, [_vp, C.c_int]),
+        "gq_hip_set_prefill_copies": (C.c_int, [_vp, C.c_int]),
+        "gq_hip_prefill_copy_bytes": (C.c_size_t, [_vp]),
         "gq_hip_decode_layer_dev": (C.c_int, [_vp, C.c_int, C.c_int, _vp]),
         "gq_hip_transformer_layer": (C.c_int, [_vp, C.c_int, C.c_int, _fp, _fp, _fp, C.c_int]),
         "gq_hip_forward_token": (C.c_int, [_vp, C.c_int, C.c_int, _fp, _fp]),

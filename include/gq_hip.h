@@ -186,7 +186,13 @@ typedef struct {
  * transformer_layer, qkv_rope) then serve the bound layers; the
  * whole-model ones (forward_token, forward_sample, decode_loop, prefill,
  * chat_turn, profile_step, time_op) need every layer, the embedding and the
- * LM head on the device and return -1 otherwise. */
+ * LM head on the device and return -1 otherwise.
+ * Bind keeps re-ordered copies of gate and up, of the LM head and of Q6_K
+ * projections (3.4 GB at the 8B shape in the Q4_K_M mix, none for Q8_0), and
+ * prompts add bf16 ones (gq_hip_set_prefill_copies): a bound weight that is
+ * written again takes another bind, unless its model is all Q8_0 and the write
+ * goes through this context (gq_hip_h2d, gq_hip_copy_dev,
+ * gq_hip_synth_quant). */
 int gq_hip_model_bind(gq_ctx *ctx, const gq_model *m);
 /* Layers the bound model holds on the device (0 when none is bound); *whole
  * (may be NULL) is 1 when the whole-model entry points can run.  No
@@ -386,6 +392,20 @@ int gq_hip_prefill(gq_ctx *ctx, const int32_t *tokens, int n_tokens, int pos, fl
  * reference has no prompt GEMM (linear_dispatch loops over tokens,
  * engine.c:119-152). */
 int gq_hip_set_prefill_mode(gq_ctx *ctx, int mode);
+/* Prompts of more than a few hundred tokens multiply by bf16 copies of the
+ * projections, which the first such prompt after gq_hip_model_bind makes: 2
+ * bytes a weight (14 GB and 8 ms at the 8B shape), kept until the next bind,
+ * and only where they take less than a quarter of the memory then free.  An
+ * allocation through the context that needs their room takes them back, as
+ * does a write through it to a bound weight; the next such prompt makes them
+ * again if there is room.  Other contexts and libraries of the process cannot
+ * take them back.  on = 0 gives them back now and makes no more (prompts then
+ * dequantize as they multiply: the same products summed in another order), 1
+ * (default) allows them.  Returns the previous setting, or -1.  No reference
+ * counterpart. */
+int gq_hip_set_prefill_copies(gq_ctx *ctx, int on);
+/* Bytes that they take on this context (0: there are none). */
+size_t gq_hip_prefill_copy_bytes(gq_ctx *ctx);
 /* Device-to-device copy by a plain streaming kernel (bytes and both pointers
  * multiples of 16), asynchronous.  No reference counterpart: the known-size
  * workload that scales the HBM byte counters of the profiles. */

@@ -262,3 +262,26 @@ def test_what_takes_the_copies_back(dev):
         assert not kept() and dev.n("dense_tile") == made
         more.free()
         held.free()
+
+
+def test_copies_switched_off_and_on(dev):
+    """gq_hip_set_prefill_copies(0) gives the copies back and makes no more; 1
+    allows them again; the setting outlives a bind."""
+    with H.Context(0) as ctx:
+        dm = H.DeviceModel(ctx, SMALL, 512)
+        for bad in (-1, 2):
+            assert dev.gq_hip_set_prefill_copies(ctx.h, bad) == -1
+        assert dev.gq_hip_prefill_copy_bytes(ctx.h) == 0
+        prompt(dm, 300)
+        assert dev.gq_hip_prefill_copy_bytes(ctx.h) == copies(SMALL)
+        used = dev.fake_used()
+        assert dev.gq_hip_set_prefill_copies(ctx.h, 0) == 1
+        assert dev.gq_hip_prefill_copy_bytes(ctx.h) == 0 and dev.fake_used() <= used - copies(SMALL)
+        n = dev.n("dense")
+        prompt(dm, 300)
+        dev.gq_hip_model_bind(ctx.h, C.byref(dm.model))
+        prompt(dm, 300)
+        assert dev.n("dense") == n
+        assert dev.gq_hip_set_prefill_copies(ctx.h, 1) == 0
+        prompt(dm, 300)
+        assert dev.n("dense") == n + 4 * SMALL.n_layers and dev.gq_hip_prefill_copy_bytes(ctx.h) == copies(SMALL)
