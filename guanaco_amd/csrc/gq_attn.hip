@@ -593,13 +593,19 @@ constexpr int kFsKeys = 64, kFsRows = 128, kFsThreads = 512;
 
 /* The launch for ntok tokens at pos: the fp32 kernel (split 0), or the
  * split-bf16 kernel with its keys in so many parts, whichever should take
- * less.  Microseconds from measured launches at head_dim 128 (at 64 half of
- * them): the fp32 kernel 2.8 per 64 keys when its 16-row workgroups fill the
- * chip twice over, down to 1.5 when they leave it nearly empty; the other 6.2
- * per block of 64 keys and workgroup, 4 at its ends, and 5 more plus the
- * parts' way through memory where it splits the keys.  Measured over sixteen
- * launches (head_dim 64 and 128, 37 to 2048 tokens at 0 to 8000): within 8% of
- * the best choice for each. */
+ * less.  A 64-key block takes a workgroup of the fp32 kernel longer the more of
+ * them share a CU; one CU runs one of the other kernel at a time, and its
+ * partial O cross memory where the keys are split.  The tiles of a causal
+ * prompt are of all lengths and fill each other's rounds, but for what the
+ * last round leaves idle.
+ *
+ * The constants, microseconds, are fitted to 4410 launches timed with every
+ * choice (fifteen head geometries at head_dim 64 and 128, 8 to 2048 tokens at 0
+ * to 7500): the rule's choices take 0.7% more than the best ones, 11% more for
+ * the worst in a hundred, and at most 6% more than the fp32 kernel.  The rule
+ * before it (half the time at head_dim 64, causal tiles that fill every round)
+ * took 75 of them to a slower kernel: 900 tokens of 8 heads at 0, head_dim 128,
+ * 61 us in five parts against 48. */
 struct FlashShape {
   int split, wgs;
 };
@@ -607,15 +613,21 @@ constexpr int kFsMaxSplit = 8;
 FlashShape flash_shape(int ntok, int pos, int n_heads, int n_kv, int hd, int n_cu, bool parts) {
   const int G = n_heads / n_kv, tpt = kFsRows / G, wgs = (ntok + tpt - 1) / tpt * n_kv;
   const int nblk = (pos + ntok - 1) / kFsKeys + 1; /* the longest tile's */
-  const double mean = (pos + 0.5 * ntok) / kFsKeys + 1, even = (double)pos / (pos + ntok);
-  /* tiles of one length run in whole rounds, causal ones fill each other's */
-  auto blocks = [&](double r) { return r <= 1 ? nblk : even * std::ceil(r) * nblk + (1 - even) * r * mean; };
-  const double narrow = (double)((ntok + 16 / G - 1) / (16 / G)) * n_kv / (2 * n_cu), scale = hd / 128.0;
-  double best = scale * blocks(narrow) * (1.5 + 1.3 * std::min(1.0, narrow));
+  const double mean = (pos + 0.5 * ntok) / kFsKeys + 1;
+  const double even = (double)pos / (pos + ntok), causal = 1 - even; /* how far the tiles are of one length, and not */
+  const bool wide = hd > 64;
+  const double w = (double)((ntok + 16 / G - 1) / (16 / G)) * n_kv / n_cu; /* fp32 workgroups a CU */
+  const double few = w <= 1 ? (wide ? 1.35 : 1.2) : (wide ? 2.45 : 1.6), many = wide ? 1.38 : 0.84;
+  double best = w <= 2 ? few * nblk
+                       : even * (nblk + mean) / 2 * many * std::max(w, std::min(std::ceil(w), 3.0)) +
+                             causal * std::max(few * nblk, 1.25 * many * w * mean);
   FlashShape f{0, wgs};
   for (int k = 1; k == 1 || (parts && k <= kFsMaxSplit && nblk / k >= 2); k++) {
-    const double us = scale * blocks((double)wgs * k / n_cu) / k * 6.2 + 4.0 +
-                      (k > 1 ? 5.0 + 8.0 * k * ntok * n_heads * hd / 4.0e6 : 0.0);
+    const double r = (double)wgs * k / n_cu;
+    const double blocks =
+        r <= 1 ? nblk : std::max((double)nblk, even * std::ceil(r) * mean + causal * (r * mean + 0.3 * nblk));
+    const double us = (wide ? 6.06 : 3.72) * blocks / k + (r > 1 ? 3.7 * causal : 0.0) +
+                      (k > 1 ? 4.4 + 12.5 * k * ntok * n_heads * hd / 4.0e6 : 0.0);
     if (us < best) best = us, f.split = k;
   }
   return f;

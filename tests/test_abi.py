@@ -56,6 +56,20 @@ assert f(37, 8000, 32, 8, 128, 256) > 0
     assert r.returncode == 0, (r.returncode, r.stderr[-500:])
 
 
+@pytest.mark.parametrize("ntok,pos,nh,nkv,hd,split", [
+    (900, 0, 8, 8, 128, 0), (768, 0, 8, 8, 128, 0), (900, 300, 8, 8, 128, 4), (768, 0, 8, 1, 128, 0), (900, 0, 8, 4, 128, 0),
+    (512, 3584, 32, 8, 128, 2), (128, 2000, 32, 8, 128, 8), (37, 8000, 32, 8, 128, 8), (77, 301, 32, 4, 64, 0),
+])
+def test_prompt_attention_rule(ntok, pos, nh, nkv, hd, split):
+    """Parts of the keys (0: one part, or the fp32 kernel) at launches that were
+    timed with every choice, at 256 CUs.  The first five had gone to five or six
+    parts, 1.2 to 1.25 times as slow."""
+    import guanaco_amd.hip as H
+    f = ctypes.CDLL(H.LIB_PATH)._Z14gq_flash_partsiiiiii  # gq_flash_parts(ntok, pos, n_heads, n_kv, hd, n_cu)
+    f.restype = ctypes.c_size_t
+    assert f(ntok, pos, nh, nkv, hd, 256) == split * ntok * nh
+
+
 def test_reference_patch_applies_and_builds(tmp_path):
     """The drop-in as a maintainer applies it: guanaco_amd/host/reference-hip.patch
     applies to the reference's src/ tree as it is, and with hip_backend.c /
