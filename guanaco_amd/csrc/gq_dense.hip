@@ -20,8 +20,7 @@
  * Measured at the 8B shape, us per layer (quantized kernels / here): 512
  * tokens: q/k/v 50 / 45, o 33 / 31, gate + up 151 / 132, down 96 / 73; 1500
  * tokens in one chunk: 152 / 118, 103 / 72, 441 / 390, 344 / 204.  A
- * 1500-token prompt 38.3 -> 32.1 ms (40.8 in chunks of 512 before).  256
- * tokens come out even, so that is where the launches change over.  At the
+ * 1500-token prompt 38.3 -> 32.1 ms (40.8 in chunks of 512 before).  At the
  * best shapes 0.95-1.1 PFLOP/s of the 1.45 that a large library product
  * reaches on the card: with the DMA left out the loop runs at 1.16.
  */

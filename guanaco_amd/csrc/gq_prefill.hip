@@ -31,7 +31,7 @@
  *
  * Launches of up to 64 tokens take two (or four) row waves x four K splits
  * a workgroup and up to eight K parts over the grid (launch_flat).  Chunks of
- * 256 tokens and more of a bound model multiply by bf16 copies of the weights
+ * more than 256 tokens of a bound model multiply by bf16 copies of the weights
  * instead (gq_dense.hip).
  *
  * The fused Q4_K gate/up launch runs a wide variant of the tile when its grid

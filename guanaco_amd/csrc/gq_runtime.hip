@@ -56,9 +56,13 @@ struct PrefillWs {
  * 8B shape on the quantized weights: 41.0 ms in chunks of 512, 38.3 in one).
  * The activations are sized for the longest chunk seen, in steps of 512. */
 constexpr int kPrefillChunk = 2048;
-/* chunks of at least this many tokens multiply by the bf16 copies of the
- * weights (dense_build) */
-constexpr int kDenseTokens = 256;
+/* Chunks of at least this many tokens multiply by the bf16 copies of the
+ * weights (dense_build): one more than two of the dequantizing GEMM's
+ * 128-token tiles.  Whole prompts over two layers, quantized / copies, us: 8B
+ * shape 256 tokens 641 / 666, 257 770 / 716, 384 828 / 788, 512 920 / 833;
+ * 1.1B Q4_K_M 296 / 315, 347 / 309, 367 / 333, 389 / 356; 1.1B Q8_0 304 / 312,
+ * 337 / 307, 365 / 335, 395 / 375. */
+constexpr int kDenseTokens = 257;
 /* prompt tokens that gq_ctx::h_in holds: a prompt is embedded in pieces of at
  * most that many */
 constexpr int kPinnedTokens = 4 * kPrefillChunk;

@@ -617,12 +617,13 @@ def test_prefill_model_rejects_bad_input(ctx):
 @pytest.mark.parametrize("T", [256, 257, 511, 700])
 @pytest.mark.parametrize("mix", ["q4_k_m", "q8_0"])
 def test_prefill_dense_copy_vs_quantized(orc, T, mix):
-    """Chunks of 256 tokens and more multiply by bf16 copies of the weights,
+    """Chunks of more than 256 tokens multiply by bf16 copies of the weights,
     made by the first such prompt; matvec path 3 dequantizes the same weights
-    as it multiplies.  Layer 0's V rows are that GEMM's own output: the same
-    products in another order (1e-5).  After it the bf16 activations may round
-    apart: 2e-3, as between the layouts above.  128-row K and V segments (half
-    a tile), a gate/up of 10 tiles, ragged token tiles."""
+    as it multiplies, as both do for 256 tokens.  Layer 0's V rows are that
+    GEMM's own output: the same products in another order (1e-5).  After it the
+    bf16 activations may round apart: 2e-3, as between the layouts above.
+    128-row K and V segments (half a tile), a gate/up of 10 tiles, ragged token
+    tiles."""
     import guanaco_amd.hip as H
     dts = {k: S.Q8_0 for k in S.LAYER_WEIGHTS} if mix == "q8_0" else dict(wv=S.Q6_K, wd=S.Q6_K)
     spec = S.ModelSpec("dense-test", n_layers=2, hidden=512, ff=1280 if mix == "q8_0" else 1536, n_heads=8, n_kv_heads=2,
@@ -632,9 +633,10 @@ def test_prefill_dense_copy_vs_quantized(orc, T, mix):
         dm = H.DeviceModel(c, spec, 768)
         toks = np.random.default_rng(T).integers(0, spec.vocab, T).astype(np.int32)
         res = {}
-        for path in ("auto", "auto_q6k_ref"):
+        for path in ("auto_q6k_ref", "auto"):
             with H.matvec_path(path):
                 _, lg, hid, _ = dm.prefill(toks, 0, want_hidden=True)
+            assert (H.lib.gq_hip_prefill_copy_bytes(c.h) > 0) == (path == "auto" and T > 256)
             k0, v0 = c.kv_read_layer(0)
             res[path] = lg, hid, v0
         a, b = res["auto"], res["auto_q6k_ref"]
@@ -658,9 +660,12 @@ def test_prefill_dense_copy_after_a_failed_allocation(orc):
         toks = np.random.default_rng(3).integers(0, spec.vocab, 300).astype(np.int32)
         with H.matvec_path("auto_q6k_ref"):
             ref = dm.prefill(toks, 0)[1]
+        assert H.lib.gq_hip_prefill_copy_bytes(c.h) == 0
         with_copy = dm.prefill(toks, 0)[1]
+        held = H.lib.gq_hip_prefill_copy_bytes(c.h)
         with pytest.raises(H.HipError):
             c.alloc(1 << 46)
+        assert H.lib.gq_hip_prefill_copy_bytes(c.h) == held > 0
         after = dm.prefill(toks, 0)[1]
         assert np.array_equal(bits(after), bits(with_copy)) and rel_l2(with_copy, ref) < 2e-3
     finally:

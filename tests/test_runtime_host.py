@@ -189,13 +189,13 @@ def test_copies_are_made_by_the_first_long_prompt(dev):
     with H.Context(0) as ctx:
         dm = H.DeviceModel(ctx, SMALL, 4096)
         dm.forward(1, 0)
-        prompt(dm, 200)
+        prompt(dm, 256)
         assert dev.gq_hip_set_prefill_mode(ctx.h, 1) == 0
         prompt(dm, 600)
         assert dev.n("dense_tile") == 0
         assert dev.gq_hip_set_prefill_mode(ctx.h, 0) == 1
         used = dev.fake_used()
-        prompt(dm, 300)
+        prompt(dm, 257)
         made = dev.n("dense_tile")
         assert made == 6 * SMALL.n_layers and dev.fake_used() >= used + copies(SMALL)
         prompt(dm, 3000)  # once
@@ -234,7 +234,7 @@ def test_what_takes_the_copies_back(dev):
     with H.Context(0) as ctx:
         dm = H.DeviceModel(ctx, SMALL, 8192)
         x = ctx.alloc(4 * 200000)
-        prompt(dm, 300)
+        prompt(dm, 257)
         made = dev.n("dense_tile")
         assert made == 6 * SMALL.n_layers
 
