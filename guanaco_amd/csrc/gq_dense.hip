@@ -271,6 +271,28 @@ int gq_launch_dense_tile(void *dst, int dtype, const void *w0, const void *w1, i
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
+/* Tile height and K parts by the time they should take: rounds of
+ * workgroups over the CUs, at a step's measured time each and a round's
+ * start and end, and the parts written and read back.  Measured (us, tall /
+ * flat tiles at their best parts): 512 tokens x 14336 gate + up rows of
+ * 4096: 132 / 157; 4096 rows of 14336: 101 / 75; 1536 tokens: 360 / 417, 197
+ * / 209.  rows: the launch's weight rows, in so many 256-row tiles; part_cap
+ * 0: no workspace for parts. */
+DnShape gq_dense_shape(int mode, int tiles, size_t rows, int T, int K, size_t part_cap, int n_cu) {
+  DnShape f{4, 1};
+  double best = 1e30;
+  for (int tm = 4; tm >= 2; tm -= 2)
+    for (int kp = 1; kp <= (mode == MV_SWIGLU || !part_cap ? 1 : kPgKParts); kp *= 2) {
+      if (kp > 1 && kp * T * rows > part_cap) continue;
+      const int wgs = tiles * ((T + 64 * tm - 1) / (64 * tm)) * kp;
+      const int rounds = (wgs + n_cu - 1) / n_cu;
+      const double us = rounds * ((double)(K / kDK) / kp * (tm == 4 ? 0.92 : 0.64) + 8.0) +
+                        (kp > 1 ? 8.0 * kp * T * (double)rows / 4.0e6 : 0.0);
+      if (us < best) best = us, f = DnShape{tm, kp};
+    }
+  return f;
+}
+
 int gq_launch_dense(int mode, const DnArgs &a0, int n_cu, hipStream_t s) {
   DnArgs a = a0;
   if (!a.x || !a.w || a.T <= 0 || a.K <= 0 || a.K % 256 || a.nseg < 1 || a.nseg > 3) return -1;
@@ -283,36 +305,20 @@ int gq_launch_dense(int mode, const DnArgs &a0, int n_cu, hipStream_t s) {
     a.rows_total += a.rows[i];
   }
   if (mode == MV_SWIGLU && (a.nseg != 1 || !a.act)) return -1;
-  /* Tile height and K parts by the time they should take: rounds of
-   * workgroups over the CUs, at a step's measured time each and a round's
-   * start and end, and the parts written and read back.  Measured (us, tall /
-   * flat tiles at their best parts): 512 tokens x 14336 gate + up rows of
-   * 4096: 132 / 157; 4096 rows of 14336: 101 / 75; 1536 tokens: 360 / 417, 197
-   * / 209. */
-  int best_tm = 4, best_kp = 1;
-  double best = 1e30;
-  for (int tm = 4; tm >= 2; tm -= 2)
-    for (int kp = 1; kp <= (mode == MV_SWIGLU || !a.part ? 1 : kPgKParts); kp *= 2) {
-      if (kp > 1 && (size_t)kp * a.T * a.rows_total > a.part_cap) continue;
-      const int wgs = tiles * ((a.T + 64 * tm - 1) / (64 * tm)) * kp;
-      const int rounds = (wgs + n_cu - 1) / n_cu;
-      const double us = rounds * ((double)(a.K / kDK) / kp * (tm == 4 ? 0.92 : 0.64) + 8.0) +
-                        (kp > 1 ? 8.0 * kp * a.T * a.rows_total / 4.0e6 : 0.0);
-      if (us < best) best = us, best_tm = tm, best_kp = kp;
-    }
-  a.kparts = best_kp;
+  const DnShape f = gq_dense_shape(mode, tiles, a.rows_total, a.T, a.K, a.part ? a.part_cap : 0, n_cu);
+  a.kparts = f.kparts;
   /* A residual launch always leaves its sums in the workspace: the RMSNorm
    * that follows adds them as it reads the row (an epilogue that reads the
    * residual back took 75 us at 512 x 4096 x 4096, one load after another). */
-  a.to_parts = best_kp > 1 || mode == MV_RESID;
-  if (a.to_parts && (!a.part || (size_t)best_kp * a.T * a.rows_total > a.part_cap)) return -1;
-  if (a.kparts_out) *a.kparts_out = a.to_parts ? best_kp : 0;
+  a.to_parts = f.kparts > 1 || mode == MV_RESID;
+  if (a.to_parts && (!a.part || (size_t)f.kparts * a.T * a.rows_total > a.part_cap)) return -1;
+  if (a.kparts_out) *a.kparts_out = a.to_parts ? f.kparts : 0;
   int rc;
-  if (mode == MV_SWIGLU) rc = best_tm == 4 ? launch_dense<MV_SWIGLU, 4>(a, tiles, s) : launch_dense<MV_SWIGLU, 2>(a, tiles, s);
-  else rc = best_tm == 4 ? launch_dense<MV_STORE, 4>(a, tiles, s) : launch_dense<MV_STORE, 2>(a, tiles, s);
+  if (mode == MV_SWIGLU) rc = f.tm == 4 ? launch_dense<MV_SWIGLU, 4>(a, tiles, s) : launch_dense<MV_SWIGLU, 2>(a, tiles, s);
+  else rc = f.tm == 4 ? launch_dense<MV_STORE, 4>(a, tiles, s) : launch_dense<MV_STORE, 2>(a, tiles, s);
   if (rc || !a.to_parts || a.kparts_out) return rc;
   PgArgs p{};
-  p.nseg = a.nseg, p.T = a.T, p.K = a.K, p.part = a.part, p.kparts = best_kp, p.rows_total = a.rows_total;
+  p.nseg = a.nseg, p.T = a.T, p.K = a.K, p.part = a.part, p.kparts = f.kparts, p.rows_total = a.rows_total;
   for (int i = 0; i < a.nseg; i++) p.seg[i].y = a.y[i], p.seg[i].rows = a.rows[i];
   return gq_launch_parts(p, mode == MV_RESID, s);
 }

@@ -338,6 +338,11 @@ struct DnArgs {
   int *kparts_out;
 };
 int gq_launch_dense(int mode, const DnArgs &a, int n_cu, hipStream_t s);
+/* the shape that it picks: 64 tm tokens a workgroup, K in so many parts */
+struct DnShape {
+  int tm, kparts;
+};
+DnShape gq_dense_shape(int mode, int tiles, size_t rows, int T, int K, size_t part_cap, int n_cu);
 /* bytes of the copy of rows x K weights (swiglu: of gate and up together) */
 size_t gq_dense_bytes(int rows, int K, bool swiglu);
 int gq_launch_dense_tile(void *dst, int dtype, const void *w0, const void *w1, int rows, int K, hipStream_t s);

@@ -695,3 +695,144 @@ def test_prefill_weights_rewritten_in_place(orc):
         assert rel_l2(got, ref) < 2e-3 and rel_l2(old, ref) > 0.1
     finally:
         c.close()
+
+
+class DnArgs(C.Structure):  # gq_internal.h
+    _fields_ = [("x", C.c_void_p), ("w", C.c_void_p), ("act", C.c_void_p), ("y", C.c_void_p * 3), ("rows", C.c_int * 3),
+                ("nseg", C.c_int), ("T", C.c_int), ("K", C.c_int), ("part", C.c_void_p), ("part_cap", C.c_size_t),
+                ("kparts", C.c_int), ("rows_total", C.c_int), ("to_parts", C.c_bool), ("kparts_out", C.c_void_p)]
+
+
+class DnShape(C.Structure):
+    _fields_ = [("tm", C.c_int), ("kparts", C.c_int)]
+
+
+def dense_lib():
+    """The launchers of gq_dense.hip, which no entry point reaches alone."""
+    import guanaco_amd.hip as H
+    lib = C.CDLL(H.LIB_PATH)
+    shape, tile, size, run = (lib._Z14gq_dense_shapeiimiimi, lib._Z20gq_launch_dense_tilePviPKvS1_iiP12ihipStream_t,
+                              lib._Z14gq_dense_bytesiib, lib._Z15gq_launch_denseiRK6DnArgsiP12ihipStream_t)
+    shape.restype, shape.argtypes = DnShape, [C.c_int, C.c_int, C.c_size_t, C.c_int, C.c_int, C.c_size_t, C.c_int]
+    tile.argtypes = [C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_void_p]
+    size.restype, size.argtypes = C.c_size_t, [C.c_int, C.c_int, C.c_bool]
+    run.argtypes = [C.c_int, C.POINTER(DnArgs), C.c_int, C.c_void_p]
+    return shape, tile, size, run, lib.hipDeviceSynchronize
+
+
+STORE, RESID, SWIGLU = 0, 1, 2
+
+
+@pytest.mark.parametrize("mode,dtype,rows,T,K,tm,kparts", [
+    (STORE, S.Q8_0, (2048, 256, 256), 513, 512, 2, 1), (STORE, S.Q4_K, (2048, 256, 256), 257, 512, 2, 2),
+    (STORE, S.Q6_K, (384,), 300, 512, 2, 4),           (STORE, S.Q4_K, (4096, 1024, 1024), 1500, 512, 4, 1),
+    (STORE, S.Q6_K, (4096, 1024, 1024), 700, 4096, 4, 2), (STORE, S.Q8_0, (4096, 1024, 1024), 257, 4096, 4, 4),
+    (RESID, S.Q4_K, (2048,), 700, 512, 2, 1),          (RESID, S.Q8_0, (2048,), 513, 512, 2, 2),
+    (RESID, S.Q6_K, (384,), 257, 1024, 2, 4),          (RESID, S.Q4_K, (6144,), 1500, 512, 4, 1),
+    (RESID, S.Q6_K, (8192,), 513, 4096, 4, 2),         (RESID, S.Q4_K, (6144,), 300, 4096, 4, 4),
+    (SWIGLU, S.Q8_0, (1280,), 257, 512, 2, 1),         (SWIGLU, S.Q4_K, (14336,), 257, 512, 4, 1),
+    (SWIGLU, S.Q6_K, (7168,), 513, 512, 4, 1),
+])
+def test_dense_gemm_shapes(ctx, orc, mode, dtype, rows, T, K, tm, kparts):
+    """The GEMM on bf16 copies at each tile height, number of K parts and
+    output that its rule picks (256 CUs), ragged tokens and half tiles among
+    them: against fp64 sums of the same bf16 operands.  fp32 accumulation over
+    K products differs by at most K 2^-24 of the sum of their magnitudes, and as
+    a random walk by far less: 1e-5 of the output's 2-norm, and no element off by
+    more than 1e-4 of the rms.  Nothing past the last token is written."""
+    import guanaco_amd.hip as H
+    shape, tile, size, run, wait = dense_lib()
+    if ctx.info()[0] != 256:
+        pytest.skip("the shapes are picked for 256 CUs")
+    per = 128 if mode == SWIGLU else 256
+    n, tiles = sum(rows), sum((r + per - 1) // per for r in rows)
+    cap = 4 * T * n
+    f = shape(mode, tiles, n, T, K, cap, 256)
+    assert (f.tm, f.kparts) == (tm, kparts)
+    print(f"dense GEMM mode {mode} rows {rows} T {T} K {K}: tm {tm}, {kparts} parts", flush=True)
+    seed = 0xDE ^ (T << 16) ^ (n << 4) ^ K
+    x = bf16_round(orc.synth_normal(seed, T * K).reshape(T, K))
+    ws = [orc.synth_quant(dtype, seed + 1 + i, r, K) for i, r in enumerate(rows * (2 if mode == SWIGLU else 1))]
+    exact = [x.astype(np.float64) @ bf16_round(_kernel_weights(dtype, w, w_rows, K)).astype(np.float64).T
+             for w, w_rows in zip(ws, rows * (2 if mode == SWIGLU else 1))]
+    bufs = [ctx.upload((x.view(np.uint32) >> 16).astype(np.uint16))]
+    wd = [ctx.upload_weight(w) for w in ws]
+    copy = ctx.alloc(sum(size(r, K, mode == SWIGLU) for r in rows))
+    part = ctx.alloc(4 * cap)
+    at = 0
+    for i, r in enumerate(rows):
+        assert tile(copy.ptr + at, dtype, wd[i], wd[1] if mode == SWIGLU else None, r, K, None) == 0
+        at += size(r, K, mode == SWIGLU)
+    a = DnArgs(x=bufs[0].ptr, w=copy.ptr, nseg=len(rows), T=T, K=K, part=part.ptr, part_cap=cap)
+    a.rows[:len(rows)] = rows
+    if mode == SWIGLU:
+        act = ctx.upload(np.full((T + 8, n), 0x7e57, np.uint16))
+        a.act = act.ptr
+        assert run(mode, C.byref(a), 256, None) == 0 and wait() == 0
+        got16 = act.download(np.uint16).reshape(T + 8, n)
+        got = (got16[:T].astype(np.uint32) << 16).view(np.float32)
+        assert (got16[T:] == 0x7e57).all()
+        ref = bf16_round(silu_mul_f32(exact[0], exact[1]))
+        assert rel_l2(got, ref) < 1e-3  # a sum that rounds the other way is off by one in 2^8
+        assert np.abs(got - ref).max() <= 2.0 ** -7 * np.abs(ref).max()
+        bufs += [act]
+    else:
+        old = [orc.synth_normal(seed + 9 + i, (T + 8) * r).reshape(T + 8, r) for i, r in enumerate(rows)]
+        ys = []
+        for leave in (False, True):  # whether the caller adds the parts
+            yd = [ctx.upload(o) for o in old]
+            for i, b in enumerate(yd):
+                a.y[i] = b.ptr
+            left = C.c_int(-1)
+            a.kparts_out = C.addressof(left) if leave else None
+            assert run(mode, C.byref(a), 256, None) == 0 and wait() == 0
+            y = [b.download().reshape(T + 8, r) for b, r in zip(yd, rows)]
+            for b, o in zip(y, old):
+                assert np.array_equal(bits(b[T:]), bits(o[T:]))
+            to_parts = mode == RESID or kparts > 1
+            if leave:
+                assert left.value == (kparts if to_parts else 0)
+            if leave and to_parts:
+                s = part.download(count=kparts * T * n).reshape(kparts, T, n).astype(np.float64).sum(0)
+                for b, o in zip(y, old):
+                    assert np.array_equal(bits(b), bits(o))  # y is left to the caller
+                y = [s[:, sum(rows[:i]):sum(rows[:i + 1])] + (old[i][:T] if mode == RESID else 0) for i in range(len(rows))]
+            ys.append([b[:T] for b in y])
+            for b in yd:
+                b.free()
+        for y in ys:
+            for got, ref, o in zip(y, exact, old):
+                ref = ref + o[:T] if mode == RESID else ref
+                assert rel_l2(got, ref) < 1e-5
+                assert np.abs(got - ref).max() < 1e-4 * np.sqrt(np.mean(ref ** 2))
+    for b in bufs + [copy, part]:
+        b.free()
+    for w in wd:
+        H.lib.gq_hip_free(ctx.h, w)
+
+
+@pytest.mark.parametrize("T,step", [(37, 37), (300, 300), (2049, 1025), (4097, 1366), (8200, 1640)])
+def test_prompt_over_chunks_equals_calls(T, step):
+    """A prompt longer than a chunk (2048 tokens) runs in equal chunks, the
+    last one ragged, whose tokens wait in pinned memory for 8192: the same
+    bits, cache rows included, as those chunks given one call each, and again
+    when it is repeated (as is a shorter one)."""
+    import guanaco_amd.hip as H
+    spec = S.ModelSpec("chunks", n_layers=2, hidden=512, ff=1024, n_heads=8, n_kv_heads=2, vocab=1000,
+                       layer_dtypes=dict(wv=S.Q6_K, wd=S.Q6_K), q4k_zero_mean=True, norm_shift=4)
+    c = H.Context(0)
+    try:
+        dm = H.DeviceModel(c, spec, 8448)
+        toks = np.random.default_rng(T).integers(0, spec.vocab, T).astype(np.int32)
+        got = []
+        for n in (step, T, T):
+            for t in range(0, T, n):
+                nxt, lg, hid, _ = dm.prefill(toks[t:t + n], t, want_hidden=True)
+            kv = [r.reshape(2, 8448, 64)[:, :T] for l in range(2) for r in c.kv_read_layer(l)]
+            got.append([np.array([nxt], np.float32), lg, hid, *kv])
+        assert (H.lib.gq_hip_prefill_copy_bytes(c.h) > 0) == (T > 256)
+        for other in got[1:]:
+            for a, b in zip(other, got[0]):
+                assert np.array_equal(bits(a), bits(b))
+    finally:
+        c.close()
