@@ -304,9 +304,10 @@ def test_prefill_gate_up_wide_tile(ctx, orc, T, N, K):
     (64, 64, 64, 0, 515, 515),     # G = 1, ragged last tile, ends at the cache end
     (64, 32, 64, 0, 1025, 1025),   # G = 2, one token past a tile
     (64, 64, 128, 0, 512, 640),    # whole tiles
+    (32, 8, 128, 0, 1000, 1000),   # G = 4, ragged
     # and in parts, merged
     (32, 8, 128, 256, 512, 768),   # G = 4, two parts
-    (32, 8, 128, 0, 1000, 1000),   # two parts, the first tile with keys in one alone
+    (32, 8, 128, 0, 900, 900),     # two parts, the first tile with keys in one alone
     (32, 4, 64, 2000, 257, 2257),  # G = 8, seven parts, one token past a tile
     (64, 32, 128, 1300, 130, 1430),  # G = 2, five parts
     (64, 8, 128, 1535, 33, 1600),  # eight parts, the first key of a block is the last one seen
