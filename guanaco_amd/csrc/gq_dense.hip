@@ -40,60 +40,106 @@ constexpr int kDN = 256, kDK = 32;
 constexpr int kDWStep = kDN * kDK * 2; /* bytes of a weight tile's step */
 
 /* ---- the copy ---------------------------------------------------------- */
-/* weights 8 o .. 8 o + 7 of a 256-column (Q8_0: 32-column) block, each the
- * fp32 value that PW<>::dequant rounds */
-__device__ void octet_q4k(const uint8_t *b, int o, float (&w)[8]) {
-  const int j = o >> 2, cc = j >> 1;
-  const uint8_t *s = b + 4;
-  const int sc = j < 4 ? s[j] & 63 : (s[j + 4] & 15) | ((s[j - 4] >> 6) << 4);
-  const int mn = j < 4 ? s[j + 4] & 63 : (s[j + 4] >> 4) | ((s[j] >> 6) << 4);
-  const float a = gq_h2f(b[0] | (b[1] << 8)) * (float)sc, m = gq_h2f(b[2] | (b[3] << 8)) * (float)mn;
-  const uint8_t *q = b + 16 + 32 * cc + 8 * (o & 3);
-  for (int i = 0; i < 8; i++) w[i] = __builtin_fmaf(a, (float)((j & 1) ? q[i] >> 4 : q[i] & 15), -m);
-}
-
-__device__ void octet_q6k(const uint8_t *b, int o, float (&w)[8]) {
-  const int n = o >> 4, g = (o >> 2) & 3, l = 8 * (o & 3);
-  const float a = gq_h2f(b[208] | (b[209] << 8)) * (float)(int8_t)b[192 + 8 * n + 2 * g + l / 16];
-  const uint8_t *ql = b + 64 * n + 32 * (g & 1) + l, *qh = b + 128 + 32 * n + l;
-  for (int i = 0; i < 8; i++) {
-    const int q = ((ql[i] >> (4 * (g >> 1))) & 15) | (((qh[i] >> (2 * g)) & 3) << 4);
-    w[i] = a * (float)(q - 32);
-  }
-}
-
-__device__ void octet_q8(const uint8_t *b, int o, float (&w)[8]) {
-  const float d = gq_h2f(b[0] | (b[1] << 8));
-  for (int i = 0; i < 8; i++) w[i] = d * (float)(int8_t)b[2 + 8 * o + i];
-}
-
-/* One workgroup per 256-row tile and 256 columns.  Tile row r is row 256
- * tile + r of w0, or with w1 (gate and up) 32-row blocks of both in turn: row
- * 128 tile + 32 (r / 64) + r % 32 of w0 where (r / 32) is even, of w1 where it
- * is odd.  Rows past `rows` are zero. */
-__global__ __launch_bounds__(256) void dense_tile_kernel(uint8_t *dst, int dtype, const uint8_t *w0, const uint8_t *w1,
-                                                         int rows, int K) {
-  const int tile = blockIdx.x, kb = blockIdx.y, tid = threadIdx.x;
-  const size_t rowbytes = dtype == GQ_Q8_0 ? (size_t)(K / 32) * 34 : (size_t)(K / 256) * (dtype == GQ_Q4_K ? 144 : 210);
-  uint8_t *out = dst + ((size_t)tile * (K / kDK) + 8 * kb) * kDWStep;
-  for (int it = 0; it < 8 * kDN * 4 / 256; it++) {
-    const int u = it * 256 + tid, st = u >> 10, r = (u >> 2) & 255, oct = (u & 3) ^ ((r >> 1) & 3);
-    const bool up = w1 && ((r >> 5) & 1);
-    const int row = w1 ? tile * 128 + 32 * (r >> 6) + (r & 31) : tile * kDN + r;
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (row < rows) {
-      const uint8_t *base = (up ? w1 : w0) + (size_t)row * rowbytes;
-      float w[8];
-      if (dtype == GQ_Q4_K) octet_q4k(base + (size_t)kb * 144, 4 * st + oct, w);
-      else if (dtype == GQ_Q6_K) octet_q6k(base + (size_t)kb * 210, 4 * st + oct, w);
-      else octet_q8(base + (size_t)(8 * kb + st) * 34, oct, w);
-      uint32_t p[4];
+/* eight bf16 of eight fp32 weights, each the value that PW<>::dequant rounds */
+__device__ __forceinline__ void put_octet(uint8_t *out, const float (&w)[8]) {
+  uint32_t p[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) p[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2){w[2 * i], w[2 * i + 1]}, gq_bf2));
-      v = make_uint4(p[0], p[1], p[2], p[3]);
-    }
-    gst<uint4>(out + (size_t)st * kDWStep + 16 * (u & 1023), v);
+  for (int i = 0; i < 4; i++) p[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((gq_f2){w[2 * i], w[2 * i + 1]}, gq_bf2));
+  gst<uint4>(out, make_uint4(p[0], p[1], p[2], p[3]));
+}
+
+__device__ __forceinline__ uint32_t byte8(const uint2 &q, int i) { return ((i < 4 ? q.x : q.y) >> (8 * (i & 3))) & 0xffu; }
+
+/* eight bytes from a 2-byte boundary */
+__device__ __forceinline__ uint2 ld8(const uint8_t *p) {
+  uint2 q;
+  q.x = gld<uint16_t>(p) | ((uint32_t)gld<uint16_t>(p + 2) << 16);
+  q.y = gld<uint16_t>(p + 4) | ((uint32_t)gld<uint16_t>(p + 6) << 16);
+  return q;
+}
+
+/* Octet oct of each of a 256-column block's eight 32-column steps (Q8_0: of
+ * eight blocks), step st to out + st * kDWStep: a lane reads its bytes of the
+ * block once for all the steps that share them. */
+__device__ __forceinline__ void octets_q4k(uint8_t *out, const uint8_t *b, int oct) {
+  const uint4 h = gld<uint4>(b); /* d, dmin, the twelve bytes of scales and mins */
+  const float d = gq_h2f(h.x & 0xffffu), dm = gq_h2f(h.x >> 16);
+  uint2 q[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) q[c] = gld<uint2>(b + 16 + 32 * c + 8 * oct);
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    const int i = 8 * (j & 3);
+    const uint32_t sc = j < 4 ? (h.y >> i) & 63 : ((h.w >> i) & 15) | (((h.y >> (i + 6)) & 3) << 4);
+    const uint32_t mn = j < 4 ? (h.z >> i) & 63 : ((h.w >> (i + 4)) & 15) | (((h.z >> (i + 6)) & 3) << 4);
+    const float a = d * (float)sc, m = dm * (float)mn;
+    float w[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) w[e] = __builtin_fmaf(a, (float)((byte8(q[j >> 1], e) >> (4 * (j & 1))) & 15), -m);
+    put_octet(out + (size_t)j * kDWStep, w);
   }
+}
+
+__device__ __forceinline__ void octets_q6k(uint8_t *out, const uint8_t *b, int oct) {
+  const float d = gq_h2f(gld<uint16_t>(b + 208));
+  uint2 ql[4], qh[2];
+#pragma unroll
+  for (int n = 0; n < 4; n++) ql[n] = ld8(b + 32 * n + 8 * oct);
+#pragma unroll
+  for (int n = 0; n < 2; n++) qh[n] = ld8(b + 128 + 32 * n + 8 * oct);
+#pragma unroll
+  for (int st = 0; st < 8; st++) {
+    const int n = st >> 2, g = st & 3;
+    const float a = d * (float)(int8_t)(gld<uint16_t>(b + 192 + 8 * n + 2 * g) >> (8 * (oct >> 1)));
+    float w[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const uint32_t lo = (byte8(ql[2 * n + (g & 1)], e) >> (4 * (g >> 1))) & 15, hi = (byte8(qh[n], e) >> (2 * g)) & 3;
+      w[e] = a * (float)((int)(lo | (hi << 4)) - 32);
+    }
+    put_octet(out + (size_t)st * kDWStep, w);
+  }
+}
+
+__device__ __forceinline__ void octets_q8(uint8_t *out, const uint8_t *b, int oct) {
+#pragma unroll
+  for (int st = 0; st < 8; st++) {
+    const float d = gq_h2f(gld<uint16_t>(b + 34 * st));
+    const uint2 q = ld8(b + 34 * st + 2 + 8 * oct);
+    float w[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) w[e] = d * (float)(int8_t)byte8(q, e);
+    put_octet(out + (size_t)st * kDWStep, w);
+  }
+}
+
+/* One workgroup per 64 rows of a 256-row tile and 256 columns, four lanes a
+ * row.  Tile row r is row 256 tile + r of w0, or with w1 (gate and up) 32-row
+ * blocks of both in turn: row 128 tile + 32 (r / 64) + r % 32 of w0 where (r /
+ * 32) is even, of w1 where it is odd.  Rows past `rows` are zero.
+ *
+ * The prompt that makes the copies waits for this; what bounds it is the 2
+ * bytes a weight it writes.  us at the 8B shape, with a load a byte and a
+ * workgroup per 256 rows / as it is: q and o 16.2 / 8.3, k and v 14.8 / 4.1, gate
+ * + up 106 / 61 (3.9 TB/s written), down 51 / 23 (Q6_K 69 / 26); the whole
+ * model 8.1 / 3.9 ms. */
+template <int DT>
+__global__ __launch_bounds__(256) void dense_tile_kernel(uint8_t *dst, const uint8_t *w0, const uint8_t *w1, int rows,
+                                                         int K) {
+  const int tile = blockIdx.x, kb = blockIdx.y, tid = threadIdx.x;
+  const int r = 64 * blockIdx.z + (tid >> 2), oct = (tid & 3) ^ ((r >> 1) & 3);
+  const bool up = w1 && ((r >> 5) & 1);
+  const int row = w1 ? tile * 128 + 32 * (r >> 6) + (r & 31) : tile * kDN + r;
+  uint8_t *out = dst + ((size_t)tile * (K / kDK) + 8 * kb) * kDWStep + 64 * r + 16 * (tid & 3);
+  if (row >= rows) {
+    for (int st = 0; st < 8; st++) gst<uint4>(out + (size_t)st * kDWStep, make_uint4(0, 0, 0, 0));
+    return;
+  }
+  constexpr size_t kBlock = DT == GQ_Q4_K ? 144 : DT == GQ_Q6_K ? 210 : 8 * 34;
+  const uint8_t *b = (up ? w1 : w0) + ((size_t)row * (K / 256) + kb) * kBlock;
+  if constexpr (DT == GQ_Q4_K) octets_q4k(out, b, oct);
+  else if constexpr (DT == GQ_Q6_K) octets_q6k(out, b, oct);
+  else octets_q8(out, b, oct);
 }
 
 /* ---- the GEMM ---------------------------------------------------------- */
@@ -264,10 +310,13 @@ size_t gq_dense_bytes(int rows, int K, bool swiglu) {
 }
 
 int gq_launch_dense_tile(void *dst, int dtype, const void *w0, const void *w1, int rows, int K, hipStream_t s) {
-  if ((dtype != GQ_Q4_K && dtype != GQ_Q6_K && dtype != GQ_Q8_0) || rows <= 0 || K <= 0 || K % 256) return -1;
-  const int per = w1 ? kDN / 2 : kDN;
-  hipLaunchKernelGGL(dense_tile_kernel, dim3((rows + per - 1) / per, K / 256), dim3(256), 0, s, (uint8_t *)dst, dtype,
-                     (const uint8_t *)w0, (const uint8_t *)w1, rows, K);
+  if (rows <= 0 || K <= 0 || K % 256 || (((uintptr_t)w0 | (uintptr_t)w1) & 15)) return -1;
+  const dim3 grid((rows + (w1 ? kDN / 2 : kDN) - 1) / (w1 ? kDN / 2 : kDN), K / 256, kDN / 64);
+  const uint8_t *a = (const uint8_t *)w0, *b = (const uint8_t *)w1;
+  if (dtype == GQ_Q4_K) hipLaunchKernelGGL(dense_tile_kernel<GQ_Q4_K>, grid, dim3(256), 0, s, (uint8_t *)dst, a, b, rows, K);
+  else if (dtype == GQ_Q6_K) hipLaunchKernelGGL(dense_tile_kernel<GQ_Q6_K>, grid, dim3(256), 0, s, (uint8_t *)dst, a, b, rows, K);
+  else if (dtype == GQ_Q8_0) hipLaunchKernelGGL(dense_tile_kernel<GQ_Q8_0>, grid, dim3(256), 0, s, (uint8_t *)dst, a, b, rows, K);
+  else return -1;
   return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 

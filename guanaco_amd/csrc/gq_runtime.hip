@@ -1476,8 +1476,8 @@ static bool pf_model_ok(const gq_ctx *c) {
 
 /* The bf16 copies of the projections (pf_model_ok) for prompts of many
  * tokens, made by the first such prompt: 2 bytes a weight, 14 GB at the 8B
- * shape, where they take 8.4 ms once and a 1500-token prompt gains 10 (made at
- * bind, programs that only decode paid 8 of its 26 ms and the memory).  Only
+ * shape, where they take 4 ms once and a 1500-token prompt gains 10 (made at bind,
+ * programs that only decode paid for them too, and held the memory).  Only
  * while they take less than a quarter of the memory that is free: a program
  * that fills the card keeps the room it had.  All of them or none. */
 static void dense_build(gq_ctx *c) {
@@ -1489,6 +1489,9 @@ static void dense_build(gq_ctx *c) {
     at[i] = need;
     if (i != 5) need += gq_dense_bytes(shape[i]->rows, shape[i]->cols, i == 4);
   }
+  for (const gq_layer &L : c->layers)
+    for (const gq_weight *w : {&L.wq, &L.wk, &L.wv, &L.wo, &L.w_gate, &L.w_up, &L.w_down})
+      if ((uintptr_t)w->data & 15) return; /* gq_launch_dense_tile reads whole 16-byte headers */
   c->dense_short = hipMemGetInfo(&fr, &tot) != hipSuccess || need * c->layers.size() >= fr / 4;
   if (c->dense_short) return;
   for (size_t l = 0; l < c->layers.size(); l++) {

@@ -394,7 +394,7 @@ int gq_hip_prefill(gq_ctx *ctx, const int32_t *tokens, int n_tokens, int pos, fl
 int gq_hip_set_prefill_mode(gq_ctx *ctx, int mode);
 /* Prompts of more than 256 tokens multiply by bf16 copies of the
  * projections, which the first such prompt after gq_hip_model_bind makes: 2
- * bytes a weight (14 GB and 8 ms at the 8B shape), kept until the next bind,
+ * bytes a weight (14 GB and 4 ms at the 8B shape), kept until the next bind,
  * and only where they take less than a quarter of the memory then free.  An
  * allocation through the context that needs their room takes them back, as
  * does a write through it to a bound weight; the next such prompt makes them

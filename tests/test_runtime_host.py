@@ -285,3 +285,18 @@ def test_copies_switched_off_and_on(dev):
         assert dev.gq_hip_set_prefill_copies(ctx.h, 1) == 0
         prompt(dm, 300)
         assert dev.n("dense") == n + 4 * SMALL.n_layers and dev.gq_hip_prefill_copy_bytes(ctx.h) == copies(SMALL)
+
+
+def test_no_copies_of_misaligned_weights(dev):
+    """Weights off a 16-byte boundary have no copies, and nothing is allocated
+    for them."""
+    with H.Context(0) as ctx:
+        dm = H.DeviceModel(ctx, SMALL, 512)
+        w = dm.layers[2].wk
+        room = ctx.alloc(S.qbytes(S.Q8_0, w.rows, w.cols) + 16)
+        w.data = room.ptr + 4
+        assert dev.gq_hip_model_bind(ctx.h, C.byref(dm.model)) == 0
+        prompt(dm, 300)
+        used = dev.fake_used()
+        prompt(dm, 300)
+        assert dev.n("dense_tile") == dev.n("dense") == 0 and dev.fake_used() == used
