@@ -24,8 +24,10 @@
  * sum l_c e^(m_c-M).  The position count is read on the device, so the same
  * launch serves every step of a captured decode graph.
  *
- * flash_prefill: causal attention of a prefill chunk (many query tokens) on
- * the fp32 matrix cores; see the kernel.
+ * Causal attention of a prompt's chunk (many query tokens): flash_prefill on
+ * the fp32 matrix cores, flash_split on the bf16 ones from exact three-way
+ * splits of the fp32 operands, whichever flash_shape finds the faster; see the
+ * kernels.
  */
 #include <algorithm>
 #include <cmath>
@@ -576,12 +578,14 @@ __global__ __launch_bounds__(256) void flash_prefill_kernel(AttnArgs a) {
  * to flash_merge_kernel.
  *
  * Microseconds with RoPE and append, 32 heads over 8, head_dim 128, beside
- * the fp32 kernel's: 512 tokens at 3584 382 -> 216 (two parts; 270 with 64
- * rows a workgroup), 2048 at 0 448 -> 256, 128 at 2000 74 -> 58 (six parts),
- * 37 at 8000 246 -> 111 (eight).  The error against float64 of the first is
- * 6e-7 -> 2.6e-7.  Bound by what comes between the matrix instructions, 2.6
- * of a block's 6.2 us: splitting 32 values and 16 probabilities a lane, the
- * exponentials, 56 KB of operands a wave from LDS.
+ * the fp32 kernel's: 512 tokens at 3584 379 -> 211 (two parts; 270 with 64
+ * rows a workgroup), 2048 at 0 429 -> 239, 128 at 2000 71 -> 56, 37 at 8000
+ * 244 -> 109 (both with the keys in parts).  The error against float64 of the
+ * first is 6e-7 -> 2.5e-7.  Bound by what comes between the matrix
+ * instructions, 192 of 32 cycles a SIMD or 2.6 of a block's 6.1 us: splitting
+ * 32 values and 16 probabilities a lane, the exponentials, 56 KB of operands a
+ * wave from LDS.  256 VGPRs at two waves per SIMD; at head_dim 128 they do
+ * not hold everything, 19 to 22 values a lane spill (64-76 bytes of scratch).
  *
  * An infinity or NaN among the operands leaves NaN in the splits and so in
  * the outputs it reaches; a tile with an output that is not finite is computed

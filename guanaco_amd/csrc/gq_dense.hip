@@ -18,11 +18,13 @@
  * which puts a row's gate and up sums into the same lanes.
  *
  * Measured at the 8B shape, us per layer (quantized kernels / here): 512
- * tokens: q/k/v 50 / 45, o 33 / 31, gate + up 151 / 132, down 96 / 73; 1500
- * tokens in one chunk: 152 / 118, 103 / 72, 441 / 390, 344 / 204.  A
- * 1500-token prompt 38.3 -> 32.1 ms (40.8 in chunks of 512 before).  At the
- * best shapes 0.95-1.1 PFLOP/s of the 1.45 that a large library product
- * reaches on the card: with the DMA left out the loop runs at 1.16.
+ * tokens: q/k/v 50 / 45, o 33 / 29, gate + up 151 / 124, down 96 / 74; 1500
+ * tokens in one chunk: 152 / 110, 103 / 70, 441 / 374, 344 / 191.  A
+ * 1500-token prompt 38.3 -> 32.1 ms (40.8 in chunks of 512 before).  At 1500
+ * tokens that is 0.69, 0.72, 0.94 and 0.92 PFLOP/s of the 1.45 that a large
+ * library product reaches on the card: 144, 192, 672 and 192 workgroups leave
+ * 44, 25, 12 and 25% of the 256 CUs idle, and one wave per SIMD waits at every
+ * step's barrier.
  */
 #include <algorithm>
 

@@ -231,11 +231,6 @@ int gq_launch_rmsnorm(const float *x, const float *w, float *out, int dim, float
  * decode step's device token, position and step, and ArgmaxHost.want) */
 int gq_launch_embed(int dtype, const void *table, int hidden, const int *token_dev, int token,
                     float *out, hipStream_t s, int *state = nullptr, int pos = 0, int want = 0);
-/* argmax of x[n] (ties -> lowest index) -> *out_index; when step_dev != NULL
- * also stores the index at tokens[*step_dev], then ++*step_dev and
- * ++*pos_dev (the decode-loop bookkeeping of one graph replay). */
-/* host: what else goes to the host.  emb_out != NULL: the winner's embedding row (emb_dtype, emb_table,
- * hidden) is also written to emb_out, by the same launch */
 /* Pinned host memory that the argmax's launches fill as they go (NULL: not
  * wanted): the index, the values x themselves (only when want is NULL or
  * *want, on the device, is not 0), and a row of row_n floats. */
@@ -247,6 +242,11 @@ struct ArgmaxHost {
   float *row_out;
   int row_n;
 };
+/* argmax of x[n] (ties -> lowest index) -> *out_index; when step_dev != NULL
+ * also stores the index at tokens[*step_dev], then ++*step_dev and
+ * ++*pos_dev (the decode-loop bookkeeping of one graph replay).  emb_out !=
+ * NULL: the winner's embedding row (emb_dtype, emb_table, hidden) is also
+ * written to emb_out, by the same launch.  host: what else goes to the host. */
 int gq_launch_argmax(const float *x, int n, float *scratch, int nblk, int *out_index,
                      int *tokens, int *step_dev, int *pos_dev, hipStream_t s, int emb_dtype = 0,
                      const void *emb_table = nullptr, int hidden = 0, float *emb_out = nullptr,

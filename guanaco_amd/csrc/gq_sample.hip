@@ -298,7 +298,7 @@ __device__ void topk_body(S &sl, const float *x, int V, int k, float T, int rnd,
  *                     slots, then the softmax and the draw as the replay has
  *                     them
  * Bounded by the latency of the dependent launches and of the last one's
- * steps, not by the 0.5 MB of logits: V 128256, k 40: 4.1 + 7.4 + 16.7 us
+ * steps, not by the 0.5 MB of logits: V 128256, k 40: 4.4 + 8.5 + 20 us
  * against the replay's 105 us; a whole gq_hip_sample_dev call 125 -> 41 us
  * (k 200: 717 -> 159, k 1: 55 -> 28; V 1024, k 1: 27 -> 24).  Kernels this
  * short are also bound by fetching their code: bisections unrolled over
