@@ -292,20 +292,33 @@ extern "C" int gq_hip_device_info(gq_ctx *c, int *n_cu, char *name, int name_len
 }
 
 /* ------------------------------------------------------------ memory */
+/* hipMalloc and hipHostMalloc whose failure is not left for the next launch's
+ * check: a caller may go on without, or ask again */
+static void *try_malloc(size_t bytes) {
+  void *p = nullptr;
+  if (hipMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
+}
+static void *try_pinned(size_t bytes) {
+  void *p = nullptr;
+  if (hipHostMalloc(&p, bytes, hipHostMallocDefault) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
+}
+
 static bool dense_drop(gq_ctx *c);
 static size_t dense_held(const gq_ctx *c);
 /* A request that finds no room takes back the bf16 copies of the weights,
  * which prompts can do without, if it fits then.  optional: the caller can do
  * without too; the copies stay. */
 static void *dev_alloc(gq_ctx *c, size_t bytes, bool optional = false) {
-  void *p = nullptr;
-  hipError_t e = hipMalloc(&p, bytes + kPad);
-  if (e != hipSuccess && !optional && dense_held(c)) {
+  void *p = try_malloc(bytes + kPad);
+  if (!p && !optional && dense_held(c)) {
     size_t fr = 0, tot = 0;
-    if (hipMemGetInfo(&fr, &tot) == hipSuccess && bytes <= fr + dense_held(c) && dense_drop(c)) e = hipMalloc(&p, bytes + kPad);
+    if (hipMemGetInfo(&fr, &tot) == hipSuccess && bytes <= fr + dense_held(c) && dense_drop(c)) p = try_malloc(bytes + kPad);
   }
-  if (e != hipSuccess) {
-    (void)hipGetLastError(); /* not for the next launch's check: a caller may go on without */
+  if (!p) {
     fail(c, -4, "hipMalloc(%zu) failed", bytes + kPad);
     return nullptr;
   }
@@ -389,10 +402,7 @@ constexpr size_t kStageBytes = (size_t)32 << 20;
 
 static int staged_h2d(gq_ctx *c, void *dst, const void *src, size_t bytes) {
   for (int i = 0; i < 2; i++) {
-    if (!c->stage[i] && hipHostMalloc(&c->stage[i], kStageBytes, hipHostMallocDefault) != hipSuccess) {
-      c->stage[i] = nullptr;
-      return fail(c, -4, "upload: pinned staging buffer");
-    }
+    if (!c->stage[i] && !(c->stage[i] = try_pinned(kStageBytes))) return fail(c, -4, "upload: pinned staging buffer");
     if (!c->stage_ev[i] && hipEventCreateWithFlags(&c->stage_ev[i], hipEventDisableTiming) != hipSuccess) {
       c->stage_ev[i] = nullptr;
       return fail(c, -4, "upload: staging event");
@@ -435,9 +445,7 @@ extern "C" int gq_hip_mem_info(int device_id, size_t *free_bytes, size_t *total_
 }
 
 extern "C" void *gq_hip_host_alloc_pinned(size_t bytes) {
-  void *p = nullptr;
-  if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) return nullptr;
-  return p;
+  return try_pinned(bytes);
 }
 
 extern "C" void gq_hip_host_free_pinned(void *p) {
@@ -1332,9 +1340,8 @@ static int ensure_pinned(gq_ctx *c, size_t out) {
   free_graph(c); /* it captured the old pointers */
   if (c->pinned) (void)hipHostFree(c->pinned);
   c->pinned = nullptr, c->h_tok = c->h_in = nullptr, c->h_out = nullptr, c->h_out_cap = 0;
-  void *p = nullptr;
-  if (hipHostMalloc(&p, sizeof(int) * (64 + kPinnedTokens) + sizeof(float) * out) != hipSuccess)
-    return fail(c, -4, "pinned memory for %zu floats", out);
+  void *p = try_pinned(sizeof(int) * (64 + kPinnedTokens) + sizeof(float) * out);
+  if (!p) return fail(c, -4, "pinned memory for %zu floats", out);
   c->pinned = p, c->h_tok = (int *)p, c->h_in = c->h_tok + 64, c->h_out = (float *)(c->h_in + kPinnedTokens);
   c->h_out_cap = out;
   return 0;

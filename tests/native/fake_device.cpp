@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <map>
 #include <string>
+#include <utility>
 
 #include "gq_internal.h"
 
@@ -24,6 +25,7 @@ std::map<char *, Block> live; /* device memory */
 size_t used, capacity = (size_t)288 << 30, refuse_from = ~(size_t)0;
 long refuse_after = -1; /* allocations granted before all are refused; -1: no such limit */
 bool refuse_pinned;
+hipError_t last = hipSuccess; /* the last call that failed, until it is asked for */
 std::map<std::string, long> counts;
 std::string errors;
 
@@ -78,7 +80,7 @@ void take(Owed &o, const char *what, const float *part, int n, size_t floats) {
 
 extern "C" {
 /* what the tests ask for and see */
-void fake_reset(size_t total) { capacity = total, refuse_from = ~(size_t)0, refuse_after = -1, refuse_pinned = false, counts.clear(), errors.clear(), owed_qkv = owed_x = Owed(); }
+void fake_reset(size_t total) { capacity = total, refuse_from = ~(size_t)0, refuse_after = -1, refuse_pinned = false, last = hipSuccess, counts.clear(), errors.clear(), owed_qkv = owed_x = Owed(); }
 void fake_refuse_from(size_t bytes) { refuse_from = bytes; } /* allocations of so many bytes and more fail */
 void fake_refuse_after(long n) { refuse_after = n; }
 void fake_refuse_pinned(int on) { refuse_pinned = on != 0; }
@@ -93,7 +95,7 @@ hipError_t hipMalloc(void **p, size_t n) {
   else if (refuse_after == 0) n = ~(size_t)0;
   if (n >= refuse_from || n > capacity - used) {
     counts["refused"]++;
-    return hipErrorOutOfMemory;
+    return last = hipErrorOutOfMemory;
   }
   /* a large block holds no more host memory than its start: nothing here
    * writes past the first floats of a part */
@@ -116,7 +118,7 @@ hipError_t hipFree(void *p) {
 hipError_t hipMemGetInfo(size_t *f, size_t *t) { return *f = capacity - used, *t = capacity, hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
   counts["host_malloc"]++;
-  if (refuse_pinned) return hipErrorOutOfMemory;
+  if (refuse_pinned) return last = hipErrorOutOfMemory;
   return (*p = calloc(1, n)) ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
@@ -135,7 +137,7 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *p, int) {
   return hipSuccess;
 }
 hipError_t hipGetSymbolAddress(void **, const void *) { return hipErrorInvalidSymbol; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() { return std::exchange(last, hipSuccess); }
 const char *hipGetErrorString(hipError_t) { return "fake device"; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return *s = (hipStream_t)&live, hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
@@ -161,7 +163,9 @@ void __hipRegisterVar(void *, void *, char *, char *, int, size_t, int, int) {}
 void __hipUnregisterFatBinary(void *) {}
 }
 
-/* ---- the launchers ---- */
+/* ---- the launchers ----
+ * each asks for the last error, as the real ones do after their launch */
+static int launched() { return hipGetLastError() == hipSuccess ? 0 : -4; }
 int gq_attn_nch(int, int max_seq) { return (max_seq + 31) / 32; }
 int gq_attn_smax(int, int) { return 32; }
 int gq_argmax_blocks(int n) { return (n + 1023) / 1024; }
@@ -178,11 +182,11 @@ void gq_matvec_set_cus(int) {}
 
 static int pgemm_parts(int mode, int T, size_t rows, float *part, size_t cap, int *out, int n) {
   if (out) *out = 0;
-  if (mode == MV_SWIGLU || !out || !part) return 0;
-  if ((size_t)n * T * rows > cap) return 0;
+  if (mode == MV_SWIGLU || !out || !part) return launched();
+  if ((size_t)n * T * rows > cap) return launched();
   leave(mode == MV_RESID ? owed_x : owed_qkv, part, n, (size_t)T * rows);
   *out = n;
-  return 0;
+  return launched();
 }
 int gq_launch_pgemm(int mode, const PgArgs &a, hipStream_t) {
   counts["pgemm"]++;
@@ -202,23 +206,23 @@ int gq_launch_dense_tile(void *dst, int, const void *w0, const void *w1, int row
   counts["dense_tile"]++;
   need("bf16 copy", dst, gq_dense_bytes(rows, K, w1 != nullptr));
   need("weights", w0, 1);
-  return 0;
+  return launched();
 }
 int gq_launch_rmsnorm_rows(const float *x, const float *, float *, int dim, int rows, float, hipStream_t, __bf16 *,
                            const float *parts, int nparts, float *) {
   need("norm", x, sizeof(float) * dim * rows);
   take(owed_x, "norm", parts, parts ? nparts : 0, (size_t)rows * dim);
-  return 0;
+  return launched();
 }
 int gq_launch_rope_append(const RopeArgs &a, hipStream_t) {
   counts["rope_append"]++;
   take(owed_qkv, "rope", a.parts, a.parts ? a.kparts : 0, (size_t)a.ntok * a.prow);
-  return 0;
+  return launched();
 }
 int gq_launch_flash_prefill(const AttnArgs &a, int, hipStream_t) {
   counts["flash"]++;
   if (a.part_o) need("attention parts", a.part_o, sizeof(float) * 2 * a.ntok * a.n_heads * (a.hd + 2));
-  return 0;
+  return launched();
 }
 int gq_launch_argmax(const float *x, int n, float *, int, int *out, int *tokens, int *, int *, hipStream_t, int, const void *, int,
                      float *, const ArgmaxHost &h) {
@@ -226,34 +230,34 @@ int gq_launch_argmax(const float *x, int n, float *, int, int *out, int *tokens,
   if (tokens) need("token log", captured_tokens = tokens, sizeof(int));
   if (h.token) *h.token = 3;
   else *out = 3;
-  return 0;
+  return launched();
 }
 int gq_launch_sample(const float *, int, float temperature, int, float, int, const SampleWs &w, int *out, hipStream_t) {
   if (temperature <= 0.f) return 1;
   counts[w.topk ? "topk_fast" : "topk_replay"]++;
   *out = 5;
-  return 0;
+  return launched();
 }
 int gq_launch_attention(const AttnArgs &a, hipStream_t, hipEvent_t) {
   need("attention parts", a.part_o, sizeof(float) * a.n_heads * a.nch * a.hd);
   need("attention sums", a.part_ml, sizeof(float) * a.n_heads * a.nch * 2);
-  return 0;
+  return launched();
 }
-int gq_launch_matvec(int, int, const MvArgs &, hipStream_t) { return 0; }
+int gq_launch_matvec(int, int, const MvArgs &, hipStream_t) { return launched(); }
 int gq_launch_matvec_pair(int, const MvArgs &, int, const MvArgs &, hipStream_t) { return 1; }
-int gq_launch_mm_tile(void *, int, const void *, const void *, int, int, hipStream_t) { return 0; }
-int gq_launch_q6k_units(void *, const void *, int, int, hipStream_t) { return 0; }
-int gq_launch_rmsnorm(const float *, const float *, float *, int, float, hipStream_t) { return 0; }
-int gq_launch_embed(int, const void *, int, const int *, int, float *out, hipStream_t, int *, int, int) { return need("embedding", out, 4), 0; }
+int gq_launch_mm_tile(void *, int, const void *, const void *, int, int, hipStream_t) { return launched(); }
+int gq_launch_q6k_units(void *, const void *, int, int, hipStream_t) { return launched(); }
+int gq_launch_rmsnorm(const float *, const float *, float *, int, float, hipStream_t) { return launched(); }
+int gq_launch_embed(int, const void *, int, const int *, int, float *out, hipStream_t, int *, int, int) { return need("embedding", out, 4), launched(); }
 int gq_launch_embed_rows(int, const void *, int, const int *tokens, int n, float *, hipStream_t) {
   counts["chunk"]++;
   for (int i = 0; i < n; i++) counts["token_sum"] += tokens[i];
-  return 0;
+  return launched();
 }
-int gq_launch_to_bf16(const float *, __bf16 *, size_t, hipStream_t) { return 0; }
-int gq_launch_silu_mul(float *, const float *, int, hipStream_t) { return 0; }
-int gq_launch_copy(void *, const void *, size_t, int, hipStream_t) { return 0; }
-int gq_launch_stream_read(const void *, size_t, uint32_t *, size_t, hipStream_t) { return 0; }
-int gq_launch_synth_quant(void *, int, int, int, uint64_t, hipStream_t) { return 0; }
-int gq_launch_synth_normal(float *, size_t, uint64_t, int, hipStream_t) { return 0; }
-int gq_launch_synth_kv(float *, int, int, int, int, int, uint64_t, hipStream_t) { return 0; }
+int gq_launch_to_bf16(const float *, __bf16 *, size_t, hipStream_t) { return launched(); }
+int gq_launch_silu_mul(float *, const float *, int, hipStream_t) { return launched(); }
+int gq_launch_copy(void *, const void *, size_t, int, hipStream_t) { return launched(); }
+int gq_launch_stream_read(const void *, size_t, uint32_t *, size_t, hipStream_t) { return launched(); }
+int gq_launch_synth_quant(void *, int, int, int, uint64_t, hipStream_t) { return launched(); }
+int gq_launch_synth_normal(float *, size_t, uint64_t, int, hipStream_t) { return launched(); }
+int gq_launch_synth_kv(float *, int, int, int, int, int, uint64_t, hipStream_t) { return launched(); }

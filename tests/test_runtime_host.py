@@ -143,6 +143,30 @@ def test_failed_bind_leaves_no_model(dev, what):
         assert dev.gq_hip_forward_token(ctx.h, 1, 300, None, None) >= 0
 
 
+@pytest.mark.parametrize("what", ["device", "retry", "pinned", "bind", "upload"])
+def test_refused_memory_is_no_launch_error(dev, what):
+    """Launches are checked by the thread's last error: memory that was refused
+    before one, and then done without or found elsewhere, is not its failure."""
+    dev.fake_reset(GB)
+    with H.Context(0) as ctx:
+        x = ctx.alloc(4096)
+        if what in ("device", "retry"):
+            prompt(H.DeviceModel(ctx, SMALL, 512), 300)
+            rest = GB - 256 - dev.fake_used()
+            assert bool(dev.gq_hip_malloc(ctx.h, rest + (copies(SMALL) // 2 if what == "retry" else GB))) == (what == "retry")
+        else:
+            dev.fake_refuse_pinned(1)
+            if what == "pinned":
+                assert not dev.gq_hip_host_alloc_pinned(4096)
+            elif what == "upload":
+                assert not dev.gq_hip_upload_weight(ctx.h, np.zeros(4096, np.uint8).ctypes.data, 4096)
+            else:
+                with pytest.raises(H.HipError, match="pinned"):
+                    H.DeviceModel(ctx, SMALL, 512)
+            dev.fake_refuse_pinned(0)
+        assert dev.gq_hip_copy_dev(ctx.h, x.ptr, x.ptr + 2048, 2048) == 0
+
+
 def test_refused_token_log(dev):
     """A decode loop whose token log finds no memory fails, and single steps
     go on with the log that their captured graph writes."""
