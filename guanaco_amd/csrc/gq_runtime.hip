@@ -309,14 +309,24 @@ static void *try_pinned(size_t bytes) {
 
 static bool dense_drop(gq_ctx *c);
 static size_t dense_held(const gq_ctx *c);
-/* A request that finds no room takes back the bf16 copies of the weights,
- * which prompts can do without, if it fits then.  optional: the caller can do
- * without too; the copies stay. */
-static void *dev_alloc(gq_ctx *c, size_t bytes, bool optional = false) {
+static void pf_drop(gq_ctx *c);
+static size_t pf_held(const gq_ctx *c);
+/* A request that finds no room takes back what prompts can do without if it
+ * fits then: their workspaces, which the next one makes as the room allows,
+ * and then the bf16 copies of the weights.  Want::prompt: the caller is a
+ * prompt, whose workspaces are in use.  Want::optional: it can do without too;
+ * nothing is taken back. */
+enum class Want { must, prompt, optional };
+static void *dev_alloc(gq_ctx *c, size_t bytes, Want want = Want::must) {
   void *p = try_malloc(bytes + kPad);
-  if (!p && !optional && dense_held(c)) {
-    size_t fr = 0, tot = 0;
-    if (hipMemGetInfo(&fr, &tot) == hipSuccess && bytes <= fr + dense_held(c) && dense_drop(c)) p = try_malloc(bytes + kPad);
+  const size_t ws = want == Want::must ? pf_held(c) : 0, copies = want != Want::optional ? dense_held(c) : 0;
+  size_t fr = 0, tot = 0;
+  if (!p && ws + copies && hipMemGetInfo(&fr, &tot) == hipSuccess && bytes <= fr + ws + copies) {
+    if (ws) {
+      pf_drop(c);
+      p = try_malloc(bytes + kPad);
+    }
+    if (!p && copies && dense_drop(c)) p = try_malloc(bytes + kPad);
   }
   if (!p) {
     fail(c, -4, "hipMalloc(%zu) failed", bytes + kPad);
@@ -1421,11 +1431,11 @@ extern "C" int gq_hip_decode_loop(gq_ctx *c, int token, int pos, int n_steps, in
  * cores, RoPE + append of every token of the chunk, then causal attention
  * (token t sees positions 0 .. pos + t). */
 template <class T>
-static int pf_ensure(gq_ctx *c, T *&p, size_t &cap, size_t n, bool optional = false) {
+static int pf_ensure(gq_ctx *c, T *&p, size_t &cap, size_t n, Want want) {
   if (cap >= n && p) return 0;
   if (p) gq_hip_free(c, p);
   cap = 0;
-  p = (T *)dev_alloc(c, sizeof(T) * n, optional);
+  p = (T *)dev_alloc(c, sizeof(T) * n, want);
   if (!p) return -4;
   cap = n;
   return 0;
@@ -1443,7 +1453,25 @@ static void pf_release(gq_ctx *c) {
   w.cap = w.H = w.F = w.kvd = 0;
 }
 
-static int pf_alloc(gq_ctx *c, int tokens, bool optional = false) {
+/* What the prompts' workspaces hold, K parts and the attention's key parts
+ * included, and their release between prompts. */
+static size_t pf_held(const gq_ctx *c) {
+  const PrefillWs &w = c->pf;
+  return w.cap * (sizeof(float) * 2 * ((size_t)w.H + w.kvd) + sizeof(__bf16) * (2 * (size_t)w.H + w.F)) +
+         sizeof(float) * (w.fs_cap + w.part_cap) + sizeof(__bf16) * w.xb_cap;
+}
+static void pf_drop(gq_ctx *c) {
+  PrefillWs &w = c->pf;
+  pf_release(c);
+  void *bufs[3] = {w.fs, w.part, w.xb};
+  for (void *p : bufs)
+    if (p) gq_hip_free(c, p);
+  w.fs = w.part = nullptr;
+  w.xb = nullptr;
+  w.fs_cap = w.part_cap = w.xb_cap = 0;
+}
+
+static int pf_alloc(gq_ctx *c, int tokens, Want want) {
   PrefillWs &w = c->pf;
   const gq_model &m = c->m;
   const int kvd_m = m.n_kv_heads * m.head_dim;
@@ -1454,11 +1482,11 @@ static int pf_alloc(gq_ctx *c, int tokens, bool optional = false) {
   float **f32[4] = {&w.x, &w.q, &w.k, &w.v};
   const size_t nf[4] = {T * H, T * H, T * kvd, T * kvd};
   for (int i = 0; i < 4; i++)
-    if (!(*f32[i] = (float *)dev_alloc(c, sizeof(float) * nf[i], optional))) return -4;
+    if (!(*f32[i] = (float *)dev_alloc(c, sizeof(float) * nf[i], want))) return -4;
   __bf16 **b16[3] = {&w.xn, &w.att, &w.act};
   const size_t nb[3] = {T * H, T * H, T * F};
   for (int i = 0; i < 3; i++)
-    if (!(*b16[i] = (__bf16 *)dev_alloc(c, sizeof(__bf16) * nb[i], optional))) return -4;
+    if (!(*b16[i] = (__bf16 *)dev_alloc(c, sizeof(__bf16) * nb[i], want))) return -4;
   w.cap = tokens;
   w.H = m.hidden, w.F = m.ff, w.kvd = kvd_m;
   return 0;
@@ -1505,7 +1533,7 @@ static void dense_build(gq_ctx *c) {
     const gq_layer &L = c->layers[l];
     const gq_weight *ws[7] = {&L.wq, &L.wk, &L.wv, &L.wo, &L.w_gate, &L.w_up, &L.w_down};
     auto &M = c->mm[l];
-    M.dn = (uint8_t *)dev_alloc(c, need, true);
+    M.dn = (uint8_t *)dev_alloc(c, need, Want::optional);
     M.dn_bytes = need, M.dn_at[0] = 0, M.dn_at[1] = at[3], M.dn_at[2] = at[4], M.dn_at[3] = at[6];
     bool ok = M.dn != nullptr;
     for (int i = 0; i < 7 && ok; i++)
@@ -1547,7 +1575,7 @@ static int pf_attention(gq_ctx *c, int layer, int pos, int T, int n_heads, float
   aa.scale = 1.0f / sqrtf((float)hd);
   PrefillWs &w = c->pf;
   if (const size_t rows = gq_flash_parts(T, pos, n_heads, c->kv_heads, hd, c->n_cu))
-    if (pf_ensure(c, w.fs, w.fs_cap, rows * (hd + 2), true) == 0) aa.part_o = w.fs, aa.part_ml = w.fs + rows * hd;
+    if (pf_ensure(c, w.fs, w.fs_cap, rows * (hd + 2), Want::optional) == 0) aa.part_o = w.fs, aa.part_ml = w.fs + rows * hd;
   return gq_launch_flash_prefill(aa, c->n_cu, c->stream);
 }
 
@@ -1555,7 +1583,7 @@ static int pf_attention(gq_ctx *c, int layer, int pos, int T, int n_heads, float
  * prompt asks for it before its first layer: a request in between could free
  * sums that a launch has left to the next. */
 static int pf_parts(gq_ctx *c, int T, size_t rows) {
-  return pf_ensure(c, c->pf.part, c->pf.part_cap, gq_parts_tokens(T) * rows, true);
+  return pf_ensure(c, c->pf.part, c->pf.part_cap, gq_parts_tokens(T) * rows, Want::optional);
 }
 
 /* One layer over the chunk (engine.c:352-554 with T tokens): 4 launches of
@@ -1631,9 +1659,9 @@ extern "C" int gq_hip_prefill(gq_ctx *c, const int32_t *tokens, int n_tokens, in
     return (n_tokens + n - 1) / n;
   };
   int chunk = chunks(kPrefillChunk);
-  if (gemm && (rc = pf_alloc(c, chunk, true))) {
+  if (gemm && (rc = pf_alloc(c, chunk, Want::optional))) {
     chunk = chunks(512);
-    if ((rc = pf_alloc(c, chunk))) return rc;
+    if ((rc = pf_alloc(c, chunk, Want::prompt))) return rc;
   }
   if (gemm && chunk >= kDenseTokens && !gq_matvec_q6k_ref()) dense_build(c);
   /* for every launch of a chunk, or for o and down alone, or none: the
@@ -1954,7 +1982,7 @@ static int sample_ensure(gq_ctx *c, int vocab, bool big, int top_k) {
   SampleWs &w = c->sw;
   if (ensure_pinned(c, 0)) return -4;
   if (const size_t tb = top_k > 0 ? gq_sample_topk_bytes(vocab, top_k) : 0; tb && w.topk_cap < vocab) {
-    void *p = dev_alloc(c, tb, true);
+    void *p = dev_alloc(c, tb, Want::optional);
     if (p) { /* without it the one-workgroup replay runs */
       if (w.topk) gq_hip_free(c, w.topk);
       w.topk = p, w.topk_cap = vocab;
@@ -2066,7 +2094,7 @@ extern "C" int gq_hip_chat_turn(gq_ctx *c, const int32_t *tokens, int n_tokens, 
  * matvec path 3 keeps the reference layout.  Freed by the caller. */
 static const uint8_t *op_units(gq_ctx *c, int dtype, const void *w, int rows, int cols) {
   if (dtype != GQ_Q6_K || cols % 2048 || gq_matvec_q6k_ref()) return nullptr;
-  uint8_t *d = (uint8_t *)dev_alloc(c, gq_q6k_units_bytes(rows, cols), true);
+  uint8_t *d = (uint8_t *)dev_alloc(c, gq_q6k_units_bytes(rows, cols), Want::optional);
   if (d && gq_launch_q6k_units(d, w, rows, cols, c->stream)) {
     gq_hip_free(c, d);
     return nullptr;
@@ -2081,7 +2109,7 @@ static PgSeg op_seg(const uint8_t *ps, const void *w, float *y, int n, int dtype
 /* fp32 x -> the bf16 copy the GEMM reads */
 static const __bf16 *pf_x16(gq_ctx *c, const float *x, size_t n) {
   PrefillWs &w = c->pf;
-  if (pf_ensure(c, w.xb, w.xb_cap, n) || gq_launch_to_bf16(x, w.xb, n, c->stream)) return nullptr;
+  if (pf_ensure(c, w.xb, w.xb_cap, n, Want::prompt) || gq_launch_to_bf16(x, w.xb, n, c->stream)) return nullptr;
   return w.xb;
 }
 

@@ -288,6 +288,34 @@ def test_what_takes_the_copies_back(dev):
         held.free()
 
 
+def test_what_takes_the_prompt_workspaces_back(dev):
+    """Between prompts their workspaces (up to 2048 tokens of activations and K
+    parts) are room that a request may need: one that fits with it gets it, one
+    that would not fit even so leaves them, and they go before the copies do."""
+    dev.fake_reset(GB)
+    with H.Context(0) as ctx:
+        dm = H.DeviceModel(ctx, SMALL, 4096)
+        prompt(dm, 2)
+        bare = dev.fake_used()
+        first = prompt(dm, 2048)
+        used = dev.fake_used()
+        held = used - bare - dev.gq_hip_prefill_copy_bytes(ctx.h)
+        assert held > 20 << 20
+        with pytest.raises(H.HipError):
+            ctx.alloc(GB)
+        assert dev.fake_used() == used
+        room = ctx.alloc(GB - 256 - used + held // 2)
+        assert dev.gq_hip_prefill_copy_bytes(ctx.h) == copies(SMALL)
+        for T in (2048, 300, 40):
+            assert prompt(dm, T) == first
+        room.free()
+        assert prompt(dm, 2048) == first
+        room = ctx.alloc(GB - 256 - dev.fake_used() + held + copies(SMALL) // 2)
+        assert dev.gq_hip_prefill_copy_bytes(ctx.h) == 0
+        room.free()
+        assert prompt(dm, 2048) == first
+
+
 def test_copies_switched_off_and_on(dev):
     """gq_hip_set_prefill_copies(0) gives the copies back and makes no more; 1
     allows them again; the setting outlives a bind."""
